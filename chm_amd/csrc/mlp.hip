@@ -49,7 +49,7 @@ struct GemmArgs {
     int ldb, transB;
     float* C;  // fp32 output (pre-activation), may be null
     int ldc;
-    const float* bias;  // per output column, may be null
+    const float* bias;  // per output column, the accumulators' start; may be null
     const float* mask;  // relu' mask source (same shape as output, ld = ldc), may be null
     int relu;
     uint16_t* Cb;  // bf16 copy of the (activated) output, may be null
@@ -107,9 +107,12 @@ __global__ void __launch_bounds__(256) k_gemm_bf16(GemmArgs g) {
     const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
     f32x4 acc[2][2];
 #pragma unroll
-    for (int a = 0; a < 2; ++a)
+    for (int b = 0; b < 2; ++b) {
+        const int col = n0 + wn + b * 16 + (lane & 15);
+        const float start = g.bias && col < g.N ? g.bias[col] : 0.f;
 #pragma unroll
-        for (int b = 0; b < 2; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int a = 0; a < 2; ++a) acc[a][b] = f32x4{start, start, start, start};
+    }
     for (int k0 = kb; k0 < ke; k0 += TK) {
         // each thread stages one 8-element (16-byte) chunk of A and one of B: 64 x 32 = 256
         // chunks per operand.  A chunk runs along the operand's contiguous dimension (k for
@@ -144,7 +147,6 @@ __global__ void __launch_bounds__(256) k_gemm_bf16(GemmArgs g) {
                     g.slab[((size_t)blockIdx.z * g.M + row) * g.N + col] = v;
                     continue;
                 }
-                if (g.bias) v += g.bias[col];
                 if (g.mask && !(g.mask[(size_t)row * g.ldc + col] > 0.f)) v = 0.f;
                 if (g.C) g.C[(size_t)row * g.ldc + col] = v;
                 if (g.relu) v = fmaxf(v, 0.f);
@@ -344,20 +346,27 @@ __global__ void k_denorm(int64_t n, const float* __restrict__ Yp, const float* _
     Y[t] = Yp[r * MlpDims::OUTP + c] * sd[c] + mu[c];
 }
 
-// Inference of the whole network in one launch: a workgroup walks 64-sample tiles
-// (persistent grid) and a tile's activations ping-pong between two 64 x 128 BF16 LDS
-// buffers, so nothing but the 16 input features and the 11 outputs of a sample touches
-// HBM (the layer-by-layer path writes and re-reads 3 x 256 MB of activations at 1M
-// faces).  The BF16 weights (73.7 KB) are read through the vector cache, where every
-// workgroup of a CU shares them.  Eight waves; in a 128-wide layer wave w computes rows
-// 16 (w % 4) .. +16 and columns 64 (w / 4) .. +64 as four 16 x 16 MFMA blocks, K in
-// steps of 32 in increasing order -- the operand layout, accumulation order and epilogue
-// (+ bias, ReLU, BF16 rounding) of k_gemm_bf16, so the output equals the layer-by-layer
-// forward bit for bit.  LDS: 41.5 KB per workgroup.
-constexpr int kInferRows = 64;
-constexpr int kInferThreads = 512;
-constexpr int kAs = MlpDims::H + 8;    // LDS row stride (BF16) of the activation tiles (16-byte rows)
-constexpr int kAs0 = MlpDims::IN + 8;  // of the input tile
+// Inference of the whole network in one launch, activations in registers.
+//
+// A wave owns 64 samples and carries them through all four layers by itself: the weights are
+// the MFMA's A operand and the activations its B operand, so a product leaves four consecutive
+// output features of one sample in a lane (C: column = sample = lane % 16, rows 4 (lane / 16)
+// + j).  The weight rows of two 16-row blocks are permuted so that a lane's 2 x 4 results are
+// the eight features 32 kk + 8 (lane / 16) .. + 7 -- the B operand of the next layer's k-step
+// kk, in natural k order -- so a layer's output feeds the next layer's MFMAs after bias, ReLU
+// and BF16 packing without touching LDS, and there is no barrier between layers.  LDS holds
+// only the weights, laid out once per workgroup in the order the lanes read them (one
+// conflict-free 16-byte load per lane and fragment, each used for four MFMAs).
+//
+// Bound: the matrix cores (304 MFMAs of 16x16x32 per 64 samples against 76 16-byte LDS reads
+// per lane) and the packing between layers.  999,968 samples: 581 -> 100 us (127 -> 737 TFLOP/s;
+// before, each 64-sample workgroup tile re-read the 74 KB of weights through the vector cache,
+// and its activations crossed LDS with a barrier per layer).
+// The bias is the accumulator's start and k runs in increasing order, as in k_gemm_bf16, so
+// the output equals the layer-by-layer forward bit for bit.
+constexpr int kInferCols = 64;      // samples per wave and tile
+constexpr int kInferThreads = 512;  // eight waves, one workgroup per CU (78 KB of weights)
+constexpr int kFrags[5] = {0, 8, 40, 72, 76};  // first weight fragment of each layer
 
 struct InferArgs {
     int64_t n;
@@ -366,87 +375,124 @@ struct InferArgs {
     const float* b[4];
     const float* norm;     // x_mean[IN], x_std[IN], y_mean[OUT], y_std[OUT]
     float* Y;              // [n x OUT] raw outputs
+    int x16;               // X is 16-byte aligned
 };
 
-// one layer on a 64-row tile: in (LDS, row stride ins, K columns) x W^T (global BF16
-// [dout x K]) + bias, dout = 128 (hidden) or 16 (output layer: waves 0-3 only); BF16
-// (+ ReLU) into outb or FP32 into outf
-__device__ __forceinline__ void infer_layer(const uint16_t* __restrict__ in, int ins, int K,
-                                            const uint16_t* __restrict__ W, const float* __restrict__ bias, int dout,
-                                            bool relu, uint16_t* __restrict__ outb, float* __restrict__ outf) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int r0 = 16 * (wave & 3);
-    const int c0 = 64 * (wave >> 2);
-    if (c0 >= dout) return;
-    const int nblk = min(4, (dout - c0) / 16);  // 16-column MFMA blocks of this wave
-    f32x4 acc[4];
+// one hidden layer of a wave's 64 samples: in[ks][cb] / out[kk][cb] are B operands (k-step,
+// 16-sample block); wf: the layer's fragments in LDS, block rb's k-step ks at rb * KS + ks
+template <int KS>
+__device__ __forceinline__ void infer_hidden(const bf16x8 (&in)[KS][4], bf16x8 (&out)[4][4],
+                                             const uint16_t* __restrict__ wf, const float* __restrict__ bias,
+                                             int lane) {
+    const int q = lane >> 4;
 #pragma unroll
-    for (int b = 0; b < 4; ++b) acc[b] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int k0 = 0; k0 < K; k0 += 32) {
-        // K = 16 (the input layer): the upper half of the 32-wide step is zero padding
-        bf16x8 a = {};
-        if (k0 + 8 * (lane >> 4) < K) a = frag8(&in[(r0 + (lane & 15)) * ins + k0 + 8 * (lane >> 4)]);
+    for (int kk = 0; kk < 4; ++kk) {
+        f32x4 acc[2][4];
 #pragma unroll
-        for (int b = 0; b < 4; ++b) {
-            if (b < nblk) {
-                bf16x8 w = {};
-                if (k0 + 8 * (lane >> 4) < K) w = frag8(&W[(c0 + 16 * b + (lane & 15)) * K + k0 + 8 * (lane >> 4)]);
-                acc[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, w, acc[b], 0, 0, 0);
-            }
+        for (int h = 0; h < 2; ++h) {
+            const f32x4 bq = *reinterpret_cast<const f32x4*>(&bias[32 * kk + 8 * q + 4 * h]);
+#pragma unroll
+            for (int cb = 0; cb < 4; ++cb) acc[h][cb] = bq;
         }
-    }
 #pragma unroll
-    for (int b = 0; b < 4; ++b) {
-        if (b < nblk) {
+        for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int row = r0 + 4 * (lane >> 4) + j;
-                const int col = c0 + 16 * b + (lane & 15);
-                float v = acc[b][j] + bias[col];
-                if (outf) {
-                    outf[row * MlpDims::OUTP + col] = v;
-                } else {
-                    if (relu) v = fmaxf(v, 0.f);
-                    outb[row * kAs + col] = to_bf16(v);
-                }
+            for (int h = 0; h < 2; ++h) {
+                const bf16x8 w = frag8(wf + (((2 * kk + h) * KS + ks) * 64 + lane) * 8);
+#pragma unroll
+                for (int cb = 0; cb < 4; ++cb)
+                    acc[h][cb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, in[ks][cb], acc[h][cb], 0, 0, 0);
             }
-        }
+#pragma unroll
+        for (int cb = 0; cb < 4; ++cb)
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) out[kk][cb][4 * h + j] = (__bf16)fmaxf(acc[h][cb][j], 0.f);
+        // keeps the scheduler from starting the next block pair's accumulators and weight
+        // reads early, which spilled 328 of the 256 registers
+        __builtin_amdgcn_sched_barrier(0);
     }
 }
 
 __global__ void __launch_bounds__(kInferThreads) k_mlp_infer(InferArgs p) {
     constexpr int H = MlpDims::H, IN = MlpDims::IN, OUT = MlpDims::OUT, OUTP = MlpDims::OUTP;
-    __shared__ __align__(16) uint16_t xin[kInferRows * kAs0];
-    __shared__ __align__(16) uint16_t act0[kInferRows * kAs];
-    __shared__ __align__(16) uint16_t act1[kInferRows * kAs];
-    __shared__ float yout[kInferRows * OUTP];
-    const int tid = threadIdx.x;
-    const float* xmu = p.norm;
-    const float* xsd = p.norm + IN;
-    const float* ymu = p.norm + 2 * IN;
-    const float* ysd = p.norm + 2 * IN + OUT;
-    const int64_t ntiles = (p.n + kInferRows - 1) / kInferRows;
-    for (int64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-        const int64_t row0 = tile * kInferRows;
-        __syncthreads();  // the previous tile's outputs are consumed
-        for (int e = tid; e < kInferRows * IN; e += kInferThreads) {
-            const int r = e / IN, c = e % IN;
-            const int64_t g = row0 + r;
-            xin[r * kAs0 + c] = g < p.n ? to_bf16((p.X[g * IN + c] - xmu[c]) / xsd[c]) : (uint16_t)0;
+    __shared__ __align__(16) uint16_t wf[kFrags[4] * 64 * 8];
+    __shared__ __align__(16) float bias[3 * H + OUTP];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    for (int e = tid; e < kFrags[4] * 64; e += kInferThreads) {
+        const int f = e >> 6, r = e & 15, q = (e >> 4) & 3;
+        const int l = f < kFrags[1] ? 0 : f < kFrags[2] ? 1 : f < kFrags[3] ? 2 : 3;
+        const int g = f - kFrags[l], ks = l == 0 ? 0 : g & 3, rb = l == 0 ? g : g >> 2;
+        const int row = l < 3 ? 32 * (rb >> 1) + 8 * (r >> 2) + 4 * (rb & 1) + (r & 3) : r;
+        const int K = l == 0 ? IN : H, col = 32 * ks + 8 * q;
+        bf16x8 v = {};
+        if (col < K) v = frag8(p.W[l] + row * K + col);  // K = 16: the upper half of the k-step is zero
+        *reinterpret_cast<bf16x8*>(&wf[e * 8]) = v;
+    }
+    for (int e = tid; e < 3 * H + OUTP; e += kInferThreads) bias[e] = p.b[e / H][e % H];
+    __syncthreads();
+    const int r = lane & 15, q = lane >> 4;
+    float xmu[8], xsd[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        xmu[j] = q < 2 ? p.norm[8 * q + j] : 0.f;
+        xsd[j] = q < 2 ? p.norm[IN + 8 * q + j] : 1.f;
+    }
+    float ymu[4], ysd[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const int o = min(4 * q + j, OUT - 1);
+        ymu[j] = p.norm[2 * IN + o];
+        ysd[j] = p.norm[2 * IN + OUT + o];
+    }
+    const int64_t ntiles = (p.n + kInferCols - 1) / kInferCols;
+    for (int64_t tile = blockIdx.x + (int64_t)gridDim.x * wave; tile < ntiles;
+         tile += (int64_t)gridDim.x * (kInferThreads / 64)) {
+        const int64_t s0 = tile * kInferCols;
+        bf16x8 x[1][4], a[4][4], c[4][4];
+#pragma unroll
+        for (int cb = 0; cb < 4; ++cb) {
+            const int64_t g = s0 + 16 * cb + r;
+            float v[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) v[j] = xmu[j];
+            if (q < 2 && g < p.n) {
+                const float* src = p.X + g * IN + 8 * q;
+                if (p.x16) {
+                    const f32x4 lo = *reinterpret_cast<const f32x4*>(src);
+                    const f32x4 hi = *reinterpret_cast<const f32x4*>(src + 4);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) v[j] = lo[j], v[4 + j] = hi[j];
+                } else {
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) v[j] = src[j];
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < 8; ++j) x[0][cb][j] = (__bf16)((v[j] - xmu[j]) / xsd[j]);
         }
-        __syncthreads();
-        infer_layer(xin, kAs0, IN, p.W[0], p.b[0], H, true, act0, nullptr);
-        __syncthreads();
-        infer_layer(act0, kAs, H, p.W[1], p.b[1], H, true, act1, nullptr);
-        __syncthreads();
-        infer_layer(act1, kAs, H, p.W[2], p.b[2], H, true, act0, nullptr);
-        __syncthreads();
-        infer_layer(act0, kAs, H, p.W[3], p.b[3], OUTP, false, nullptr, yout);
-        __syncthreads();
-        for (int e = tid; e < kInferRows * OUT; e += kInferThreads) {
-            const int r = e / OUT, c = e % OUT;
-            const int64_t g = row0 + r;
-            if (g < p.n) p.Y[g * OUT + c] = yout[r * OUTP + c] * ysd[c] + ymu[c];
+        infer_hidden<1>(x, a, wf, bias, lane);
+        infer_hidden<4>(a, c, wf + kFrags[1] * 512, bias + H, lane);
+        infer_hidden<4>(c, a, wf + kFrags[2] * 512, bias + 2 * H, lane);
+        f32x4 acc[4];
+#pragma unroll
+        for (int cb = 0; cb < 4; ++cb) acc[cb] = *reinterpret_cast<const f32x4*>(&bias[3 * H + 4 * q]);
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) {
+            const bf16x8 w = frag8(wf + ((kFrags[3] + ks) * 64 + lane) * 8);
+#pragma unroll
+            for (int cb = 0; cb < 4; ++cb)
+                acc[cb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, a[ks][cb], acc[cb], 0, 0, 0);
+        }
+#pragma unroll
+        for (int cb = 0; cb < 4; ++cb) {
+            const int64_t g = s0 + 16 * cb + r;
+            if (g < p.n) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    if (4 * q + j < OUT) p.Y[g * OUT + 4 * q + j] = acc[cb][j] * ysd[j] + ymu[j];
+            }
         }
     }
 }
@@ -684,7 +730,7 @@ bool Mlp::fused_inference_ok() {
     if (fused_ok < 0) {
         int cus = 0;
         PB_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
-        infer_blocks = 2 * (cus > 0 ? cus : 256);  // two workgroups per CU (104 VGPRs, 8 waves each)
+        infer_blocks = cus > 0 ? cus : 256;  // one workgroup (eight waves) per CU
         fused_ok = 1;
     }
     return fused_ok == 1;
@@ -700,7 +746,8 @@ void Mlp::predict_fused(const float* X, float* Y, int64_t n, hipStream_t s) {
     }
     a.norm = norm.p;
     a.Y = Y;
-    const int64_t tiles = (n + kInferRows - 1) / kInferRows;
+    a.x16 = ((uintptr_t)X & 15) == 0;
+    const int64_t tiles = (n + kInferCols - 1) / kInferCols;
     const unsigned grid = (unsigned)std::min<int64_t>(tiles, infer_blocks);
     hipLaunchKernelGGL(k_mlp_infer, dim3(grid), dim3(kInferThreads), 0, s, a);
     PB_HIP(hipGetLastError());

@@ -35,7 +35,7 @@ class Mlp {
     int device = 0;
     hipStream_t stream = nullptr;
     int fused_ok = -1;       // fused inference set up on this device (-1: not yet)
-    int infer_blocks = 512;  // persistent grid of the fused inference (two workgroups per CU)
+    int infer_blocks = 256;  // persistent grid of the fused inference (one workgroup per CU)
 
   private:
     void ensure(int64_t n);
