@@ -3,15 +3,13 @@
 // (gfx950's v_mfma_f32_16x16x32_bf16), trained on the GPU by its own forward
 // and backward kernels with Adam.
 //
-// Every layer is a GEMM with a fused epilogue.  Activations are stored
-// [samples x features] row-major; for a layer with weights W [out x in]
-//   forward   Z = A_in W^T + b,   A_out = relu(Z)        (M=samples, N=out, K=in)
-//   backward  dW = dZ^T A_in,     db = colsum(dZ)        (M=out, N=in, K=samples)
-//             dA_in = dZ W,       dZ_in = dA_in * [Z_in > 0]  (M=samples, N=in, K=out)
-// The GEMM stages 64x32 A and 32x64 B tiles of BF16 in LDS, both k-contiguous
-// (As[row][k], Bs[col][k]); each of the four wavefronts owns a 32x32 quarter of
-// the 64x64 output tile, i.e. 2x2 MFMA 16x16 blocks, with the operand fragments
-// read from LDS in the MFMA lane layout as one 16-byte load per lane
+// For a layer with weights W [out x in], activations A and pre-activations Z [samples x features]
+//   forward   Z = A_in W^T + b,   A_out = relu(Z)
+//   backward  dW = dZ^T A_in,     db = colsum(dZ),   dZ_in = (dZ W) * [Z_in > 0]
+// Inference (k_mlp_infer) carries a wave's samples through all layers in registers; training
+// (k_mlp_train) runs forward and backward of a 64-sample tile in one workgroup and keeps the
+// weight gradients in its accumulators; k_gemm_bf16 is the layer-by-layer forward that the
+// fused inference is checked against.  MFMA operand layout of v_mfma_f32_16x16x32_bf16
 // (A: row = lane%16, k = 8*(lane/16)+j, j < 8; B: col = lane%16, same k;
 // C: col = lane%16, row = 4*(lane/16)+j, j < 4).
 #include <cmath>
@@ -41,86 +39,47 @@ __device__ __forceinline__ uint16_t to_bf16(float f) {
     return (uint16_t)(u >> 16);
 }
 
+// C [M x N] = A [M x K] B^T + bias, B [N x K] (k contiguous in both)
 struct GemmArgs {
     int M, N, K;
     const uint16_t* A;
-    int lda, transA;
     const uint16_t* B;
-    int ldb, transB;
-    float* C;  // fp32 output (pre-activation), may be null
-    int ldc;
-    const float* bias;  // per output column, the accumulators' start; may be null
-    const float* mask;  // relu' mask source (same shape as output, ld = ldc), may be null
-    int relu;
-    uint16_t* Cb;  // bf16 copy of the (activated) output, may be null
-    int ldcb;
-    float* slab;  // split-K: blockIdx.z writes its raw partial product to slab[z][M][N]
-    int ksplit;   // K range per blockIdx.z
+    const float* bias;  // per output column, the accumulators' start
+    float* C;           // fp32 output, may be null
+    uint16_t* Cb;       // bf16 copy of relu(C), may be null
 };
 
-// One 16-byte chunk of a 64 x 32 operand tile into LDS T[64][TK + 8] (T[row][k]).
-// kmajor = 0: element (row, k) at X[row * ld + k] (k contiguous; chunk = 8 k of one row);
-// kmajor = 1: element (row, k) at X[k * ld + row] (row contiguous; chunk = 8 rows of one k).
-// rows: the matrix's row count (M or N); r0 / k0: the tile origin; ke: end of the K range.
-__device__ __forceinline__ void stage_chunk(const uint16_t* __restrict__ X, int ld, int kmajor, int rows, int r0,
-                                            int k0, int ke, int tid, uint16_t (*T)[TK + 8]) {
+// One 16-byte chunk of a 64 x 32 operand tile into LDS T[64][TK + 8] (T[row][k]): 8 k of one
+// row.  rows: the matrix's row count (M or N); r0 / k0: the tile origin.
+__device__ __forceinline__ void stage_chunk(const uint16_t* __restrict__ X, int ld, int rows, int r0, int k0, int tid,
+                                            uint16_t (*T)[TK + 8]) {
     typedef uint16_t u16x8 __attribute__((ext_vector_type(8)));
-    if (!kmajor) {
-        const int r = tid >> 2, c = (tid & 3) * 8;  // 64 rows x 4 chunks
-        const int gr = r0 + r, gk = k0 + c;
-        u16x8 v = {0, 0, 0, 0, 0, 0, 0, 0};
-        const size_t off = (size_t)gr * ld + gk;
-        if (gr < rows && gk + 8 <= ke && ((uintptr_t)(X + off) & 15) == 0) {
-            v = *reinterpret_cast<const u16x8*>(X + off);
-        } else if (gr < rows) {
-#pragma unroll
-            for (int j = 0; j < 8; ++j)
-                if (gk + j < ke) v[j] = X[off + j];
-        }
-        *reinterpret_cast<u16x8*>(&T[r][c]) = v;
-    } else {
-        const int kk = tid >> 3, r = (tid & 7) * 8;  // 32 k x 8 chunks of 8 rows
-        const int gk = k0 + kk, gr = r0 + r;
-        u16x8 v = {0, 0, 0, 0, 0, 0, 0, 0};
-        const size_t off = (size_t)gk * ld + gr;
-        if (gk < ke) {
-            if (gr + 8 <= rows && ((uintptr_t)(X + off) & 15) == 0) {
-                v = *reinterpret_cast<const u16x8*>(X + off);
-            } else {
-#pragma unroll
-                for (int j = 0; j < 8; ++j)
-                    if (gr + j < rows) v[j] = X[off + j];
-            }
-        }
-#pragma unroll
-        for (int j = 0; j < 8; ++j) T[r + j][kk] = v[j];
-    }
+    const int r = tid >> 2, c = (tid & 3) * 8;  // 64 rows x 4 chunks
+    const int gr = r0 + r, gk = k0 + c;
+    u16x8 v = {0, 0, 0, 0, 0, 0, 0, 0};
+    if (gr < rows && gk < ld) v = *reinterpret_cast<const u16x8*>(X + (size_t)gr * ld + gk);  // ld is 16 or 128
+    *reinterpret_cast<u16x8*>(&T[r][c]) = v;
 }
 
+// 64x32 A and B tiles of BF16 in LDS; each of the four wavefronts owns a 32x32 quarter of the
+// 64x64 output tile, i.e. 2x2 MFMA blocks, one 16-byte LDS read per lane and fragment.
 __global__ void __launch_bounds__(256) k_gemm_bf16(GemmArgs g) {
     __shared__ __align__(16) uint16_t As[TM][TK + 8];
     __shared__ __align__(16) uint16_t Bs[TN][TK + 8];
     const int m0 = blockIdx.y * TM, n0 = blockIdx.x * TN;
-    const int kb = blockIdx.z * g.ksplit;
-    const int ke = min(g.K, kb + g.ksplit);
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
     f32x4 acc[2][2];
 #pragma unroll
     for (int b = 0; b < 2; ++b) {
         const int col = n0 + wn + b * 16 + (lane & 15);
-        const float start = g.bias && col < g.N ? g.bias[col] : 0.f;
+        const float start = col < g.N ? g.bias[col] : 0.f;
 #pragma unroll
         for (int a = 0; a < 2; ++a) acc[a][b] = f32x4{start, start, start, start};
     }
-    for (int k0 = kb; k0 < ke; k0 += TK) {
-        // each thread stages one 8-element (16-byte) chunk of A and one of B: 64 x 32 = 256
-        // chunks per operand.  A chunk runs along the operand's contiguous dimension (k for
-        // A [M x K] / B [N x K], m or n for the transposed storage) and is loaded with one
-        // vector load when it lies inside the matrix, element by element (zero-filled)
-        // otherwise; the LDS layout (As[m][k], Bs[n][k]) is the same either way.
-        stage_chunk(g.A, g.lda, g.transA, g.M, m0, k0, ke, tid, As);
-        stage_chunk(g.B, g.ldb, g.transB ^ 1, g.N, n0, k0, ke, tid, Bs);
+    for (int k0 = 0; k0 < g.K; k0 += TK) {
+        stage_chunk(g.A, g.K, g.M, m0, k0, tid, As);
+        stage_chunk(g.B, g.K, g.N, n0, k0, tid, Bs);
         __syncthreads();
 #pragma unroll
         for (int tm = 0; tm < 2; ++tm) {
@@ -142,198 +101,29 @@ __global__ void __launch_bounds__(256) k_gemm_bf16(GemmArgs g) {
                 const int row = m0 + wm + tm * 16 + 4 * (lane >> 4) + j;
                 const int col = n0 + wn + tn * 16 + (lane & 15);
                 if (row >= g.M || col >= g.N) continue;
-                float v = acc[tm][tn][j];
-                if (g.slab) {
-                    g.slab[((size_t)blockIdx.z * g.M + row) * g.N + col] = v;
-                    continue;
-                }
-                if (g.mask && !(g.mask[(size_t)row * g.ldc + col] > 0.f)) v = 0.f;
-                if (g.C) g.C[(size_t)row * g.ldc + col] = v;
-                if (g.relu) v = fmaxf(v, 0.f);
-                if (g.Cb) g.Cb[(size_t)row * g.ldcb + col] = to_bf16(v);
+                const float v = acc[tm][tn][j];
+                if (g.C) g.C[(size_t)row * g.N + col] = v;
+                if (g.Cb) g.Cb[(size_t)row * g.N + col] = to_bf16(fmaxf(v, 0.f));
             }
 }
 
-constexpr int kMaxSplits = 64;  // split-K factor of the weight-gradient GEMMs (K = batch rows)
-
-// C[r][c] = sum over z = 0 .. splits-1, in that order, of slab[z][r][c] (deterministic split-K)
-__global__ void k_sum_slabs(int M, int N, int splits, const float* __restrict__ slab, float* __restrict__ C,
-                            int ldc) {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= (int64_t)M * N) return;
-    const size_t mn = (size_t)M * N;
-    float acc = 0.f;
-    int z = 0;
-    for (; z + 8 <= splits; z += 8) {  // eight loads in flight, added in slab order
-        float v[8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) v[u] = slab[(size_t)(z + u) * mn + t];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) acc += v[u];
-    }
-    for (; z < splits; ++z) acc += slab[(size_t)z * mn + t];
-    C[(t / N) * ldc + t % N] = acc;
-}
-
-// Split-K GEMMs (splits > 1) need ws with room for splits * M * N floats; the
-// partial products are summed in a fixed order, so results do not depend on
-// scheduling (bias, masks and bf16 copies are not supported with splits).
-void gemm(hipStream_t s, GemmArgs g, int splits = 1, float* ws = nullptr) {
-    if (splits < 1) splits = 1;
-    g.ksplit = ((g.K + splits - 1) / splits + TK - 1) / TK * TK;
-    splits = (g.K + g.ksplit - 1) / g.ksplit;
-    g.slab = splits > 1 ? ws : nullptr;
-    if (splits > 1 && (!ws || g.bias || g.mask || g.relu || g.Cb || !g.C))
-        throw Error(PBSM3D_EINVAL, "split-K GEMM needs a workspace and a plain FP32 output");
-    dim3 grid((g.N + TN - 1) / TN, (g.M + TM - 1) / TM, splits);
-    hipLaunchKernelGGL(k_gemm_bf16, grid, dim3(256), 0, s, g);
-    if (splits > 1) {
-        const int64_t mn = (int64_t)g.M * g.N;
-        hipLaunchKernelGGL(k_sum_slabs, dim3((unsigned)((mn + 255) / 256)), dim3(256), 0, s, g.M, g.N, splits, ws,
-                           g.C, g.ldc);
-    }
-}
-
-// x (rows x 16, f32) -> normalised bf16 rows; optional row gather idx
-__global__ void k_prep_inputs(int64_t n, const float* __restrict__ X, const int64_t* __restrict__ idx,
-                              const float* __restrict__ mu, const float* __restrict__ sd, uint16_t* __restrict__ Xb) {
+// x (rows x 16, f32) -> normalised bf16 rows
+__global__ void k_prep_inputs(int64_t n, const float* __restrict__ X, const float* __restrict__ mu,
+                              const float* __restrict__ sd, uint16_t* __restrict__ Xb) {
     const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= n * MlpDims::IN) return;
-    const int64_t r = t / MlpDims::IN;
     const int c = (int)(t % MlpDims::IN);
-    const int64_t src = idx ? idx[r] : r;
-    Xb[t] = to_bf16((X[src * MlpDims::IN + c] - mu[c]) / sd[c]);
+    Xb[t] = to_bf16((X[t] - mu[c]) / sd[c]);
 }
 
-// targets -> normalised f32 rows (OUTP wide, padding zero)
-__global__ void k_prep_targets(int64_t n, const float* __restrict__ Y, const int64_t* __restrict__ idx,
-                               const float* __restrict__ mu, const float* __restrict__ sd, float* __restrict__ T) {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= n * MlpDims::OUTP) return;
-    const int64_t r = t / MlpDims::OUTP;
-    const int c = (int)(t % MlpDims::OUTP);
-    const int64_t src = idx ? idx[r] : r;
-    T[t] = c < MlpDims::OUT ? (Y[src * MlpDims::OUT + c] - mu[c]) / sd[c] : 0.f;
-}
-
-// dY = 2 (Yp - T) / (n * OUT) on the real outputs, and per-block sums of the squared error
-__global__ void k_mse_grad(int64_t n, const float* __restrict__ Yp, const float* __restrict__ T,
-                           uint16_t* __restrict__ dYb, float* __restrict__ dY, float* __restrict__ partial) {
-    __shared__ float red[256];
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    float se = 0.f;
-    if (t < n * MlpDims::OUTP) {
-        const int c = (int)(t % MlpDims::OUTP);
-        float g = 0.f;
-        if (c < MlpDims::OUT) {
-            const float d = Yp[t] - T[t];
-            se = d * d;
-            g = 2.f * d / (float)(n * MlpDims::OUT);
-        }
-        dYb[t] = to_bf16(g);
-        if (dY) dY[t] = g;
-    }
-    red[threadIdx.x] = se;
-    __syncthreads();
-    for (int o = 128; o > 0; o >>= 1) {
-        if ((int)threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) partial[blockIdx.x] = red[0];
-}
-
-// Column sums of a bf16 matrix (rows x cols, cols dividing 256) into f32 (bias gradients),
-// in two fixed-order passes: workgroup b sums rows [b R, (b + 1) R) with the 256 / cols
-// threads of each column reading interleaved rows (a row's columns are read together, so
-// the loads are coalesced; eight loads in flight per thread), then one workgroup per
-// column adds the per-workgroup sums (each thread a strided subset, then a fixed-order
-// block sum).
-constexpr int kColsumBlocks = 512;
-__global__ void __launch_bounds__(256) k_colsum_part(int64_t rows, int cols, int64_t R,
-                                                     const uint16_t* __restrict__ D, float* __restrict__ part) {
-    __shared__ float red[256];
-    const int c = threadIdx.x % cols, lanes = 256 / cols, sub = threadIdx.x / cols;
-    const int64_t r0 = (int64_t)blockIdx.x * R, r1 = min(rows, r0 + R);
-    float s = 0.f;
-    int64_t r = r0 + sub;
-    for (; r + 7 * lanes < r1; r += 8 * lanes) {
-        uint16_t v[8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) v[u] = D[(r + u * lanes) * cols + c];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) s += __uint_as_float((uint32_t)v[u] << 16);
-    }
-    for (; r < r1; r += lanes) s += __uint_as_float((uint32_t)D[r * cols + c] << 16);
-    red[threadIdx.x] = s;
-    __syncthreads();
-    if (threadIdx.x < cols) {
-        float t = 0.f;
-        for (int k = 0; k < lanes; ++k) t += red[k * cols + threadIdx.x];
-        part[(int64_t)blockIdx.x * cols + threadIdx.x] = t;
-    }
-}
-__global__ void __launch_bounds__(256) k_colsum_final(int nb, int cols, const float* __restrict__ part,
-                                                      float* __restrict__ out) {
-    __shared__ float red[256];
-    const int c = blockIdx.x;
-    float t = 0.f;
-    for (int b = threadIdx.x; b < nb; b += 256) t += part[(int64_t)b * cols + c];
-    red[threadIdx.x] = t;
-    __syncthreads();
-    for (int o = 128; o > 0; o >>= 1) {
-        if ((int)threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) out[c] = red[0];
-}
-
-// *acc += scale * (sum of the partials, in a fixed order): one workgroup
-__global__ void __launch_bounds__(256) k_loss_accum(int64_t nb, const float* __restrict__ partial, double scale,
-                                                    double* __restrict__ acc) {
-    __shared__ double red[256];
-    double s = 0;
-    for (int64_t k = threadIdx.x; k < nb; k += 256) s += partial[k];
-    red[threadIdx.x] = s;
-    __syncthreads();
-    for (int o = 128; o > 0; o >>= 1) {
-        if ((int)threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) *acc += red[0] * scale;
-}
-
-// Adam over all eight parameter tensors (four weight matrices, four bias vectors) in one
-// launch: element t belongs to segment k with off[k] <= t < off[k + 1]
-struct AdamSegs {
-    float* p[8];
-    float* m[8];
-    float* v[8];
-    const float* g[8];
-    uint16_t* pb[8];
-    const uint8_t* keep[8];
-    int64_t off[9];
-};
-__global__ void k_adam_all(AdamSegs a, float lr, float b1, float b2, float eps, float c1, float c2) {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= a.off[8]) return;
-    int k = 0;
-#pragma unroll
-    for (int j = 1; j < 8; ++j) k += t >= a.off[j] ? 1 : 0;
-    const int64_t i = t - a.off[k];
-    if (a.keep[k] && !a.keep[k][i]) return;
-    const float gt = a.g[k][i];
-    const float mt = b1 * a.m[k][i] + (1.f - b1) * gt;
-    const float vt = b2 * a.v[k][i] + (1.f - b2) * gt * gt;
-    a.m[k][i] = mt;
-    a.v[k][i] = vt;
-    const float pt = a.p[k][i] - lr * (mt / c1) / (sqrtf(vt / c2) + eps);
-    a.p[k][i] = pt;
-    if (a.pb[k]) a.pb[k][i] = to_bf16(pt);
-}
-
-__global__ void k_to_bf16(int64_t n, const float* __restrict__ a, uint16_t* __restrict__ b) {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t < n) b[t] = to_bf16(a[t]);
+// BF16 copies of one layer's weights W [dout x din]: as they are, and transposed
+__global__ void k_pack_weights(int din, int dout, const float* __restrict__ W, uint16_t* __restrict__ Wb,
+                               uint16_t* __restrict__ WbT) {
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= din * dout) return;
+    const uint16_t v = to_bf16(W[t]);
+    Wb[t] = v;
+    WbT[(t % din) * dout + t / din] = v;
 }
 
 // de-normalise network outputs (OUTP wide) into OUT-wide rows
@@ -497,14 +287,334 @@ __global__ void __launch_bounds__(kInferThreads) k_mlp_infer(InferArgs p) {
     }
 }
 
-__global__ void k_sample_idx(int64_t nb, int64_t n, uint64_t key, int64_t* idx) {
-    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= nb) return;
+// Row t of a training batch: a counter hash of the batch key, modulo the sample count.
+__device__ __forceinline__ int64_t sample_row(uint64_t key, int64_t t, int64_t n) {
     uint64_t z = key + (uint64_t)t * 0x9E3779B97F4A7C15ull;
     z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
     z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
     z ^= z >> 31;
-    idx[t] = (int64_t)(z % (uint64_t)n);
+    return (int64_t)(z % (uint64_t)n);
+}
+
+// Forward, loss and backward of a training batch in one launch.
+//
+// A workgroup of eight waves takes tiles of 64 samples; wave w owns the 16 hidden features
+// 16 w .. + 15 of every layer.  Its weight fragments (W for the forward products, W^T for the
+// backward ones) and its rows of every weight gradient stay in registers for all of the
+// workgroup's tiles (the latter as MFMA accumulators), so per tile only activations and
+// back-propagated gradients pass through LDS: once as [sample][feature], the B operand of the
+// next product, and once as [feature][sample], the operands of dW = dZ^T A (k = samples).  A
+// bias gradient is the product of dZ^T with a vector of ones.  The ReLU masks stay in the
+// registers of the lane that computed them.  Each workgroup writes its gradients to a slab of
+// its own; k_mlp_update adds the slabs in a fixed order, so results do not depend on
+// scheduling.
+//
+// Bound: LDS reads and the nine barriers of a tile (a tile's 900 MFMAs take about 3 us on a
+// CU), then the slabs (149 KB per workgroup).  A batch of 8,192 took 215 us in 29 launches
+// (11 GEMMs of 13 us, split-K and column sums, one launch per elementwise step); it takes
+// 27.7 us here and 7.0 us in k_mlp_update.
+constexpr int kTrainCols = 64;
+constexpr int kTrainThreads = 512;
+constexpr int kLs = MlpDims::H + 8;      // LDS row stride (BF16) of [sample][128 features]
+constexpr int kLt = kTrainCols + 8;      // of [feature][64 samples]
+constexpr int kLx = MlpDims::IN + 8;     // of [sample][16 features]
+// flat parameters: W1 b1 W2 b2 W3 b3 W4 b4
+constexpr int kOffW[4] = {0, 2176, 18688, 35200}, kOffB[4] = {2048, 18560, 35072, 37248};
+constexpr int kParams = 37264;
+
+struct TrainArgs {
+    int64_t n;        // samples of the batch
+    int64_t total;    // > 0: batch row t is sample_row(key, t, total) of X / Y; 0: row t itself
+    uint64_t key;
+    const float *X, *Y;
+    const float* norm;
+    const uint16_t *W[4], *WT[4];  // BF16 [dout x din] and [din x dout]
+    const float* b[4];
+    float* slab;   // [gridDim.x][kParams]
+    double* loss;  // [gridDim.x] summed squared error
+};
+
+__device__ __forceinline__ uint16_t bf16_bits(float f) { return __builtin_bit_cast(uint16_t, (__bf16)f); }
+
+// four consecutive features of one sample to both layouts
+__device__ __forceinline__ void put4(const float (&v)[4], uint16_t* __restrict__ s, uint16_t* __restrict__ t) {
+    typedef uint16_t u16x4 __attribute__((ext_vector_type(4)));
+    u16x4 u;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) u[j] = bf16_bits(v[j]);
+    if (s) *reinterpret_cast<u16x4*>(s) = u;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) t[j * kLt] = u[j];
+}
+
+__global__ void __launch_bounds__(kTrainThreads) k_mlp_train(TrainArgs p) {
+    constexpr int H = MlpDims::H, IN = MlpDims::IN, OUT = MlpDims::OUT, OUTP = MlpDims::OUTP;
+    constexpr int T = kTrainCols;
+    __shared__ __align__(16) uint16_t xs[T * kLx], xt[IN * kLt];
+    __shared__ __align__(16) uint16_t as[2][T * kLs];   // activations / gradients by sample, in turn
+    __shared__ __align__(16) uint16_t at[3][H * kLt];   // activations of the hidden layers by feature
+    __shared__ __align__(16) uint16_t dt[2][H * kLt];   // gradients by feature, in turn
+    __shared__ __align__(16) uint16_t ds4[T * kLx], dt4[OUTP * kLt];
+    __shared__ __align__(16) float bias[3 * H + OUTP];
+    __shared__ int64_t src[T];
+    __shared__ double s_loss[4];
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, r = lane & 15, q = lane >> 4;
+    const int f0 = 16 * w + 4 * q;  // the lane's first output feature
+    const bf16x8 zero8 = {};
+    bf16x8 ones;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) ones[j] = (__bf16)1.0f;
+    // weight fragments of this wave (rows 16 w .. of W, and of W^T)
+    const bf16x8 w1 = q < 2 ? frag8(p.W[0] + (16 * w + r) * IN + 8 * q) : zero8;
+    const bf16x8 t4 = q < 2 ? frag8(p.WT[3] + (16 * w + r) * OUTP + 8 * q) : zero8;
+    bf16x8 w2[4], w3[4], t2[4], t3[4];
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+        const int o = (16 * w + r) * H + 32 * ks + 8 * q;
+        w2[ks] = frag8(p.W[1] + o);
+        w3[ks] = frag8(p.W[2] + o);
+        t2[ks] = frag8(p.WT[1] + o);
+        t3[ks] = frag8(p.WT[2] + o);
+    }
+    for (int e = tid; e < 3 * H + OUTP; e += kTrainThreads) bias[e] = p.b[e / H][e % H];
+    auto bias_of = [&](int l) { return *reinterpret_cast<const f32x4*>(&bias[l * H + (l < 3 ? f0 : 4 * q)]); };
+    const f32x4 zero4 = {0.f, 0.f, 0.f, 0.f};
+    f32x4 g1 = zero4, g2[8], g3[8], g4 = zero4, gb1 = zero4, gb2 = zero4, gb3 = zero4, gb4 = zero4;
+#pragma unroll
+    for (int c = 0; c < 8; ++c) g2[c] = g3[c] = zero4;
+    double se = 0.0;
+
+    // Z = W A + b of 16 features x 64 samples; relu to both layouts; the mask Z > 0, bit 4 cb + j
+    auto forward = [&](const bf16x8 (&wk)[4], f32x4 bias, const uint16_t* in, uint16_t* os, uint16_t* ot) {
+        uint32_t mask = 0;
+#pragma unroll
+        for (int cb = 0; cb < 4; ++cb) {
+            f32x4 acc = bias;
+#pragma unroll
+            for (int ks = 0; ks < 4; ++ks)
+                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wk[ks], frag8(in + (16 * cb + r) * kLs + 32 * ks + 8 * q),
+                                                              acc, 0, 0, 0);
+            float v[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                mask |= (acc[j] > 0.f ? 1u : 0u) << (4 * cb + j);
+                v[j] = fmaxf(acc[j], 0.f);
+            }
+            put4(v, os + (16 * cb + r) * kLs + f0, ot + f0 * kLt + 16 * cb + r);
+        }
+        return mask;
+    };
+    // dZ_in = (W^T dZ) masked, to both layouts (os may be null)
+    auto backward = [&](const bf16x8 (&tk)[4], uint32_t mask, const uint16_t* in, uint16_t* os, uint16_t* ot) {
+#pragma unroll
+        for (int cb = 0; cb < 4; ++cb) {
+            f32x4 acc = zero4;
+#pragma unroll
+            for (int ks = 0; ks < 4; ++ks)
+                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(tk[ks], frag8(in + (16 * cb + r) * kLs + 32 * ks + 8 * q),
+                                                              acc, 0, 0, 0);
+            float v[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) v[j] = (mask >> (4 * cb + j)) & 1u ? acc[j] : 0.f;
+            put4(v, os ? os + (16 * cb + r) * kLs + f0 : nullptr, ot + f0 * kLt + 16 * cb + r);
+        }
+        __builtin_amdgcn_sched_barrier(0);  // keeps the next phase's operand reads out of this one's registers
+    };
+    // rows 16 w .. of dW += dZ^T A over the tile's samples, and of db
+    auto weight_grad = [&](const uint16_t* dz, const uint16_t* a, f32x4 (&g)[8], f32x4& gb) {
+#pragma unroll
+        for (int ks = 0; ks < T / 32; ++ks) {
+            const bf16x8 d = frag8(dz + (16 * w + r) * kLt + 32 * ks + 8 * q);
+            gb = __builtin_amdgcn_mfma_f32_16x16x32_bf16(d, ones, gb, 0, 0, 0);
+#pragma unroll
+            for (int c = 0; c < 8; ++c)
+                g[c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(d, frag8(a + (16 * c + r) * kLt + 32 * ks + 8 * q), g[c],
+                                                               0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+
+    const int64_t ntiles = (p.n + T - 1) / T;
+    for (int64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+        if (tid < T) {
+            const int64_t row = tile * T + tid;
+            src[tid] = row >= p.n ? -1 : p.total > 0 ? sample_row(p.key, row, p.total) : row;
+        }
+        __syncthreads();  // the previous tile's readers are done, src is there
+        for (int e = tid; e < T * IN; e += kTrainThreads) {
+            const int s = e / IN, c = e % IN;
+            const int64_t g = src[s];
+            const uint16_t v = g >= 0 ? bf16_bits((p.X[g * IN + c] - p.norm[c]) / p.norm[IN + c]) : (uint16_t)0;
+            xs[s * kLx + c] = v;
+            xt[c * kLt + s] = v;
+        }
+        __syncthreads();
+        // ---- forward
+        uint32_t m1 = 0;
+#pragma unroll
+        for (int cb = 0; cb < 4; ++cb) {
+            const bf16x8 x = q < 2 ? frag8(xs + (16 * cb + r) * kLx + 8 * q) : zero8;
+            const f32x4 acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w1, x, bias_of(0), 0, 0, 0);
+            float v[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                m1 |= (acc[j] > 0.f ? 1u : 0u) << (4 * cb + j);
+                v[j] = fmaxf(acc[j], 0.f);
+            }
+            put4(v, as[0] + (16 * cb + r) * kLs + f0, at[0] + f0 * kLt + 16 * cb + r);
+        }
+        __syncthreads();
+        const uint32_t m2 = forward(w2, bias_of(1), as[0], as[1], at[1]);
+        __syncthreads();
+        const uint32_t m3 = forward(w3, bias_of(2), as[1], as[0], at[2]);
+        __syncthreads();
+        // ---- output layer, loss and its gradient: waves 0 .. 3, 16 samples each
+        if (w < 4) {
+            const int s = 16 * w + r;
+            const int64_t g = src[s];
+            f32x4 acc = bias_of(3);
+#pragma unroll
+            for (int ks = 0; ks < 4; ++ks)
+                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(frag8(p.W[3] + r * H + 32 * ks + 8 * q),
+                                                              frag8(as[0] + s * kLs + 32 * ks + 8 * q), acc, 0, 0, 0);
+            float v[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int o = 4 * q + j;
+                v[j] = 0.f;
+                if (o < OUT && g >= 0) {
+                    const float y = (p.Y[g * OUT + o] - p.norm[2 * IN + o]) / p.norm[2 * IN + OUT + o];
+                    const float d = acc[j] - y;
+                    se = fma((double)d, (double)d, se);
+                    v[j] = 2.f * d / (float)(p.n * OUT);
+                }
+            }
+            put4(v, ds4 + s * kLx + 4 * q, dt4 + 4 * q * kLt + s);
+        }
+        __syncthreads();
+        // ---- backward
+#pragma unroll
+        for (int cb = 0; cb < 4; ++cb) {
+            const bf16x8 d = q < 2 ? frag8(ds4 + (16 * cb + r) * kLx + 8 * q) : zero8;
+            const f32x4 acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(t4, d, zero4, 0, 0, 0);
+            float v[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) v[j] = (m3 >> (4 * cb + j)) & 1u ? acc[j] : 0.f;
+            put4(v, as[1] + (16 * cb + r) * kLs + f0, dt[0] + f0 * kLt + 16 * cb + r);
+        }
+#pragma unroll
+        for (int ks = 0; ks < T / 32; ++ks) {
+            const bf16x8 d = frag8(dt4 + r * kLt + 32 * ks + 8 * q);
+            g4 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(d, frag8(at[2] + (16 * w + r) * kLt + 32 * ks + 8 * q), g4, 0, 0,
+                                                         0);
+            gb4 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(d, ones, gb4, 0, 0, 0);
+        }
+        __syncthreads();
+        backward(t3, m2, as[1], as[0], dt[1]);
+        weight_grad(dt[0], at[1], g3, gb3);
+        __syncthreads();
+        backward(t2, m1, as[0], nullptr, dt[0]);
+        weight_grad(dt[1], at[0], g2, gb2);
+        __syncthreads();
+#pragma unroll
+        for (int ks = 0; ks < T / 32; ++ks) {
+            const bf16x8 d = frag8(dt[0] + (16 * w + r) * kLt + 32 * ks + 8 * q);
+            g1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(d, frag8(xt + r * kLt + 32 * ks + 8 * q), g1, 0, 0, 0);
+            gb1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(d, ones, gb1, 0, 0, 0);
+        }
+        __syncthreads();  // src and xs are rewritten next
+    }
+    // ---- this workgroup's slab
+    float* sl = p.slab + (size_t)blockIdx.x * kParams;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        sl[kOffW[0] + (f0 + j) * IN + r] = g1[j];
+        sl[kOffW[3] + (4 * q + j) * H + 16 * w + r] = g4[j];
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+            sl[kOffW[1] + (f0 + j) * H + 16 * c + r] = g2[c][j];
+            sl[kOffW[2] + (f0 + j) * H + 16 * c + r] = g3[c][j];
+        }
+        if (r == 0) {
+            sl[kOffB[0] + f0 + j] = gb1[j];
+            sl[kOffB[1] + f0 + j] = gb2[j];
+            sl[kOffB[2] + f0 + j] = gb3[j];
+            if (w == 0) sl[kOffB[3] + 4 * q + j] = gb4[j];
+        }
+    }
+    if (w < 4) {
+        se = wave_sum(se);
+        if (lane == 0) s_loss[w] = se;
+    }
+    __syncthreads();
+    if (tid == 0) p.loss[blockIdx.x] = s_loss[0] + s_loss[1] + s_loss[2] + s_loss[3];
+}
+
+// Sums the slabs of a batch in a fixed order (eight interleaved groups, then the groups in
+// order), and steps Adam with the sums or writes them out (ADAM = false).  Eight threads per
+// parameter keep enough loads in flight to read the slabs at memory rate.
+struct UpdateArgs {
+    const float* slab;
+    int nslab;
+    const double* loss;
+    double loss_scale;
+    double* loss_acc;  // += loss_scale * (sum of loss[])
+    float *p[8], *m[8], *v[8], *g[8];  // W1 b1 W2 b2 W3 b3 W4 b4
+    uint16_t *pb[4], *pbT[4];          // BF16 weights and their transposes
+    int off[9];
+    float lr, c1, c2;
+};
+constexpr int kUpdCols = 32, kUpdGroups = 8;
+template <bool ADAM>
+__global__ void __launch_bounds__(kUpdCols* kUpdGroups) k_mlp_update(UpdateArgs a) {
+    __shared__ float red[kUpdGroups][kUpdCols];
+    const int col = threadIdx.x % kUpdCols, grp = threadIdx.x / kUpdCols;
+    const int t = blockIdx.x * kUpdCols + col;
+    float acc = 0.f;
+    if (t < kParams) {
+        int s = grp;
+        for (; s + 7 * kUpdGroups < a.nslab; s += 8 * kUpdGroups) {
+            float v[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) v[u] = a.slab[(size_t)(s + u * kUpdGroups) * kParams + t];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) acc += v[u];
+        }
+        for (; s < a.nslab; s += kUpdGroups) acc += a.slab[(size_t)s * kParams + t];
+    }
+    red[grp][col] = acc;
+    __syncthreads();
+    if (blockIdx.x == 0 && threadIdx.x < 64) {
+        double e = 0;
+        for (int k = threadIdx.x; k < a.nslab; k += 64) e += a.loss[k];
+        e = wave_sum(e);
+        if (threadIdx.x == 0) *a.loss_acc += e * a.loss_scale;
+    }
+    if (grp != 0 || t >= kParams) return;
+    float gt = red[0][col];
+#pragma unroll
+    for (int k = 1; k < kUpdGroups; ++k) gt += red[k][col];
+    int seg = 0;
+#pragma unroll
+    for (int j = 1; j < 8; ++j) seg += t >= a.off[j] ? 1 : 0;
+    const int i = t - a.off[seg];
+    if constexpr (ADAM) {
+        const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
+        const float mt = b1 * a.m[seg][i] + (1.f - b1) * gt;
+        const float vt = b2 * a.v[seg][i] + (1.f - b2) * gt * gt;
+        a.m[seg][i] = mt;
+        a.v[seg][i] = vt;
+        const float pt = a.p[seg][i] - a.lr * (mt / a.c1) / (sqrtf(vt / a.c2) + eps);
+        a.p[seg][i] = pt;
+        if ((seg & 1) == 0) {
+            const int l = seg >> 1, din = l == 0 ? MlpDims::IN : MlpDims::H, dout = l == 3 ? MlpDims::OUTP : MlpDims::H;
+            const uint16_t v = to_bf16(pt);
+            a.pb[l][i] = v;
+            a.pbT[l][(i % din) * dout + i / din] = v;
+        }
+    } else {
+        a.g[seg][i] = gt;
+    }
 }
 
 unsigned g1(int64_t n) { return (unsigned)((n + 255) / 256); }
@@ -528,6 +638,7 @@ Mlp::Mlp(int device_, uint64_t seed) : device(device_) {
             for (int i = 0; i < di; ++i) w[(size_t)o * di + i] = (l == 3 && o >= MlpDims::OUT) ? 0.f : (float)(nd(rng) * sc);
         W[l].alloc(w.size());
         Wb[l].alloc(w.size());
+        WbT[l].alloc(w.size());
         bvec[l].alloc(dn);
         gW[l].alloc(w.size());
         gb[l].alloc(dn);
@@ -539,24 +650,17 @@ Mlp::Mlp(int device_, uint64_t seed) : device(device_) {
         PB_HIP(hipMemcpyAsync(bvec[l].p, b.data(), b.size() * 4, hipMemcpyHostToDevice, stream));
         for (auto* d : {&mW[l], &vW[l]}) PB_HIP(hipMemsetAsync(d->p, 0, d->bytes(), stream));
         for (auto* d : {&mb[l], &vb[l]}) PB_HIP(hipMemsetAsync(d->p, 0, d->bytes(), stream));
-        hipLaunchKernelGGL(k_to_bf16, dim3(g1(w.size())), dim3(256), 0, stream, (int64_t)w.size(), W[l].p, Wb[l].p);
+        hipLaunchKernelGGL(k_pack_weights, dim3(g1(w.size())), dim3(256), 0, stream, di, dn, W[l].p, Wb[l].p, WbT[l].p);
     }
-    // output rows >= OUT stay zero: mask their updates
-    std::vector<uint8_t> keep((size_t)MlpDims::OUTP * MlpDims::H, 1), keepb(MlpDims::OUTP, 1);
-    for (int o = MlpDims::OUT; o < MlpDims::OUTP; ++o) {
-        keepb[o] = 0;
-        for (int i = 0; i < MlpDims::H; ++i) keep[(size_t)o * MlpDims::H + i] = 0;
-    }
-    keepW4.alloc(keep.size());
-    keepb4.alloc(keepb.size());
-    PB_HIP(hipMemcpyAsync(keepW4.p, keep.data(), keep.size(), hipMemcpyHostToDevice, stream));
-    PB_HIP(hipMemcpyAsync(keepb4.p, keepb.data(), keepb.size(), hipMemcpyHostToDevice, stream));
-    std::vector<float> one(32, 1.f), zero(32, 0.f);
     norm.alloc(2 * MlpDims::IN + 2 * MlpDims::OUT);
     std::vector<float> nrm(norm.n, 0.f);
     for (int c = 0; c < MlpDims::IN; ++c) nrm[MlpDims::IN + c] = 1.f;
     for (int c = 0; c < MlpDims::OUT; ++c) nrm[2 * MlpDims::IN + MlpDims::OUT + c] = 1.f;
     PB_HIP(hipMemcpyAsync(norm.p, nrm.data(), nrm.size() * 4, hipMemcpyHostToDevice, stream));
+    loss_dev.alloc(1);
+    int cus = 0;
+    PB_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
+    max_blocks = cus > 0 ? cus : 256;  // one workgroup (eight waves) of either fused kernel per CU
     PB_HIP(hipStreamSynchronize(stream));
 }
 
@@ -568,19 +672,8 @@ void Mlp::ensure(int64_t n) {
     if (n <= cap) return;
     cap = n;
     Xb.alloc(n * MlpDims::IN);
-    for (int l = 0; l < 3; ++l) {
-        Z[l].alloc(n * MlpDims::H);
-        Ab[l].alloc(n * MlpDims::H);
-        dZb[l].alloc(n * MlpDims::H);
-    }
+    for (int l = 0; l < 3; ++l) Ab[l].alloc(n * MlpDims::H);
     Yp.alloc(n * MlpDims::OUTP);
-    Tn.alloc(n * MlpDims::OUTP);
-    dYb.alloc(n * MlpDims::OUTP);
-    idx.alloc(n);
-    partial.alloc(g1(n * MlpDims::OUTP) + 1);
-    if (!splitws.p) splitws.alloc((size_t)kMaxSplits * MlpDims::H * MlpDims::H);
-    if (!colpart.p) colpart.alloc((size_t)kColsumBlocks * MlpDims::H);
-    loss_dev.alloc(1);
 }
 
 const float* Mlp::xmu() const { return norm.p; }
@@ -588,8 +681,7 @@ const float* Mlp::xsd() const { return norm.p + MlpDims::IN; }
 const float* Mlp::ymu() const { return norm.p + 2 * MlpDims::IN; }
 const float* Mlp::ysd() const { return norm.p + 2 * MlpDims::IN + MlpDims::OUT; }
 
-void Mlp::forward_prepared(int64_t n, bool keep_z) {
-    hipStream_t s = stream;
+void Mlp::forward_prepared(int64_t n, hipStream_t s) {
     const uint16_t* in = Xb.p;
     for (int l = 0; l < 4; ++l) {
         GemmArgs g{};
@@ -597,125 +689,71 @@ void Mlp::forward_prepared(int64_t n, bool keep_z) {
         g.N = MlpDims::dout(l);
         g.K = MlpDims::din(l);
         g.A = in;
-        g.lda = MlpDims::din(l);
         g.B = Wb[l].p;
-        g.ldb = MlpDims::din(l);
-        g.transB = 1;
         g.bias = bvec[l].p;
-        if (l < 3) {
-            g.C = keep_z ? Z[l].p : nullptr;  // pre-activations: only the backward pass reads them
-            g.ldc = MlpDims::H;
-            g.relu = 1;
-            g.Cb = Ab[l].p;
-            g.ldcb = MlpDims::H;
-            in = Ab[l].p;
-        } else {
+        if (l < 3)
+            in = g.Cb = Ab[l].p;
+        else
             g.C = Yp.p;
-            g.ldc = MlpDims::OUTP;
-        }
-        gemm(s, g);
+        hipLaunchKernelGGL(k_gemm_bf16, dim3((g.N + TN - 1) / TN, (g.M + TM - 1) / TM), dim3(256), 0, s, g);
     }
 }
 
-double Mlp::backward_prepared(int64_t n, float* dY_f32, double* loss_acc) {
-    hipStream_t s = stream;
-    const unsigned nb = g1(n * MlpDims::OUTP);
-    hipLaunchKernelGGL(k_mse_grad, dim3(nb), dim3(256), 0, s, n, Yp.p, Tn.p, dYb.p, dY_f32, partial.p);
-    // weight gradients: K = n samples split into up to 64 slabs of >= 512 rows, so that the
-    // 128 x 128 outputs (4 tiles) still give 256 workgroups at a batch of 32,768
-    const int splits = (int)std::min<int64_t>(kMaxSplits, std::max<int64_t>(1, n / 512));
-    const uint16_t* dcur = dYb.p;  // gradient w.r.t. this layer's pre-activation (bf16)
-    for (int l = 3; l >= 0; --l) {
-        const int di = MlpDims::din(l), dn = MlpDims::dout(l);
-        const uint16_t* ain = l == 0 ? Xb.p : Ab[l - 1].p;
-        GemmArgs gw{};  // gW = dZ^T A_in  (M=dout, N=din, K=n)
-        gw.M = dn;
-        gw.N = di;
-        gw.K = (int)n;
-        gw.A = dcur;
-        gw.lda = dn;
-        gw.transA = 1;
-        gw.B = ain;
-        gw.ldb = di;
-        gw.C = gW[l].p;
-        gw.ldc = di;
-        gemm(s, gw, splits, splitws.p);
-        {
-            const int64_t R = std::max<int64_t>(64, (n + kColsumBlocks - 1) / kColsumBlocks);
-            const int nbk = (int)((n + R - 1) / R);
-            hipLaunchKernelGGL(k_colsum_part, dim3(nbk), dim3(256), 0, s, n, dn, R, dcur, colpart.p);
-            hipLaunchKernelGGL(k_colsum_final, dim3(dn), dim3(256), 0, s, nbk, dn, colpart.p, gb[l].p);
-        }
-        if (l > 0) {  // dZ_{l-1} = (dZ W) * [Z_{l-1} > 0]   (M=n, N=din, K=dout)
-            GemmArgs gd{};
-            gd.M = (int)n;
-            gd.N = di;
-            gd.K = dn;
-            gd.A = dcur;
-            gd.lda = dn;
-            gd.B = Wb[l].p;
-            gd.ldb = di;
-            gd.mask = Z[l - 1].p;
-            gd.ldc = di;
-            gd.Cb = dZb[l - 1].p;
-            gd.ldcb = di;
-            gemm(s, gd);
-            dcur = dZb[l - 1].p;
-        }
+void Mlp::batch_pass(const float* X, const float* Y, int64_t n, int64_t total, uint64_t key, bool adam, float lr) {
+    const int64_t tiles = (n + kTrainCols - 1) / kTrainCols;
+    const int blocks = (int)std::min<int64_t>(tiles, max_blocks);
+    if (slab.n < (size_t)blocks * kParams) {
+        slab.alloc((size_t)blocks * kParams);
+        loss_part.alloc(blocks);
     }
-    if (loss_acc) {  // training: the batch loss is added on the device, no host round trip per batch
-        hipLaunchKernelGGL(k_loss_accum, dim3(1), dim3(256), 0, s, (int64_t)nb, partial.p, 1.0 / (double)(n * MlpDims::OUT),
-                           loss_acc);
-        return 0.0;
-    }
-    std::vector<float> hp(nb);
-    PB_HIP(hipMemcpyAsync(hp.data(), partial.p, nb * sizeof(float), hipMemcpyDeviceToHost, s));
-    PB_HIP(hipStreamSynchronize(s));
-    double se = 0;
-    for (float v : hp) se += v;
-    return se / (double)(n * MlpDims::OUT);
-}
-
-void Mlp::adam_step(float lr) {
-    ++t_adam;
-    const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
-    const float c1 = 1.f - std::pow(b1, (float)t_adam), c2 = 1.f - std::pow(b2, (float)t_adam);
-    AdamSegs a{};
-    a.off[0] = 0;
+    TrainArgs a{};
+    a.n = n;
+    a.total = total;
+    a.key = key;
+    a.X = X;
+    a.Y = Y;
+    a.norm = norm.p;
+    UpdateArgs u{};
+    u.off[0] = 0;
     for (int l = 0; l < 4; ++l) {
-        const int64_t nw = (int64_t)MlpDims::din(l) * MlpDims::dout(l), nbias = MlpDims::dout(l);
+        a.W[l] = u.pb[l] = Wb[l].p;
+        a.WT[l] = u.pbT[l] = WbT[l].p;
+        a.b[l] = bvec[l].p;
         const int kw = 2 * l, kb = 2 * l + 1;
-        a.p[kw] = W[l].p, a.m[kw] = mW[l].p, a.v[kw] = vW[l].p, a.g[kw] = gW[l].p, a.pb[kw] = Wb[l].p;
-        a.keep[kw] = l == 3 ? keepW4.p : nullptr;
-        a.off[kw + 1] = a.off[kw] + nw;
-        a.p[kb] = bvec[l].p, a.m[kb] = mb[l].p, a.v[kb] = vb[l].p, a.g[kb] = gb[l].p, a.pb[kb] = nullptr;
-        a.keep[kb] = l == 3 ? keepb4.p : nullptr;
-        a.off[kb + 1] = a.off[kb] + nbias;
+        u.p[kw] = W[l].p, u.m[kw] = mW[l].p, u.v[kw] = vW[l].p, u.g[kw] = gW[l].p;
+        u.p[kb] = bvec[l].p, u.m[kb] = mb[l].p, u.v[kb] = vb[l].p, u.g[kb] = gb[l].p;
+        u.off[kw + 1] = u.off[kw] + MlpDims::din(l) * MlpDims::dout(l);
+        u.off[kb + 1] = u.off[kb] + MlpDims::dout(l);
     }
-    hipLaunchKernelGGL(k_adam_all, dim3(g1(a.off[8])), dim3(256), 0, stream, a, lr, b1, b2, eps, c1, c2);
-}
-
-void Mlp::prepare(const float* X, const float* Y, int64_t n, const int64_t* rows) {
-    ensure(n);
-    hipLaunchKernelGGL(k_prep_inputs, dim3(g1(n * MlpDims::IN)), dim3(256), 0, stream, n, X, rows, xmu(), xsd(), Xb.p);
-    if (Y)
-        hipLaunchKernelGGL(k_prep_targets, dim3(g1(n * MlpDims::OUTP)), dim3(256), 0, stream, n, Y, rows, ymu(), ysd(),
-                           Tn.p);
+    a.slab = slab.p;
+    a.loss = loss_part.p;
+    u.slab = slab.p;
+    u.nslab = blocks;
+    u.loss = loss_part.p;
+    u.loss_scale = 1.0 / (double)(n * MlpDims::OUT);
+    u.loss_acc = loss_dev.p;
+    hipLaunchKernelGGL(k_mlp_train, dim3(blocks), dim3(kTrainThreads), 0, stream, a);
+    const dim3 ug((kParams + kUpdCols - 1) / kUpdCols), ub(kUpdCols * kUpdGroups);
+    if (adam) {
+        ++t_adam;
+        u.lr = lr;
+        u.c1 = 1.f - std::pow(0.9f, (float)t_adam);
+        u.c2 = 1.f - std::pow(0.999f, (float)t_adam);
+        hipLaunchKernelGGL(k_mlp_update<true>, ug, ub, 0, stream, u);
+    } else {
+        hipLaunchKernelGGL(k_mlp_update<false>, ug, ub, 0, stream, u);
+    }
+    PB_HIP(hipGetLastError());
 }
 
 double Mlp::train(const float* X, const float* Y, int64_t n, int epochs, int batch, float lr, uint64_t seed) {
-    ensure(batch);
     const int64_t per_epoch = (n + batch - 1) / batch;
     double loss = 0;
     for (int e = 0; e < epochs; ++e) {
         PB_HIP(hipMemsetAsync(loss_dev.p, 0, sizeof(double), stream));
         for (int64_t b = 0; b < per_epoch; ++b) {
             const uint64_t key = seed * 0x9E3779B97F4A7C15ull + (uint64_t)(e * per_epoch + b) * 0xD1B54A32D192ED03ull;
-            hipLaunchKernelGGL(k_sample_idx, dim3(g1(batch)), dim3(256), 0, stream, (int64_t)batch, n, key, idx.p);
-            prepare(X, Y, batch, idx.p);
-            forward_prepared(batch);
-            backward_prepared(batch, nullptr, loss_dev.p);
-            adam_step(lr);
+            batch_pass(X, Y, batch, n, key, true, lr);
         }
         double acc = 0;
         PB_HIP(hipMemcpyAsync(&acc, loss_dev.p, sizeof(double), hipMemcpyDeviceToHost, stream));
@@ -724,16 +762,6 @@ double Mlp::train(const float* X, const float* Y, int64_t n, int epochs, int bat
     }
     PB_HIP(hipStreamSynchronize(stream));
     return loss;
-}
-
-bool Mlp::fused_inference_ok() {
-    if (fused_ok < 0) {
-        int cus = 0;
-        PB_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
-        infer_blocks = cus > 0 ? cus : 256;  // one workgroup (eight waves) per CU
-        fused_ok = 1;
-    }
-    return fused_ok == 1;
 }
 
 void Mlp::predict_fused(const float* X, float* Y, int64_t n, hipStream_t s) {
@@ -748,34 +776,23 @@ void Mlp::predict_fused(const float* X, float* Y, int64_t n, hipStream_t s) {
     a.Y = Y;
     a.x16 = ((uintptr_t)X & 15) == 0;
     const int64_t tiles = (n + kInferCols - 1) / kInferCols;
-    const unsigned grid = (unsigned)std::min<int64_t>(tiles, infer_blocks);
+    const unsigned grid = (unsigned)std::min<int64_t>(tiles, max_blocks);
     hipLaunchKernelGGL(k_mlp_infer, dim3(grid), dim3(kInferThreads), 0, s, a);
     PB_HIP(hipGetLastError());
 }
 
-void Mlp::predict(const float* X, float* Y, int64_t n, hipStream_t s) {
-    if (n <= 0) return;
-    if (fused_inference_ok()) {
-        predict_fused(X, Y, n, s);
-        return;
-    }
-    // layer by layer: runs on the caller's stream, chunked so that the workspace stays bounded
-    predict_layers(X, Y, n, s);
-}
-
+// layer by layer on the caller's stream, chunked so that the workspace stays bounded
 void Mlp::predict_layers(const float* X, float* Y, int64_t n, hipStream_t s) {
-    const hipStream_t own = stream;
-    stream = s;
     const int64_t chunk = 1 << 20;
     for (int64_t o = 0; o < n; o += chunk) {
         const int64_t m = std::min(chunk, n - o);
         ensure(m);
-        prepare(X + o * MlpDims::IN, nullptr, m, nullptr);
-        forward_prepared(m, false);
-        hipLaunchKernelGGL(k_denorm, dim3(g1(m * MlpDims::OUT)), dim3(256), 0, stream, m, Yp.p, ymu(), ysd(),
+        hipLaunchKernelGGL(k_prep_inputs, dim3(g1(m * MlpDims::IN)), dim3(256), 0, s, m, X + o * MlpDims::IN, xmu(),
+                           xsd(), Xb.p);
+        forward_prepared(m, s);
+        hipLaunchKernelGGL(k_denorm, dim3(g1(m * MlpDims::OUT)), dim3(256), 0, s, m, Yp.p, ymu(), ysd(),
                            Y + o * MlpDims::OUT);
     }
-    stream = own;
 }
 
 int64_t Mlp::param_count() {
@@ -804,7 +821,8 @@ void Mlp::set_params(const float* host) {
         o += nw;
         PB_HIP(hipMemcpyAsync(bvec[l].p, host + o, nb * 4, hipMemcpyHostToDevice, stream));
         o += nb;
-        hipLaunchKernelGGL(k_to_bf16, dim3(g1(nw)), dim3(256), 0, stream, nw, W[l].p, Wb[l].p);
+        hipLaunchKernelGGL(k_pack_weights, dim3(g1(nw)), dim3(256), 0, stream, MlpDims::din(l), MlpDims::dout(l), W[l].p,
+                           Wb[l].p, WbT[l].p);
     }
     PB_HIP(hipStreamSynchronize(stream));
 }
@@ -820,9 +838,11 @@ double Mlp::gradients(const float* Xh, const float* Yh, int64_t n, float* grads_
     Y.alloc(n * MlpDims::OUT);
     PB_HIP(hipMemcpyAsync(X.p, Xh, X.bytes(), hipMemcpyHostToDevice, stream));
     PB_HIP(hipMemcpyAsync(Y.p, Yh, Y.bytes(), hipMemcpyHostToDevice, stream));
-    prepare(X.p, Y.p, n, nullptr);
-    forward_prepared(n);
-    const double loss = backward_prepared(n, nullptr);
+    PB_HIP(hipMemsetAsync(loss_dev.p, 0, sizeof(double), stream));
+    batch_pass(X.p, Y.p, n, 0, 0, false, 0.f);
+    double loss = 0;
+    PB_HIP(hipMemcpyAsync(&loss, loss_dev.p, sizeof(double), hipMemcpyDeviceToHost, stream));
+    PB_HIP(hipStreamSynchronize(stream));
     if (grads_host) get_params(grads_host, true);
     return loss;
 }

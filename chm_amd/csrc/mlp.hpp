@@ -20,12 +20,13 @@ class Mlp {
     ~Mlp();
     // X: [n x IN] f32, Y: [n x OUT] f32 device arrays (raw units; normalised inside)
     double train(const float* X, const float* Y, int64_t n, int epochs, int batch, float lr, uint64_t seed);
-    // inference: the fused one-launch kernel (or layer by layer through the training
-    // GEMM; the two agree bit for bit)
-    void predict(const float* X, float* Y, int64_t n, hipStream_t s);
+    // inference: the fused one-launch kernel, or layer by layer through a GEMM (a check of the
+    // fused one: the two agree bit for bit)
+    void predict(const float* X, float* Y, int64_t n, hipStream_t s) {
+        if (n > 0) predict_fused(X, Y, n, s);
+    }
     void predict_fused(const float* X, float* Y, int64_t n, hipStream_t s);
     void predict_layers(const float* X, float* Y, int64_t n, hipStream_t s);
-    bool fused_inference_ok();
     double gradients(const float* Xh, const float* Yh, int64_t n, float* grads_host);  // MSE gradients, host arrays
     static int64_t param_count();
     void get_params(float* host, bool grads);
@@ -34,34 +35,28 @@ class Mlp {
 
     int device = 0;
     hipStream_t stream = nullptr;
-    int fused_ok = -1;       // fused inference set up on this device (-1: not yet)
-    int infer_blocks = 256;  // persistent grid of the fused inference (one workgroup per CU)
+    int max_blocks = 256;  // workgroups of the fused kernels (one per CU)
 
   private:
     void ensure(int64_t n);
-    void prepare(const float* X, const float* Y, int64_t n, const int64_t* rows);
-    // keep_z: also store the FP32 pre-activations of the hidden layers (for backward)
-    void forward_prepared(int64_t n, bool keep_z = true);
-    // loss_acc (device, may be null): the batch's mean squared error is added there on the
-    // device and 0 is returned; null: the loss is returned (a host round trip)
-    double backward_prepared(int64_t n, float* dY_f32, double* loss_acc = nullptr);
-    void adam_step(float lr);
+    void forward_prepared(int64_t n, hipStream_t s);
+    // gradients of one batch (total > 0: rows sampled from total by key), then an Adam step or
+    // the gradients into gW / gb; adds the batch's mean squared error to loss_dev
+    void batch_pass(const float* X, const float* Y, int64_t n, int64_t total, uint64_t key, bool adam, float lr);
     const float* xmu() const;
     const float* xsd() const;
     const float* ymu() const;
     const float* ysd() const;
 
     DevBuf<float> W[4], bvec[4], gW[4], gb[4], mW[4], vW[4], mb[4], vb[4];
-    DevBuf<uint16_t> Wb[4];
-    DevBuf<uint8_t> keepW4, keepb4;
+    DevBuf<uint16_t> Wb[4], WbT[4];  // BF16 weights [dout x din], and transposed
     DevBuf<float> norm;
     int64_t cap = 0;
-    DevBuf<uint16_t> Xb, Ab[3], dZb[3], dYb;
-    DevBuf<float> Z[3], Yp, Tn, partial;
-    DevBuf<float> splitws;  // split-K partial products of the weight gradients
-    DevBuf<float> colpart;  // per-workgroup column sums of the bias gradients
-    DevBuf<double> loss_dev;  // the epoch's summed batch losses (training)
-    DevBuf<int64_t> idx;
+    DevBuf<uint16_t> Xb, Ab[3];  // workspace of the layer-by-layer forward
+    DevBuf<float> Yp;
+    DevBuf<float> slab;        // gradients of one batch, one slab per workgroup
+    DevBuf<double> loss_part;  // summed squared error per workgroup
+    DevBuf<double> loss_dev;   // the epoch's summed batch losses
     int64_t t_adam = 0;
 };
 

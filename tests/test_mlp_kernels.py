@@ -46,3 +46,59 @@ def test_inference_matches_the_layer_by_layer_gemms(n, offset):
     rows = np.r_[0:k, n - k:n]
     ref = mlp_oracle.predict(p, X[rows], norm, bf16=True)
     assert np.abs(Y1.cpu().numpy()[rows] - ref).max() <= 1e-2 * np.abs(ref).max()
+
+
+# one 64-sample tile per workgroup, partial tiles, more tiles than workgroups (256 x 64 = 16384)
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 16, 63, 64, 65, 200, 4097, 16384, 16384 + 100, 3 * 16384 + 7])
+def test_gradients_match_the_reference(n):
+    print(f"[case] mlp gradients n={n}", flush=True)
+    rng = np.random.default_rng(100 + n)
+    net, p, norm = _net(6, rng)
+    X = (rng.normal(0, 1.5, (n, 16)) * norm[1] + norm[0]).astype(np.float32)
+    Y = rng.normal(0, 1, (n, 11)).astype(np.float32)
+    loss, g = net.gradients(X, Y)
+    rloss, rg = mlp_oracle.loss_and_grad(p, X, Y, norm, bf16=True)
+    # the bound of the whole-batch check: BF16 roundings that fall the other way after an FP32 sum
+    # in another order, 2^-9 of a value each
+    assert abs(loss - rloss) <= 1e-3 * rloss
+    o = 0
+    for r, c in mlp_oracle.SHAPES:
+        for size in (r * c, r):
+            a, b = g[o:o + size], rg[o:o + size]
+            assert np.linalg.norm(a - b) <= 2e-2 * np.linalg.norm(b) + 1e-7, (o, size)
+            o += size
+
+
+@pytest.mark.gpu
+def test_training_step_is_adam_on_the_sampled_rows():
+    """One batch of a one-batch epoch: the counter hash's rows, their gradient, Adam's first step."""
+    import torch
+
+    print("[case] mlp training step", flush=True)
+    n, seed, lr = 333, 9, 1e-3
+    rng = np.random.default_rng(7)
+    net, p, norm = _net(8, rng)
+    X = (rng.normal(0, 1.5, (n, 16)) * norm[1] + norm[0]).astype(np.float32)
+    Y = rng.normal(0, 1, (n, 11)).astype(np.float32)
+    loss = net.train(torch.tensor(X, device="cuda:0"), torch.tensor(Y, device="cuda:0"), epochs=1, batch=n, lr=lr,
+                     seed=seed)
+    m64, golden = (1 << 64) - 1, 0x9E3779B97F4A7C15
+
+    def row(t):
+        z = (seed * golden + t * golden) & m64
+        z = ((z ^ (z >> 30)) * 0xBF58476D1CE4E5B9) & m64
+        z = ((z ^ (z >> 27)) * 0x94D049BB133111EB) & m64
+        return (z ^ (z >> 31)) % n
+
+    rows = [row(t) for t in range(n)]
+    rloss, rg = mlp_oracle.loss_and_grad(p, X[rows], Y[rows], norm, bf16=True)
+    assert abs(loss - rloss) <= 1e-3 * rloss
+    step = net.get_params() - p
+    # Adam's first step is lr g / (|g| + eps): lr against the gradient's sign where it is not tiny
+    # (the parameter's own rounding: 2^-24 of values up to 1.5, 1e-4 of lr)
+    big = np.abs(rg) > 0.05 * np.abs(rg).max()
+    np.testing.assert_allclose(step[big], -lr * np.sign(rg[big]), rtol=1e-3)
+    # output rows past the eleven targets are never stepped
+    o = p.size - 16 * 128 - 16
+    assert np.all(step[o + 11 * 128:o + 16 * 128] == 0) and np.all(step[-5:] == 0)
