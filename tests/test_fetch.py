@@ -155,6 +155,54 @@ def test_gpu_fetch_matches_oracle(pb, oracle, mesh_c1, veg, kw):
     ctx.close()
 
 
+def _fetch_by_search(ctx, cx, cy, cz, can, cfg, vw):
+    """The fetch loop in numpy over the library's (brute-force checked) nearest-face search."""
+    b = vw * (math.pi / 180.0)
+    sb, cb = np.sin(b), np.cos(b)
+    out = np.full(len(cx), cfg.max_distance)
+    still = np.ones(len(cx), dtype=bool)
+    veg = can is not None and cfg.incl_veg
+    for j in range(1, cfg.steps + 1):
+        dist = j * (cfg.max_distance / cfg.steps)
+        f = ctx.nearest(cx + dist * sb, cy + dist * cb)
+        top = can[f] if veg else np.zeros(len(cx))
+        with np.errstate(divide="ignore", invalid="ignore"):
+            shelter = ((33.33333333 * 5 - 25.0 * 0.001) / (np.log(0.12 * top / 0.001) * 0.001)) ** (1 / 0.8) * 0.001
+        hit = still & ((cz[f] + top >= cz + dist * cfg.I) | ((dist < shelter) & (top > 0)))
+        out[hit] = dist
+        still &= ~hit
+    if veg:
+        out[can > 1] = 0.0
+    return out
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("points,veg,kw", [
+    (200500, True, {"steps": 23}), (200500, False, {}),  # more than 400,000 faces: the queue kernel
+    (3000, True, {"steps": 37, "I": 0.3}),
+    (3000, False, {"steps": 1}), (12, True, {"steps": 16, "max_distance": 20000.0}), (700, False, {"I": -0.5})])
+def test_gpu_fetch_lanes_and_cell_bounds(pb, points, veg, kw):
+    """Steps decided by a cell's bounds and steps that search give the same fetch as searching
+    at every step, by the queue or 16 lanes per face, step counts that do not fill the lanes,
+    sparse cells, and NaN heights (a face that never rises above the sight line)."""
+    print(f"[case] fetch lanes points={points} veg={veg} {kw}", flush=True)
+    cx, cy, cz = _centroids(meshgen.synthetic_mesh(points, seed=2))
+    F = len(cx)
+    rng = np.random.default_rng(points)
+    cz[rng.integers(0, F, max(1, F // 500))] = np.nan
+    can = np.where(rng.random(F) < 0.5, 0.0, rng.uniform(0.0, 1.3, F)) if veg else None
+    cfg = _fetch_cfg(**kw)
+    vw = rng.uniform(0.0, 360.0, F)
+    vw[::101] = np.nan
+    ctx = pb.Fetch(cx, cy, cz, can, cfg)
+    got = ctx.run(vw)
+    want = _fetch_by_search(ctx, cx, cy, cz, can, cfg, np.where(np.isnan(vw), 0.0, vw))
+    keep = np.zeros(F, dtype=bool) if can is None else (can > 1) & bool(cfg.incl_veg)
+    want = np.where(np.isnan(vw) & ~keep, cfg.max_distance, want)
+    np.testing.assert_array_equal(got, want)
+    ctx.close()
+
+
 @pytest.mark.gpu
 def test_gpu_fetch_device_arrays_feed_the_step(pb, oracle, mesh_c1):
     """fetch computed on the GPU from device-resident vw_dir, handed to the PBSM3D
