@@ -5,7 +5,9 @@
 // every face; k_smooth then gives each face the thin-plate-spline value of its
 // (at most three) neighbours' point-scaled winds at its own centroid
 // (scale_wind_vert.cpp:199-233, TPSpline.cpp:39-180): an (n+1) x (n+1) system
-// per face, solved in registers by Gaussian elimination with partial pivoting.
+// per face, solved in registers by Gaussian elimination with partial pivoting --
+// once per context, for the weights of the neighbours (k_weights), as it depends
+// on the mesh alone.
 // E1 (the reference takes GSL's gsl_sf_expint_E1) is evaluated from
 // Abramowitz & Stegun: the power series 5.1.11 for x <= 1 and the continued
 // fraction 5.1.22 by Lentz's method above.
@@ -113,18 +115,14 @@ __device__ __forceinline__ double tps_basis(double sx, double sy, double ex, dou
 
 __global__ void k_clear_flag(double* flag) { *flag = 0.0; }
 
-// neigh[i * sf + j * sj] is neighbour j of face i (sf = 1, sj = F: the context's j-major
-// copy; sf = 3, sj = 1: the ABI's face-major array).  CHECKED: the indices come straight
-// from the caller's device memory, unvalidated: one outside [-1, F) counts as no
-// neighbour and sets *bad = 1.
+// The neighbours of face i that exist, in slot order, and their count.  neigh[i * sf + j * sj]
+// is neighbour j of face i (sf = 1, sj = F: the context's j-major copy; sf = 3, sj = 1: the
+// ABI's face-major array).  CHECKED: the indices come straight from the caller's device
+// memory, unvalidated: one outside [-1, F) counts as no neighbour and sets *bad = 1.
 template <bool CHECKED>
-__global__ void __launch_bounds__(kBlock) k_smooth(int64_t F, const int32_t* __restrict__ neigh, int64_t sf, int64_t sj,
-                                                   const double* __restrict__ cx, const double* __restrict__ cy,
-                                                   const double* __restrict__ pt, double* __restrict__ out,
-                                                   double* __restrict__ bad) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= F) return;
-    double sx[3], sy[3], sz[3];
+__device__ __forceinline__ int tps_sites(int64_t F, int64_t i, const int32_t* neigh, int64_t sf, int64_t sj,
+                                         const double* cx, const double* cy, int32_t site[3], double sx[3],
+                                         double sy[3], double* bad) {
     int n = 0;
 #pragma unroll
     for (int j = 0; j < 3; ++j) {
@@ -134,21 +132,26 @@ __global__ void __launch_bounds__(kBlock) k_smooth(int64_t F, const int32_t* __r
             nb = -1;
         }
         if (nb < 0) continue;
+        site[n] = nb;
         sx[n] = cx[nb];
         sy[n] = cy[nb];
-        sz[n] = pt[nb];
         ++n;
     }
-    if (n == 0) {
-        out[i] = fmax(0.1, pt[i]);
-        return;
-    }
+    return n;
+}
+
+// The (n + 1) x (n + 1) spline system of n sites with NR right-hand sides (rhs[r][q]: the
+// value of site r in right-hand side q), by Gaussian elimination with partial pivoting;
+// x[q][...] = the constant, then the coefficient of each site.
+template <int NR>
+__device__ __forceinline__ void tps_solve(int n, const double sx[3], const double sy[3], const double rhs[3][NR],
+                                          double x[NR][4]) {
     const int m = n + 1;
-    double A[4][5];
+    double A[4][4 + NR];
 #pragma unroll
     for (int r = 0; r < 4; ++r)
 #pragma unroll
-        for (int cc = 0; cc < 5; ++cc) A[r][cc] = 0;
+        for (int cc = 0; cc < 4 + NR; ++cc) A[r][cc] = 0;
     for (int r = 0; r < n; ++r)
         for (int j = r; j < n; ++j) {
             const double xdiff = sx[r] - sx[j], ydiff = sy[r] - sy[j];
@@ -162,32 +165,105 @@ __global__ void __launch_bounds__(kBlock) k_smooth(int64_t F, const int32_t* __r
         A[m - 1][r] = 1;
     }
     A[m - 1][0] = 0;
-    for (int r = 0; r < n; ++r) A[r][m] = sz[r];
-    A[m - 1][m] = 0.0;
+    for (int q = 0; q < NR; ++q) {
+        for (int r = 0; r < n; ++r) A[r][m + q] = rhs[r][q];
+        A[m - 1][m + q] = 0.0;
+    }
     for (int k = 0; k < m; ++k) {
         int p = k;
         for (int r = k + 1; r < m; ++r)
             if (fabs(A[r][k]) > fabs(A[p][k])) p = r;
         if (p != k)
-            for (int cc = 0; cc <= m; ++cc) {
+            for (int cc = 0; cc < m + NR; ++cc) {
                 const double t = A[k][cc];
                 A[k][cc] = A[p][cc];
                 A[p][cc] = t;
             }
         for (int r = k + 1; r < m; ++r) {
             const double f = A[r][k] / A[k][k];
-            for (int cc = k; cc <= m; ++cc) A[r][cc] -= f * A[k][cc];
+            for (int cc = k; cc < m + NR; ++cc) A[r][cc] -= f * A[k][cc];
         }
     }
-    double x[4];
-    for (int k = m - 1; k >= 0; --k) {
-        double s = A[k][m];
-        for (int cc = k + 1; cc < m; ++cc) s -= A[k][cc] * x[cc];
-        x[k] = s / A[k][k];
+    for (int q = 0; q < NR; ++q)
+        for (int k = m - 1; k >= 0; --k) {
+            double s = A[k][m + q];
+            for (int cc = k + 1; cc < m; ++cc) s -= A[k][cc] * x[q][cc];
+            x[q][k] = s / A[k][k];
+        }
+}
+
+// Smoothing from the caller's own geometry arrays (pbsm3d_wind_run_noalloc, which keeps nothing
+// between calls): the spline system is set up and solved on every call.
+__global__ void __launch_bounds__(kBlock) k_smooth_checked(int64_t F, const int32_t* __restrict__ neigh,
+                                                           const double* __restrict__ cx,
+                                                           const double* __restrict__ cy,
+                                                           const double* __restrict__ pt, double* __restrict__ out,
+                                                           double* __restrict__ bad) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= F) return;
+    int32_t site[3];
+    double sx[3], sy[3], sz[3][1], x[1][4];
+    const int n = tps_sites<true>(F, i, neigh, 3, 1, cx, cy, site, sx, sy, bad);
+    if (n == 0) {
+        out[i] = fmax(0.1, pt[i]);
+        return;
     }
-    double z0 = x[0];
-    for (int r = 1; r < m; ++r) z0 = z0 + x[r] * tps_basis(sx[r - 1], sy[r - 1], cx[i], cy[i]);
+    for (int r = 0; r < n; ++r) sz[r][0] = pt[site[r]];
+    tps_solve<1>(n, sx, sy, sz, x);
+    double z0 = x[0][0];
+    for (int r = 1; r <= n; ++r) z0 = z0 + x[0][r] * tps_basis(sx[r - 1], sy[r - 1], cx[i], cy[i]);
     out[i] = fmax(0.1, z0);
+}
+
+// The spline's value at a face's own centroid is linear in its neighbours' winds, and both
+// the system and the basis depend on the mesh alone.  It reproduces constants, so the weights
+// add up to one and the value is p1 + w2 (p2 - p1) + w3 (p3 - p1) over the neighbours that
+// exist in slot order; this form keeps the weights' rounding off the common part of the
+// winds.  w[i] = w2 and w[F + i] = w3, 0 where there is no such neighbour.
+__global__ void __launch_bounds__(kBlock) k_weights(int64_t F, const int32_t* __restrict__ neigh,
+                                                    const double* __restrict__ cx, const double* __restrict__ cy,
+                                                    double* __restrict__ w) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= F) return;
+    int32_t site[3];
+    double sx[3], sy[3], unit[3][2] = {{0, 0}, {1, 0}, {0, 1}}, x[2][4];
+    const int n = tps_sites<false>(F, i, neigh, 1, F, cx, cy, site, sx, sy, nullptr);
+    double val[2] = {0, 0};
+    if (n > 1) {
+        tps_solve<2>(n, sx, sy, unit, x);
+        for (int r = 1; r <= n; ++r) {
+            const double b = tps_basis(sx[r - 1], sy[r - 1], cx[i], cy[i]);
+            for (int q = 0; q < n - 1; ++q) val[q] = (r == 1 ? x[q][0] : val[q]) + x[q][r] * b;
+        }
+    }
+    w[i] = val[0];
+    w[F + i] = val[1];
+}
+
+// Smoothing with the context's weights: three gathers and two products per face, bound by
+// the gathers (12 B of indices, 16 B of weights, 24 B gathered, 8 B out per face).  Solving the
+// spline per call took six E1 series per face: 999,968 faces, both kernels, 262 us, now 35 us.
+__global__ void __launch_bounds__(kBlock) k_smooth(int64_t F, const int32_t* __restrict__ neigh,
+                                                   const double* __restrict__ w, const double* __restrict__ pt,
+                                                   double* __restrict__ out) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= F) return;
+    int32_t nb[3];
+    double p[3];
+#pragma unroll
+    for (int j = 0; j < 3; ++j) nb[j] = neigh[i + j * F];
+    const double w2 = w[i], w3 = w[F + i];
+#pragma unroll
+    for (int j = 0; j < 3; ++j) p[j] = pt[nb[j] < 0 ? i : nb[j]];
+    // the first neighbour's wind, and the differences to the second and third
+    const bool h0 = nb[0] >= 0, h1 = nb[1] >= 0, h2 = nb[2] >= 0;
+    const double p1 = h0 ? p[0] : h1 ? p[1] : p[2];  // without neighbours: the face's own
+    const double d2 = h0 ? (h1 ? p[1] - p1 : h2 ? p[2] - p1 : 0.0) : (h1 && h2 ? p[2] - p1 : 0.0);
+    const double d3 = h0 && h1 && h2 ? p[2] - p1 : 0.0;
+    double z = p1 + (w2 * d2 + w3 * d3);
+    // an infinite neighbour makes NaN, and so the floor, as in the solve
+    if ((h0 || h1 || h2) && isinf(z)) z = NAN;
+    out[i] = fmax(0.1, z);
 }
 
 }  // namespace
@@ -201,7 +277,7 @@ struct pbsm3d_wind_ctx {
     int64_t F = 0;
     pbsm3d_wind_config cfg{};
     DevBuf<int32_t> neigh;  // j-major [j*F + i]
-    DevBuf<double> cx, cy, canopy, lai, stage_u, stage_sd, stage_out, point;
+    DevBuf<double> cx, cy, canopy, lai, stage_u, stage_sd, stage_out, point, weights;  // weights: [2F] of k_smooth
     bool veg = false;
     std::string err;
     ~pbsm3d_wind_ctx() {
@@ -300,6 +376,12 @@ int pbsm3d_wind_create(pbsm3d_wind_ctx** out, int device, int64_t F, const int32
         if (canopy) up(c->canopy, canopy);
         if (lai) up(c->lai, lai);
         for (DevBuf<double>* b : {&c->stage_u, &c->stage_sd, &c->stage_out, &c->point}) b->alloc(F);
+        if (cfg->smooth) {
+            c->weights.alloc(2 * F);
+            hipLaunchKernelGGL(k_weights, dim3(grid_for(F)), dim3(kBlock), 0, s, F, c->neigh.p, c->cx.p, c->cy.p,
+                               c->weights.p);
+            PB_HIP(hipGetLastError());
+        }
         PB_HIP(hipStreamSynchronize(s));
     });
     if (rc != PBSM3D_OK) {
@@ -332,8 +414,8 @@ int pbsm3d_wind_run(pbsm3d_wind_ctx* c, const double* U_R, const double* snowdep
                    c->cfg.smooth ? c->point.p : dout};
         hipLaunchKernelGGL(k_point_scale, dim3(grid_for(F)), dim3(kBlock), 0, s, a);
         if (c->cfg.smooth)
-            hipLaunchKernelGGL(k_smooth<false>, dim3(grid_for(F)), dim3(kBlock), 0, s, F, c->neigh.p, (int64_t)1, F,
-                               c->cx.p, c->cy.p, c->point.p, dout, (double*)nullptr);
+            hipLaunchKernelGGL(k_smooth, dim3(grid_for(F)), dim3(kBlock), 0, s, F, c->neigh.p, c->weights.p,
+                               c->point.p, dout);
         PB_HIP(hipGetLastError());
         if (!on_device) PB_HIP(hipMemcpyAsync(U2, dout, F * sizeof(double), hipMemcpyDeviceToHost, s));
         PB_HIP(hipStreamSynchronize(s));
@@ -365,8 +447,7 @@ int pbsm3d_wind_run_noalloc(int device, int64_t F, const int32_t* neigh, const d
         WindArgs a{F, cfg->ignore_canopy, cfg->z0_snow, canopy, lai, U_R, snowdepthavg, cfg->smooth ? scr : U2};
         hipLaunchKernelGGL(k_point_scale, dim3(grid_for(F)), dim3(kBlock), 0, s, a);
         if (cfg->smooth)
-            hipLaunchKernelGGL(k_smooth<true>, dim3(grid_for(F)), dim3(kBlock), 0, s, F, neigh, (int64_t)3, (int64_t)1,
-                               x, y, scr, U2, bad);
+            hipLaunchKernelGGL(k_smooth_checked, dim3(grid_for(F)), dim3(kBlock), 0, s, F, neigh, x, y, scr, U2, bad);
         PB_HIP(hipGetLastError());
         PB_HIP(hipStreamSynchronize(s));
         double flag = 0;

@@ -144,6 +144,31 @@ def test_gpu_wind_matches_oracle(pb, oracle, mesh_c1, veg, smooth):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("points", [3, 4, 300])
+def test_gpu_wind_weights_edges(pb, oracle, points):
+    """Faces with no, one, two and three neighbours, and winds that are not finite: a NaN or
+    infinite neighbour gives the 0.1 floor, as in the spline solve."""
+    print(f"[case] wind weights points={points}", flush=True)
+    mesh = meshgen.synthetic_mesh(points, seed=4, extent=3000.0)
+    F = mesh.n_faces
+    cx, cy = _centroids(mesh)
+    nb = mesh.neigh.copy()
+    nb[0] = -1  # an isolated face
+    U_R = meshgen.forcing_c2(F, seed=2)["U_R"]
+    cases = [U_R]
+    if F > 100:
+        bad = U_R.copy()
+        bad[50], bad[70], bad[90] = np.nan, np.inf, -np.inf
+        cases.append(bad)
+    w = pb.Wind(nb, cx, cy, None, None, _cfg())
+    for u in cases:
+        got = w.run(u, np.full(F, 0.4))
+        want = oracle.scale_wind(nb, cx, cy, None, None, _cfg(), u, np.full(F, 0.4))
+        np.testing.assert_allclose(got, want, rtol=1e-12, atol=0)
+    w.close()
+
+
+@pytest.mark.gpu
 def test_gpu_chain_wind_fetch_step(pb, oracle, mesh_c1):
     """U_R -> scale_wind_vert -> U_2m_above_srf and vw_dir -> fetchr -> fetch, both on
     device arrays, feeding the PBSM3D step: the same fields as the oracle chain."""
