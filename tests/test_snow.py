@@ -181,6 +181,28 @@ def test_gpu_snow_matches_oracle_bitwise(pb, oracle):
 
 
 @pytest.mark.gpu
+def test_gpu_snow_any_state_matches_oracle_bitwise(pb, oracle):
+    """States that the update itself never makes (a lower layer's mass, heat or water where no
+    layer is): every member it does not renew is kept, as in the oracle."""
+    print("[case] snow drift from arbitrary states", flush=True)
+    rng = np.random.default_rng(31)
+    n = 4099
+    cfg = _cfg()
+    sn = pb.Snow(n, rng.uniform(0, 120, n), cfg)
+    st = sn.get_state() + rng.uniform(0.0, 1.0, (len(F_), n))
+    st[F_["layer_count"]] = rng.integers(0, 3, n)
+    st[F_["z_s"], ::5] = 0.0
+    st[F_["m_s"], ::7] = 0.1
+    sn.set_state(st)
+    ref = st.copy()
+    for d in _drifts(rng, n, 3):
+        sn.drift(d)
+        ref = oracle.snow_drift(ref, cfg, d)
+        np.testing.assert_array_equal(sn.get_state(), ref)
+    sn.close()
+
+
+@pytest.mark.gpu
 def test_gpu_chain_step_snow_step(pb, oracle, mesh_small):
     """PBSM3D step -> drift_mass -> snowcover update -> swe / snowdepthavg of the next step,
     on device arrays, against the same chain through the oracles."""
