@@ -115,43 +115,47 @@ __device__ __forceinline__ double tps_basis(double sx, double sy, double ex, dou
 
 __global__ void k_clear_flag(double* flag) { *flag = 0.0; }
 
-// The neighbours of face i that exist, in slot order, and their count.  neigh[i * sf + j * sj]
-// is neighbour j of face i (sf = 1, sj = F: the context's j-major copy; sf = 3, sj = 1: the
-// ABI's face-major array).  CHECKED: the indices come straight from the caller's device
-// memory, unvalidated: one outside [-1, F) counts as no neighbour and sets *bad = 1.
+// The neighbours of face i (nb[j], -1 where there is none), the centroids of those that exist in
+// slot order, and their count.  neigh[i * sf + j * sj] is neighbour j of face i (sf = 1, sj = F:
+// the context's j-major copy; sf = 3, sj = 1: the ABI's face-major array).  CHECKED: the indices
+// come straight from the caller's device memory, unvalidated: one outside [-1, F) counts as no
+// neighbour and sets *bad = 1.
 template <bool CHECKED>
 __device__ __forceinline__ int tps_sites(int64_t F, int64_t i, const int32_t* neigh, int64_t sf, int64_t sj,
-                                         const double* cx, const double* cy, int32_t site[3], double sx[3],
+                                         const double* cx, const double* cy, int32_t nb[3], double sx[3],
                                          double sy[3], double* bad) {
     int n = 0;
 #pragma unroll
     for (int j = 0; j < 3; ++j) {
-        int32_t nb = neigh[i * sf + j * sj];
-        if (CHECKED && (nb < -1 || nb >= F)) {
+        nb[j] = neigh[i * sf + j * sj];
+        if (CHECKED && (nb[j] < -1 || nb[j] >= F)) {
             *bad = 1.0;
-            nb = -1;
+            nb[j] = -1;
         }
-        if (nb < 0) continue;
-        site[n] = nb;
-        sx[n] = cx[nb];
-        sy[n] = cy[nb];
+        if (nb[j] < 0) continue;
+        sx[n] = cx[nb[j]];
+        sy[n] = cy[nb[j]];
         ++n;
     }
     return n;
 }
 
-// The (n + 1) x (n + 1) spline system of n sites with NR right-hand sides (rhs[r][q]: the
-// value of site r in right-hand side q), by Gaussian elimination with partial pivoting;
-// x[q][...] = the constant, then the coefficient of each site.
-template <int NR>
-__device__ __forceinline__ void tps_solve(int n, const double sx[3], const double sy[3], const double rhs[3][NR],
-                                          double x[NR][4]) {
+// The spline's value at (x, y) is linear in the sites' winds, and both the system and the basis
+// depend on the mesh alone.  It reproduces constants, so the weights add up to one and the
+// value is p1 + w2 (p2 - p1) + w3 (p3 - p1) over the sites in order; this form keeps the
+// weights' rounding off the common part of the winds.  w[0] = w2 and w[1] = w3 (0 where there
+// is no such site): the values for a unit wind at that site, from the (n + 1) x (n + 1) system by
+// Gaussian elimination with partial pivoting.
+__device__ __forceinline__ void tps_weights(int n, const double sx[3], const double sy[3], double x, double y,
+                                            double w[2]) {
+    w[0] = w[1] = 0;
+    if (n < 2) return;
     const int m = n + 1;
-    double A[4][4 + NR];
+    double A[4][6];
 #pragma unroll
     for (int r = 0; r < 4; ++r)
 #pragma unroll
-        for (int cc = 0; cc < 4 + NR; ++cc) A[r][cc] = 0;
+        for (int cc = 0; cc < 6; ++cc) A[r][cc] = 0;
     for (int r = 0; r < n; ++r)
         for (int j = r; j < n; ++j) {
             const double xdiff = sx[r] - sx[j], ydiff = sy[r] - sy[j];
@@ -165,35 +169,51 @@ __device__ __forceinline__ void tps_solve(int n, const double sx[3], const doubl
         A[m - 1][r] = 1;
     }
     A[m - 1][0] = 0;
-    for (int q = 0; q < NR; ++q) {
-        for (int r = 0; r < n; ++r) A[r][m + q] = rhs[r][q];
-        A[m - 1][m + q] = 0.0;
-    }
+    for (int q = 0; q < 2; ++q)
+        for (int r = 0; r < m; ++r) A[r][m + q] = r == q + 1 && r < n ? 1.0 : 0.0;
     for (int k = 0; k < m; ++k) {
         int p = k;
         for (int r = k + 1; r < m; ++r)
             if (fabs(A[r][k]) > fabs(A[p][k])) p = r;
         if (p != k)
-            for (int cc = 0; cc < m + NR; ++cc) {
+            for (int cc = 0; cc < m + 2; ++cc) {
                 const double t = A[k][cc];
                 A[k][cc] = A[p][cc];
                 A[p][cc] = t;
             }
         for (int r = k + 1; r < m; ++r) {
             const double f = A[r][k] / A[k][k];
-            for (int cc = k; cc < m + NR; ++cc) A[r][cc] -= f * A[k][cc];
+            for (int cc = k; cc < m + 2; ++cc) A[r][cc] -= f * A[k][cc];
         }
     }
-    for (int q = 0; q < NR; ++q)
+    double c[2][4];
+    for (int q = 0; q < 2; ++q)
         for (int k = m - 1; k >= 0; --k) {
             double s = A[k][m + q];
-            for (int cc = k + 1; cc < m; ++cc) s -= A[k][cc] * x[q][cc];
-            x[q][k] = s / A[k][k];
+            for (int cc = k + 1; cc < m; ++cc) s -= A[k][cc] * c[q][cc];
+            c[q][k] = s / A[k][k];
         }
+    for (int r = 1; r < m; ++r) {
+        const double b = tps_basis(sx[r - 1], sy[r - 1], x, y);
+        for (int q = 0; q < n - 1; ++q) w[q] = (r == 1 ? c[q][0] : w[q]) + c[q][r] * b;
+    }
+}
+
+// The smoothed wind of a face whose neighbours have the winds p[j]; where there is none
+// (nb[j] < 0), p[j] is the face's own.
+__device__ __forceinline__ double smoothed(const int32_t nb[3], const double p[3], double w2, double w3) {
+    const bool h0 = nb[0] >= 0, h1 = nb[1] >= 0, h2 = nb[2] >= 0;
+    const double p1 = h0 ? p[0] : h1 ? p[1] : p[2];
+    const double d2 = h0 ? (h1 ? p[1] - p1 : h2 ? p[2] - p1 : 0.0) : (h1 && h2 ? p[2] - p1 : 0.0);
+    const double d3 = h0 && h1 && h2 ? p[2] - p1 : 0.0;
+    double z = p1 + (w2 * d2 + w3 * d3);
+    // an infinite neighbour makes NaN, and so the floor, as solving the system with it does
+    if ((h0 || h1 || h2) && isinf(z)) z = NAN;
+    return fmax(0.1, z);
 }
 
 // Smoothing from the caller's own geometry arrays (pbsm3d_wind_run_noalloc, which keeps nothing
-// between calls): the spline system is set up and solved on every call.
+// between calls): the weights are formed on every call.
 __global__ void __launch_bounds__(kBlock) k_smooth_checked(int64_t F, const int32_t* __restrict__ neigh,
                                                            const double* __restrict__ cx,
                                                            const double* __restrict__ cy,
@@ -201,48 +221,32 @@ __global__ void __launch_bounds__(kBlock) k_smooth_checked(int64_t F, const int3
                                                            double* __restrict__ bad) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= F) return;
-    int32_t site[3];
-    double sx[3], sy[3], sz[3][1], x[1][4];
-    const int n = tps_sites<true>(F, i, neigh, 3, 1, cx, cy, site, sx, sy, bad);
-    if (n == 0) {
-        out[i] = fmax(0.1, pt[i]);
-        return;
-    }
-    for (int r = 0; r < n; ++r) sz[r][0] = pt[site[r]];
-    tps_solve<1>(n, sx, sy, sz, x);
-    double z0 = x[0][0];
-    for (int r = 1; r <= n; ++r) z0 = z0 + x[0][r] * tps_basis(sx[r - 1], sy[r - 1], cx[i], cy[i]);
-    out[i] = fmax(0.1, z0);
+    int32_t nb[3];
+    double sx[3], sy[3], p[3], w[2];
+    const int n = tps_sites<true>(F, i, neigh, 3, 1, cx, cy, nb, sx, sy, bad);
+#pragma unroll
+    for (int j = 0; j < 3; ++j) p[j] = pt[nb[j] < 0 ? i : nb[j]];
+    tps_weights(n, sx, sy, cx[i], cy[i], w);
+    out[i] = smoothed(nb, p, w[0], w[1]);
 }
 
-// The spline's value at a face's own centroid is linear in its neighbours' winds, and both
-// the system and the basis depend on the mesh alone.  It reproduces constants, so the weights
-// add up to one and the value is p1 + w2 (p2 - p1) + w3 (p3 - p1) over the neighbours that
-// exist in slot order; this form keeps the weights' rounding off the common part of the
-// winds.  w[i] = w2 and w[F + i] = w3, 0 where there is no such neighbour.
+// The weights of every face: w[i] = w2, w[F + i] = w3.
 __global__ void __launch_bounds__(kBlock) k_weights(int64_t F, const int32_t* __restrict__ neigh,
                                                     const double* __restrict__ cx, const double* __restrict__ cy,
                                                     double* __restrict__ w) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= F) return;
-    int32_t site[3];
-    double sx[3], sy[3], unit[3][2] = {{0, 0}, {1, 0}, {0, 1}}, x[2][4];
-    const int n = tps_sites<false>(F, i, neigh, 1, F, cx, cy, site, sx, sy, nullptr);
-    double val[2] = {0, 0};
-    if (n > 1) {
-        tps_solve<2>(n, sx, sy, unit, x);
-        for (int r = 1; r <= n; ++r) {
-            const double b = tps_basis(sx[r - 1], sy[r - 1], cx[i], cy[i]);
-            for (int q = 0; q < n - 1; ++q) val[q] = (r == 1 ? x[q][0] : val[q]) + x[q][r] * b;
-        }
-    }
-    w[i] = val[0];
-    w[F + i] = val[1];
+    int32_t nb[3];
+    double sx[3], sy[3], v[2];
+    const int n = tps_sites<false>(F, i, neigh, 1, F, cx, cy, nb, sx, sy, nullptr);
+    tps_weights(n, sx, sy, cx[i], cy[i], v);
+    w[i] = v[0];
+    w[F + i] = v[1];
 }
 
 // Smoothing with the context's weights: three gathers and two products per face, bound by
 // the gathers (12 B of indices, 16 B of weights, 24 B gathered, 8 B out per face).  Solving the
-// spline per call took six E1 series per face: 999,968 faces, both kernels, 262 us, now 35 us.
+// spline per call took six E1 series per face: 999,968 faces, both kernels, 262 us, now 33 us.
 __global__ void __launch_bounds__(kBlock) k_smooth(int64_t F, const int32_t* __restrict__ neigh,
                                                    const double* __restrict__ w, const double* __restrict__ pt,
                                                    double* __restrict__ out) {
@@ -255,15 +259,7 @@ __global__ void __launch_bounds__(kBlock) k_smooth(int64_t F, const int32_t* __r
     const double w2 = w[i], w3 = w[F + i];
 #pragma unroll
     for (int j = 0; j < 3; ++j) p[j] = pt[nb[j] < 0 ? i : nb[j]];
-    // the first neighbour's wind, and the differences to the second and third
-    const bool h0 = nb[0] >= 0, h1 = nb[1] >= 0, h2 = nb[2] >= 0;
-    const double p1 = h0 ? p[0] : h1 ? p[1] : p[2];  // without neighbours: the face's own
-    const double d2 = h0 ? (h1 ? p[1] - p1 : h2 ? p[2] - p1 : 0.0) : (h1 && h2 ? p[2] - p1 : 0.0);
-    const double d3 = h0 && h1 && h2 ? p[2] - p1 : 0.0;
-    double z = p1 + (w2 * d2 + w3 * d3);
-    // an infinite neighbour makes NaN, and so the floor, as in the solve
-    if ((h0 || h1 || h2) && isinf(z)) z = NAN;
-    out[i] = fmax(0.1, z);
+    out[i] = smoothed(nb, p, w2, w3);
 }
 
 }  // namespace
