@@ -165,20 +165,56 @@ template <typename T>
 void spmv_col(hipStream_t s, int64_t F, int L, const int32_t* rp, const T* val, const int32_t* neigh,
               const uint16_t* slots, const T* x, const T* b, T* y, double* partial);
 inline int64_t spmv_col_blocks(int64_t F) { return (F + kBlock - 1) / kBlock; }
-// partial[block*(nv+1) + c] = sum over the block's rows of V_c . w (c < nv), w . w (c == nv)
+// partial[block*(nv+1) + c] = sum over the block's rows of V_c . w (c < nv), w . w (c == nv); the
+// basis vectors lie ld apart.  gate (may be NULL): the launch does nothing while *gate == 0.
 template <typename T>
-void mdot(hipStream_t s, int64_t n, const T* V, int nv, const T* w, double* partial, int nblk);
+void mdot(hipStream_t s, int64_t n, const T* V, int64_t ld, int nv, const T* w, double* partial, int nblk,
+          const double* gate = nullptr);
 // out[c] = sum_b partial[b*stride + c] for c < ncols (fixed order, deterministic)
 void reduce_cols(hipStream_t s, const double* partial, int nblk, int stride, int ncols, double* out);
-// w -= sum_c h[c] V_c ; partial[block] = sum w.w (after the update)
+// w = (*scale) w - sum_c coef[c] V_c (scale NULL: 1); partial[block] = sum w.w (after the update)
 template <typename T>
-void gs_update(hipStream_t s, int64_t n, const T* V, int nv, const double* h, T* w, double* partial, int nblk);
-// v = w * (1 / *nrm)   (nrm on device)
+void gs_update(hipStream_t s, int64_t n, const T* V, int64_t ld, int nv, const double* coef, const double* scale, T* w,
+               double* partial, int nblk, const double* gate = nullptr);
+// u = sum_c coef[c] V_c  (coef on device)
 template <typename T>
-void scale_by_inv(hipStream_t s, int64_t n, const T* w, const double* nrm, T* v);
-// u = sum_c y[c] V_c  (y on device)
-template <typename T>
-void combine(hipStream_t s, int64_t n, const T* V, int nv, const double* y, T* u);
+void combine(hipStream_t s, int64_t n, const T* V, int64_t ld, int nv, const double* coef, T* u);
+// a vector of up to this many bytes stays in the caches between two reads (4 MB of L2 per XCD,
+// 256 MB behind them): k_mdot's split of the columns
+constexpr int64_t kCachedVector = 16 << 20;
+
+// Device scalars of a GMRES(m) cycle, m <= 31, in one allocation of kDoubles.
+struct GmresSc {
+    static constexpr int kDoubles = 32 * 32 + 7 * 32;
+    double *H;       // [32 x 32] column j of the triangular factor at H + 32 j
+    double *hcol, *coef, *scal, *cs, *sn, *g;  // [32] each; scal[c]: v_c = scal[c] w_c
+    double *before, *gate;
+    static GmresSc of(double* p) {
+        GmresSc a;
+        a.H = p;
+        p += 32 * 32;
+        for (double** q : {&a.hcol, &a.coef, &a.scal, &a.cs, &a.sn, &a.g}) {
+            *q = p;
+            p += 32;
+        }
+        a.before = p;
+        a.gate = p + 1;
+        return a;
+    }
+};
+// What a kernel reports to the host that waits for it: values, then the number of the report.
+// Pinned coherent memory; the host polls seq (wait_slot), which costs the stream nothing, where
+// an event record delays the kernels on either side of it by about 6 us.
+struct HostSlot {
+    double v[31];
+    uint64_t seq;
+};
+void wait_slot(hipStream_t s, const HostSlot* slot, uint64_t seq);
+void gmres_start(hipStream_t s, const GmresSc& a, double beta);
+void gmres_h(hipStream_t s, const GmresSc& a, const double* partial, int nblk, int j, int pass);
+void gmres_gate(hipStream_t s, const GmresSc& a, const double* ss, int nblk);
+void gmres_step(hipStream_t s, const GmresSc& a, const double* ss, int nblk, int j, HostSlot* slot, uint64_t seq);
+void gmres_y(hipStream_t s, const GmresSc& a, int k);
 // max |b| per block into partial
 void absmax(hipStream_t s, int64_t n, const double* b, double* partial, int nblk);
 void reduce_max(hipStream_t s, const double* partial, int nblk, double* out);

@@ -1,11 +1,16 @@
 // GMRES(m) with classical Gram-Schmidt and a conditional second pass (the
 // DGKS test ||w_after|| < ||w_before|| / sqrt(2)), as iterated classical
-// Gram-Schmidt does.  The basis lives in HBM; each Arnoldi step is
-//   z = M^-1 v_j ; v_{j+1} = A z ; h = V^T v_{j+1} (one batched pass) ;
-//   v_{j+1} -= V h (one pass, fused norm) ; v_{j+1} /= ||v_{j+1}||
-// and only the (j+2) Hessenberg entries travel to the host, where the Givens
-// rotations and the least-squares solve run in FP64.
+// Gram-Schmidt does.  The basis lives in HBM, its vectors unscaled with their
+// factors beside them; each Arnoldi step is
+//   z = M^-1 w_j ; u = A z ; h = V^T u (one batched pass) ;
+//   w_{j+1} = s_j u - V h (one pass, fused norm)
+// The Hessenberg column, its Givens rotations and the least-squares solve stay
+// on the device; the host reads only the residual estimate of the step before
+// the one it queues, so the stream does not wait for it (a 5,000 x 5 system
+// spent 78 us per step with a synchronisation in each, of which the kernels
+// took 55).
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <vector>
 
@@ -13,11 +18,6 @@
 
 namespace pb {
 namespace {
-
-// device scalar slots
-inline int off_h() { return 0; }
-inline int off_ss(int m) { return m + 2; }
-inline int off_y(int m) { return m + 4; }
 
 constexpr int kVecBlocks = 512;  // two workgroups per CU
 
@@ -27,14 +27,33 @@ inline int reduce_blocks(int64_t n) {
     return (int)(b < 1 ? 1 : b);
 }
 
+// workgroups of a kernel that takes four rows per thread
+inline int reduce_blocks4(int64_t n) { return reduce_blocks((n + 3) / 4); }
+
 }  // namespace
+
+void wait_slot(hipStream_t s, const HostSlot* slot, uint64_t seq) {
+    const volatile uint64_t* at = &slot->seq;
+    for (uint32_t spin = 1; *at != seq; ++spin) {
+        if (spin % 4096 == 0) {  // a stream that failed, or ended without the report, never writes it
+            const hipError_t e = hipStreamQuery(s);
+            if (e != hipErrorNotReady && *at != seq) {
+                PB_HIP(e);
+                throw Error(PBSM3D_EHIP, "a kernel ended without its report");
+            }
+        }
+        __builtin_ia32_pause();
+    }
+    std::atomic_thread_fence(std::memory_order_acquire);
+}
 
 template <typename T>
 void GmresWork<T>::ensure(int64_t n_, int m_) {
     if (n == n_ && m == m_ && V.p) return;
     n = n_;
     m = m_;
-    V.alloc((size_t)(m + 1) * n);
+    ld = (n + 63) / 64 * 64;
+    V.alloc((size_t)(m + 1) * ld);
     z.alloc(n);
     u.alloc(n);
     // residual partials: one per block of kBlock rows, or ceil(F / kBlock) * L <= n / kBlock + L
@@ -43,30 +62,35 @@ void GmresWork<T>::ensure(int64_t n_, int m_) {
     size_t pbytes = (size_t)kReduceBlocks * (m + 2);
     if (pbytes < spmv_blocks) pbytes = spmv_blocks;
     partial.alloc(pbytes);
-    dsc.alloc(2 * m + 8);
-    hsc.alloc(2 * m + 8);
+    ss.alloc(kReduceBlocks);
+    dsc.alloc(GmresSc::kDoubles + 1);
+    hsc.alloc(1);
+    slot.alloc(2);
+    slot.p[0].seq = slot.p[1].seq = seq = 0;
 }
+
+// How far the last known residual must lie above the target for the host to queue another Arnoldi
+// step before the estimate of the one in flight: a step rarely gains more, and one queued past
+// the end is work for nothing.
+constexpr double kAhead = 30.0;
 
 template <typename T>
 int gmres_cycle(hipStream_t s, GmresWork<T>& w, const CsrOp<T>& A, const PcFn<T>& M, const T* r0, double beta,
                 double stop_abs, int max_steps, T* out, double* resid_est) {
-    const int64_t n = A.n;
-    const int m = w.m;
-    const int nblk = reduce_blocks(n);
+    const int64_t n = A.n, ld = w.ld;
+    const int nblk = reduce_blocks4(n);
     T* V = w.V.p;
-    double* d_h = w.dsc.p + off_h();
-    double* d_ss = w.dsc.p + off_ss(m);
-    double* d_y = w.dsc.p + off_y(m);
-    double* hs = w.hsc.p;
-    if (max_steps > m) max_steps = m;
+    const GmresSc sc = GmresSc::of(w.dsc.p);
+    HostSlot* dslot = nullptr;
+    PB_HIP(hipHostGetDevicePointer((void**)&dslot, w.slot.p, 0));
+    if (max_steps > w.m) max_steps = w.m;
 
-    std::vector<double> H((size_t)(m + 1) * m, 0.0), cs(m, 0.0), sn(m, 0.0), g(m + 1, 0.0), h(m + 2, 0.0), y(m, 0.0);
     scale_host<T>(s, n, r0, 1.0 / beta, V);
-    g[0] = beta;
-    int k = 0;
-    for (int j = 0; j < max_steps; ++j) {
-        T* vj = V + (size_t)j * n;
-        T* vj1 = V + (size_t)(j + 1) * n;
+    gmres_start(s, sc, beta);
+    const uint64_t seq0 = w.seq;
+    auto queue = [&](int j) {
+        T* vj = V + (size_t)j * ld;
+        T* vj1 = V + (size_t)(j + 1) * ld;
         {
             ProfScope ps(A.prof, s, PBSM3D_K_PRECOND);
             M(s, vj, w.z.p);
@@ -75,66 +99,47 @@ int gmres_cycle(hipStream_t s, GmresWork<T>& w, const CsrOp<T>& A, const PcFn<T>
             ProfScope ps(A.prof, s, sizeof(T) == 8 ? PBSM3D_K_SPMV64 : PBSM3D_K_SPMV32);
             op_spmv<T>(s, A, w.z.p, vj1);
         }
-        for (int i = 0; i <= j; ++i) h[i] = 0.0;
-        double ss_before = 0, ss_after = 0;
-        for (int pass = 0; pass < 2; ++pass) {
-            {
-                ProfScope ps(A.prof, s, PBSM3D_K_ORTHO);
-                mdot<T>(s, n, V, j + 1, vj1, w.partial.p, nblk);
-                reduce_cols(s, w.partial.p, nblk, j + 2, j + 2, d_h);
-                gs_update<T>(s, n, V, j + 1, d_h, vj1, w.partial.p, nblk);
-                reduce_cols(s, w.partial.p, nblk, 1, 1, d_ss);
-            }
-            PB_HIP(hipMemcpyAsync(hs, w.dsc.p, sizeof(double) * (m + 3), hipMemcpyDeviceToHost, s));
-            PB_HIP(hipStreamSynchronize(s));
-            for (int i = 0; i <= j; ++i) h[i] += hs[off_h() + i];
-            if (pass == 0) ss_before = hs[off_h() + j + 1];
-            ss_after = hs[off_ss(m)];
-            if (w.passes < 2 || !(ss_after < 0.5 * ss_before)) break;  // no re-orthogonalisation needed
+        ProfScope ps(A.prof, s, PBSM3D_K_ORTHO);
+        mdot<T>(s, n, V, ld, j + 1, vj1, w.partial.p, nblk);
+        gmres_h(s, sc, w.partial.p, nblk, j, 0);
+        gs_update<T>(s, n, V, ld, j + 1, sc.coef, sc.scal + j, vj1, w.ss.p, nblk);
+        if (w.passes > 1) {
+            gmres_gate(s, sc, w.ss.p, nblk);
+            mdot<T>(s, n, V, ld, j + 1, vj1, w.partial.p, nblk, sc.gate);
+            gmres_h(s, sc, w.partial.p, nblk, j, 1);
+            gs_update<T>(s, n, V, ld, j + 1, sc.coef, nullptr, vj1, w.ss.p, nblk, sc.gate);
         }
-        const double hn = std::sqrt(ss_after);
-        if (hn > 0) scale_by_inv<T>(s, n, vj1, d_ss, vj1);
-        for (int i = 0; i <= j; ++i) H[(size_t)i * m + j] = h[i];
-        H[(size_t)(j + 1) * m + j] = hn;
-        for (int i = 0; i < j; ++i) {
-            const double a = H[(size_t)i * m + j], b = H[(size_t)(i + 1) * m + j];
-            H[(size_t)i * m + j] = cs[i] * a + sn[i] * b;
-            H[(size_t)(i + 1) * m + j] = -sn[i] * a + cs[i] * b;
+        gmres_step(s, sc, w.ss.p, nblk, j, dslot + (j & 1), ++w.seq);
+        PB_HIP(hipGetLastError());
+    };
+    double res = beta;
+    int queued = 0, known = 0;
+    while (known < max_steps) {
+        if (queued < max_steps && (queued == known || (queued == known + 1 && res > kAhead * stop_abs))) {
+            queue(queued++);
+            continue;
         }
-        const double a = H[(size_t)j * m + j], b = H[(size_t)(j + 1) * m + j];
-        const double rr = std::hypot(a, b);
-        cs[j] = rr > 0 ? a / rr : 1.0;
-        sn[j] = rr > 0 ? b / rr : 0.0;
-        H[(size_t)j * m + j] = rr;
-        H[(size_t)(j + 1) * m + j] = 0.0;
-        g[j + 1] = -sn[j] * g[j];
-        g[j] = cs[j] * g[j];
-        k = j + 1;
-        if (std::fabs(g[j + 1]) <= stop_abs || hn == 0.0) break;
+        const HostSlot& sl = w.slot.p[known & 1];
+        wait_slot(s, &sl, seq0 + known + 1);
+        ++known;
+        res = sl.v[0];
+        if (res <= stop_abs || sl.v[1] == 0.0) break;
     }
-    for (int i = k - 1; i >= 0; --i) {
-        double sacc = g[i];
-        for (int q = i + 1; q < k; ++q) sacc -= H[(size_t)i * m + q] * y[q];
-        y[i] = sacc / H[(size_t)i * m + i];
-    }
-    for (int i = 0; i < k; ++i) hs[off_y(m) + i] = y[i];
-    PB_HIP(hipMemcpyAsync(d_y, hs + off_y(m), sizeof(double) * k, hipMemcpyHostToDevice, s));
-    combine<T>(s, n, V, k, d_y, w.u.p);
+    gmres_y(s, sc, known);
+    combine<T>(s, n, V, ld, known, sc.coef, w.u.p);
     {
         ProfScope ps(A.prof, s, PBSM3D_K_PRECOND);
         M(s, w.u.p, out);
     }
-    // the pinned staging buffer is reused by the next cycle: wait for the copy
-    PB_HIP(hipStreamSynchronize(s));
-    *resid_est = std::fabs(g[k]);
-    return k;
+    *resid_est = res;
+    return known;
 }
 
 double dev_norm2(hipStream_t s, GmresWork<double>& w, int64_t n, const double* v) {
     const int nblk = reduce_blocks(n);
-    mdot<double>(s, n, nullptr, 0, v, w.partial.p, nblk);
-    reduce_cols(s, w.partial.p, nblk, 1, 1, w.dsc.p + off_ss(w.m) + 1);
-    PB_HIP(hipMemcpyAsync(w.hsc.p, w.dsc.p + off_ss(w.m) + 1, sizeof(double), hipMemcpyDeviceToHost, s));
+    mdot<double>(s, n, nullptr, 0, 0, v, w.partial.p, nblk);
+    reduce_cols(s, w.partial.p, nblk, 1, 1, w.dsc.p + GmresSc::kDoubles);
+    PB_HIP(hipMemcpyAsync(w.hsc.p, w.dsc.p + GmresSc::kDoubles, sizeof(double), hipMemcpyDeviceToHost, s));
     PB_HIP(hipStreamSynchronize(s));
     return std::sqrt(w.hsc.p[0]);
 }
@@ -160,8 +165,8 @@ double residual_norm(hipStream_t s, GmresWork<T>& w, const CsrOp<double>& A, con
         ProfScope ps(A.prof, s, PBSM3D_K_RESIDUAL);
         nblk = op_residual(s, A, x, b, r, w.partial.p);
     }
-    reduce_cols(s, w.partial.p, nblk, 1, 1, w.dsc.p + off_ss(w.m) + 1);
-    PB_HIP(hipMemcpyAsync(w.hsc.p, w.dsc.p + off_ss(w.m) + 1, sizeof(double), hipMemcpyDeviceToHost, s));
+    reduce_cols(s, w.partial.p, nblk, 1, 1, w.dsc.p + GmresSc::kDoubles);
+    PB_HIP(hipMemcpyAsync(w.hsc.p, w.dsc.p + GmresSc::kDoubles, sizeof(double), hipMemcpyDeviceToHost, s));
     PB_HIP(hipStreamSynchronize(s));
     return std::sqrt(w.hsc.p[0]);
 }
@@ -169,9 +174,9 @@ double residual_norm(hipStream_t s, GmresWork<T>& w, const CsrOp<double>& A, con
 template <typename T>
 double norm_of(hipStream_t s, GmresWork<T>& w, int64_t n, const double* v) {
     const int nblk = reduce_blocks(n);
-    mdot<double>(s, n, nullptr, 0, v, w.partial.p, nblk);
-    reduce_cols(s, w.partial.p, nblk, 1, 1, w.dsc.p + off_ss(w.m) + 1);
-    PB_HIP(hipMemcpyAsync(w.hsc.p, w.dsc.p + off_ss(w.m) + 1, sizeof(double), hipMemcpyDeviceToHost, s));
+    mdot<double>(s, n, nullptr, 0, 0, v, w.partial.p, nblk);
+    reduce_cols(s, w.partial.p, nblk, 1, 1, w.dsc.p + GmresSc::kDoubles);
+    PB_HIP(hipMemcpyAsync(w.hsc.p, w.dsc.p + GmresSc::kDoubles, sizeof(double), hipMemcpyDeviceToHost, s));
     PB_HIP(hipStreamSynchronize(s));
     return std::sqrt(w.hsc.p[0]);
 }
@@ -269,7 +274,7 @@ int64_t spmv_dots(hipStream_t s, const CsrOp<T>& A, const T* x, T* y, const T* w
     if (A.split) return split_apply_dots<T>(s, *A.co, A.F, A.L, *A.split, x, y, w, partial, A.mode, stop);
     if (A.pos) return pos_spmv_dots<T>(s, A.variant, *A.co, A.F, A.L, *A.pos, x, y, w, partial);
     op_spmv<T>(s, A, x, y);
-    mdot<T>(s, A.n, w, 1, y, partial, nblk);
+    mdot<T>(s, A.n, w, 0, 1, y, partial, nblk);
     return nblk;
 }
 
@@ -312,7 +317,7 @@ int bicg_run(hipStream_t s, BicgWork<T>& w, const CsrOp<T>& A, const PcFn<T>& M,
         axpy_dots<T>(s, n, 1.0, w.v.p, b, w.r.p, nullptr, w.partial.p, nblk);
     }
     PB_HIP(hipMemcpyAsync(w.rh.p, w.r.p, n * sizeof(T), hipMemcpyDeviceToDevice, s));
-    mdot<T>(s, n, w.rh.p, 1, w.r.p, w.partial.p, nblk);
+    mdot<T>(s, n, w.rh.p, 0, 1, w.r.p, w.partial.p, nblk);
     bicg_stage(s, w.partial.p, nblk, 2, 0, sc);
     fetch();
     double rr = std::sqrt(h[SC_RR]);

@@ -85,12 +85,16 @@ struct SolveInfo {
 template <typename T>
 struct GmresWork {
     int64_t n = 0;
+    int64_t ld = 0;  // distance of the basis vectors: n rounded up, so that each starts aligned
     int m = 0;
     int passes = 2;  // Gram-Schmidt passes allowed per Arnoldi step
     DevBuf<T> V, z, u;
     DevBuf<double> partial;  // kReduceBlocks * (m + 2)
-    DevBuf<double> dsc;      // device scalars
-    HostBuf<double> hsc;     // pinned mirror
+    DevBuf<double> ss;       // kReduceBlocks partial sums of the new vector's norm
+    DevBuf<double> dsc;      // GmresSc, then the norm that norm_of / residual_norm report
+    HostBuf<double> hsc;     // pinned mirror of that norm
+    HostBuf<HostSlot> slot;  // reports of two Arnoldi steps in flight
+    uint64_t seq = 0;        // number of the last report
     void ensure(int64_t n_, int m_);
 };
 

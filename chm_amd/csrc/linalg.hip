@@ -139,11 +139,6 @@ __global__ void __launch_bounds__(kBlock) k_spmv_plain(int64_t n, const int32_t*
     y[r] = acc;
 }
 
-// Batched dot products of w against nv <= kNV basis vectors plus w.w: w is
-// read once, each basis vector once; FP64 accumulation.  Each wavefront
-// shuffle-reduces all nv+1 sums, then the block combines its wavefronts in LDS.
-constexpr int kNV = 32;
-
 // four consecutive elements per thread: one 16-byte (float) or two 16-byte
 // (double) loads per lane, so each wavefront load moves 1-2 KB
 __device__ __forceinline__ void load4(const double* p, double (&o)[4]) {
@@ -167,56 +162,73 @@ __device__ __forceinline__ void store4(float* p, const double (&o)[4]) {
     *reinterpret_cast<float4*>(p) = float4{(float)o[0], (float)o[1], (float)o[2], (float)o[3]};
 }
 
-// VEC: n % 4 == 0, every vector 4-element aligned
-template <typename T, bool VEC>
-__global__ void __launch_bounds__(kBlock) k_mdot(int64_t n, const T* __restrict__ V, int nv, const T* __restrict__ w,
-                                                 double* __restrict__ partial) {
-    __shared__ double s_acc[kBlock / 64][kNV + 1];
-    double acc[kNV + 1];
-#pragma unroll
-    for (int c = 0; c <= kNV; ++c) acc[c] = 0.0;
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    if constexpr (VEC) {
-        const int64_t n4 = n / 4;
-        for (int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; g < n4; g += stride) {
-            double wv[4];
-            load4(w + 4 * g, wv);
-#pragma unroll
-            for (int q = 0; q < 4; ++q) acc[kNV] = fma(wv[q], wv[q], acc[kNV]);
-#pragma unroll
-            for (int c = 0; c < kNV; ++c)
-                if (c < nv) {
-                    double vv[4];
-                    load4(V + (int64_t)c * n + 4 * g, vv);
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) acc[c] = fma(vv[q], wv[q], acc[c]);
-                }
-        }
+// Basis vectors whose loads are in flight together: a column at a time, each behind its own
+// branch, left a small system waiting out one load latency per basis vector.
+constexpr int kCols = 8;
+
+// Elements 4 g .. 4 g + 3 of p, those past n as zero (g is the thread's group of four).
+template <typename T>
+__device__ __forceinline__ void load4_tail(const T* p, int64_t g, int64_t n, double (&o)[4]) {
+    if (4 * g + 4 <= n) {
+        load4(p + 4 * g, o);
     } else {
-        for (int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; k < n; k += stride) {
-            const double wk = (double)w[k];
-            acc[kNV] = fma(wk, wk, acc[kNV]);
 #pragma unroll
-            for (int c = 0; c < kNV; ++c)
-                if (c < nv) acc[c] = fma((double)V[(int64_t)c * n + k], wk, acc[c]);
+        for (int q = 0; q < 4; ++q) o[q] = 4 * g + q < n ? (double)p[4 * g + q] : 0.0;
+    }
+}
+
+// Batched dot products of w against nv basis vectors (ld apart) plus w.w, FP64 accumulation:
+// partial[block * (nv + 1) + c].  NCH chunks of kCols columns per workgroup, the rest of the
+// columns along gridDim.y: 1 while w stays in the caches, so that a small system still fills
+// the chip, else all of them, so that w is read once.  Each wavefront shuffle-reduces its sums,
+// then the workgroup adds its wavefronts in LDS.  gate (may be NULL): returns at entry when 0.
+template <typename T, int NCH>
+__global__ void __launch_bounds__(kBlock) k_mdot(int64_t n, int64_t ld, const T* __restrict__ V, int nv,
+                                                 const T* __restrict__ w, double* __restrict__ partial,
+                                                 const double* __restrict__ gate) {
+    if (gate && *gate == 0.0) return;
+    __shared__ double s_acc[kBlock / 64][NCH * kCols + 1];
+    double acc[NCH * kCols], ww = 0.0;
+#pragma unroll
+    for (int c = 0; c < NCH * kCols; ++c) acc[c] = 0.0;
+    const int first = (int)blockIdx.y * NCH * kCols;
+    const int64_t stride = (int64_t)gridDim.x * blockDim.x, n4 = (n + 3) / 4;
+    for (int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; g < n4; g += stride) {
+        double wv[4];
+        load4_tail(w, g, n, wv);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) ww = fma(wv[q], wv[q], ww);
+#pragma unroll
+        for (int h = 0; h < NCH; ++h) {
+            const int c0 = first + h * kCols;
+            if (c0 < nv) {
+                double vv[kCols][4];
+#pragma unroll
+                for (int c = 0; c < kCols; ++c) load4_tail(V + (int64_t)min(c0 + c, nv - 1) * ld, g, n, vv[c]);
+#pragma unroll
+                for (int c = 0; c < kCols; ++c)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) acc[h * kCols + c] = fma(vv[c][q], wv[q], acc[h * kCols + c]);
+            }
         }
     }
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
 #pragma unroll
-    for (int c = 0; c <= kNV; ++c) {
-        if (c < nv || c == kNV) {
+    for (int c = 0; c < NCH * kCols; ++c)
+        if (first + c < nv) {
             const double v = wave_sum(acc[c]);
             if (lane == 0) s_acc[wid][c] = v;
         }
+    if (first == 0) {
+        ww = wave_sum(ww);
+        if (lane == 0) s_acc[wid][NCH * kCols] = ww;
     }
     __syncthreads();
     const int t = threadIdx.x;
-    if (t <= nv) {
-        const int src = t == nv ? kNV : t;
-        double s = 0;
-        for (int q = 0; q < (int)(blockDim.x >> 6); ++q) s += s_acc[q][src];
-        partial[(int64_t)blockIdx.x * (nv + 1) + t] = s;
-    }
+    if (t > NCH * kCols || (t < NCH * kCols ? first + t >= nv : first != 0)) return;
+    double sum = 0;
+    for (int q = 0; q < kBlock / 64; ++q) sum += s_acc[q][t];
+    partial[(int64_t)blockIdx.x * (nv + 1) + (t < NCH * kCols ? first + t : nv)] = sum;
 }
 
 __global__ void __launch_bounds__(kBlock) k_reduce_cols(const double* __restrict__ partial, int nblk, int stride,
@@ -229,68 +241,155 @@ __global__ void __launch_bounds__(kBlock) k_reduce_cols(const double* __restrict
     if (threadIdx.x == 0) out[c] = s;
 }
 
-template <typename T, bool VEC>
-__global__ void __launch_bounds__(kBlock) k_gs_update(int64_t n, const T* __restrict__ V, int nv,
-                                                      const double* __restrict__ h, T* __restrict__ w,
-                                                      double* __restrict__ partial) {
+// Scalars of one GMRES cycle on the device (GmresSc::of lays them out).
+// Column j's projections from mdot's partials of u = A M^-1 w_j (pass 0) or of the updated vector
+// (pass 1).  Basis vectors are stored unscaled, v_c = scal[c] w_c: coef[c] is what gs_update
+// multiplies w_c with, hcol[c] the Hessenberg entry, summed over the passes.
+__global__ void __launch_bounds__(kBlock) k_gmres_h(GmresSc a, const double* __restrict__ partial, int nblk, int j,
+                                                    int pass) {
     __shared__ double s_red[kBlock / 64];
-    double hc[kNV];
-#pragma unroll
-    for (int c = 0; c < kNV; ++c) hc[c] = c < nv ? h[c] : 0.0;
-    double acc = 0.0;
-    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-    if constexpr (VEC) {
-        const int64_t n4 = n / 4;
-        for (int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; g < n4; g += stride) {
-            double wv[4];
-            load4(w + 4 * g, wv);
-#pragma unroll
-            for (int c = 0; c < kNV; ++c)
-                if (c < nv) {
-                    double vv[4];
-                    load4(V + (int64_t)c * n + 4 * g, vv);
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) wv[q] = fma(-hc[c], vv[q], wv[q]);
-                }
-            double wr[4];
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                wr[q] = (double)(T)wv[q];  // the value actually stored
-                acc = fma(wr[q], wr[q], acc);
-            }
-            store4(w + 4 * g, wr);
+    if (pass && *a.gate == 0.0) return;
+    const int c = blockIdx.x, nv = j + 1;
+    double s = 0;
+    for (int b = threadIdx.x; b < nblk; b += blockDim.x) s += partial[(int64_t)b * (nv + 1) + c];
+    s = block_sum(s, s_red);
+    if (threadIdx.x != 0) return;
+    const double sj = pass ? 1.0 : a.scal[j];
+    if (c == nv) {
+        if (!pass) *a.before = s * sj * sj;
+        return;
+    }
+    const double h = s * a.scal[c] * sj;
+    a.coef[c] = h * a.scal[c];
+    a.hcol[c] = pass ? a.hcol[c] + h : h;
+}
+
+// gate = 1 when the first pass cancelled enough for a second one (the DGKS test)
+__global__ void __launch_bounds__(kBlock) k_gmres_gate(GmresSc a, const double* __restrict__ ss, int nblk) {
+    __shared__ double s_red[kBlock / 64];
+    double s = 0;
+    for (int b = threadIdx.x; b < nblk; b += blockDim.x) s += ss[b];
+    s = block_sum(s, s_red);
+    if (threadIdx.x == 0) *a.gate = s < 0.5 * *a.before ? 1.0 : 0.0;
+}
+
+// Closes Arnoldi step j: the new vector's norm from gs_update's partials, the Givens rotations of
+// column j and of the right-hand side, and (|g_{j+1}|, h_{j+1,j}) to the host.
+__global__ void __launch_bounds__(kBlock) k_gmres_step(GmresSc a, const double* __restrict__ ss, int nblk, int j,
+                                                       HostSlot* slot, uint64_t seq) {
+    __shared__ double s_red[kBlock / 64], s_h[32], s_c[32], s_s[32];
+    const int t = threadIdx.x;
+    if (t <= j) s_h[t] = a.hcol[t];
+    if (t < j) {
+        s_c[t] = a.cs[t];
+        s_s[t] = a.sn[t];
+    }
+    double s = 0;
+    for (int b = t; b < nblk; b += blockDim.x) s += ss[b];
+    s = block_sum(s, s_red);
+    if (t == 0) {
+        const double hn = sqrt(s);
+        double p = s_h[0];
+        for (int i = 0; i < j; ++i) {
+            const double q = s_h[i + 1];
+            s_h[i] = s_c[i] * p + s_s[i] * q;
+            p = -s_s[i] * p + s_c[i] * q;
         }
-    } else {
-        for (int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; k < n; k += stride) {
-            double wk = (double)w[k];
+        const double rr = hypot(p, hn);
+        const double c = rr > 0 ? p / rr : 1.0, sn = rr > 0 ? hn / rr : 0.0;
+        s_h[j] = rr;
+        const double gj = a.g[j];
+        a.cs[j] = c;
+        a.sn[j] = sn;
+        a.g[j] = c * gj;
+        a.g[j + 1] = -sn * gj;
+        a.scal[j + 1] = hn > 0 ? 1.0 / hn : 0.0;
+        slot->v[0] = fabs(sn * gj);
+        slot->v[1] = hn;
+        __hip_atomic_store(&slot->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+    __syncthreads();
+    if (t <= j) a.H[(int64_t)j * 32 + t] = s_h[t];
+}
+
+__global__ void k_gmres_start(GmresSc a, double beta) {
+    a.scal[0] = 1.0;
+    a.g[0] = beta;
+}
+
+// y from the k x k triangular system (one wavefront, column by column), as factors of the stored
+// basis vectors
+__global__ void __launch_bounds__(64) k_gmres_y(GmresSc a, int k) {
+    const int t = threadIdx.x;
+    double g = t < k ? a.g[t] : 0.0, y = 0;
+    for (int i = k - 1; i >= 0; --i) {
+        const double yi = __shfl(g, i) / a.H[i * 32 + i];
+        if (t == i) y = yi;
+        if (t < i) g = fma(-a.H[i * 32 + t], yi, g);
+    }
+    if (t < k) a.coef[t] = y * a.scal[t];
+}
+
+// w = scale w - sum_c coef[c] V_c, partial[block] = sum of the stored w.w
+template <typename T>
+__global__ void __launch_bounds__(kBlock) k_gs_update(int64_t n, int64_t ld, const T* __restrict__ V, int nv,
+                                                      const double* __restrict__ coef,
+                                                      const double* __restrict__ scale, T* __restrict__ w,
+                                                      double* __restrict__ partial, const double* __restrict__ gate) {
+    if (gate && *gate == 0.0) return;
+    __shared__ double s_red[kBlock / 64];
+    const double sj = scale ? *scale : 1.0;
+    double acc = 0.0;
+    const int64_t stride = (int64_t)gridDim.x * blockDim.x, n4 = (n + 3) / 4;
+    for (int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; g < n4; g += stride) {
+        double wv[4];
+        load4_tail(w, g, n, wv);
 #pragma unroll
-            for (int c = 0; c < kNV; ++c)
-                if (c < nv) wk = fma(-hc[c], (double)V[(int64_t)c * n + k], wk);
-            const T wt = (T)wk;
-            w[k] = wt;
-            acc = fma((double)wt, (double)wt, acc);
+        for (int q = 0; q < 4; ++q) wv[q] *= sj;
+        for (int c0 = 0; c0 < nv; c0 += kCols) {
+            double vv[kCols][4];
+#pragma unroll
+            for (int c = 0; c < kCols; ++c) load4_tail(V + (int64_t)min(c0 + c, nv - 1) * ld, g, n, vv[c]);
+#pragma unroll
+            for (int c = 0; c < kCols; ++c) {
+                const double hc = c0 + c < nv ? coef[c0 + c] : 0.0;
+#pragma unroll
+                for (int q = 0; q < 4; ++q) wv[q] = c0 + c < nv ? fma(-hc, vv[c][q], wv[q]) : wv[q];
+            }
+        }
+        double wr[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            wr[q] = (double)(T)wv[q];  // the value actually stored
+            acc = fma(wr[q], wr[q], acc);
+        }
+        if (4 * g + 4 <= n) {
+            store4(w + 4 * g, wr);
+        } else {
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                if (4 * g + q < n) w[4 * g + q] = (T)wr[q];
         }
     }
     const double s = block_sum(acc, s_red);
     if (threadIdx.x == 0) partial[blockIdx.x] = s;
 }
 
+// u = sum_c coef[c] V_c
 template <typename T>
-__global__ void __launch_bounds__(kBlock) k_scale_by_inv(int64_t n, const T* __restrict__ w, const double* nrm,
-                                                         T* __restrict__ v) {
-    const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= n) return;
-    const double inv = 1.0 / sqrt(*nrm);
-    v[k] = (T)((double)w[k] * inv);
-}
-
-template <typename T>
-__global__ void __launch_bounds__(kBlock) k_combine(int64_t n, const T* __restrict__ V, int nv,
-                                                    const double* __restrict__ y, T* __restrict__ u) {
+__global__ void __launch_bounds__(kBlock) k_combine(int64_t n, int64_t ld, const T* __restrict__ V, int nv,
+                                                    const double* __restrict__ coef, T* __restrict__ u) {
     const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= n) return;
     double s = 0.0;
-    for (int c = 0; c < nv; ++c) s = fma(y[c], (double)V[(int64_t)c * n + k], s);
+    for (int c0 = 0; c0 < nv; c0 += kCols) {
+        double v[kCols];
+#pragma unroll
+        for (int c = 0; c < kCols; ++c) v[c] = (double)V[(int64_t)min(c0 + c, nv - 1) * ld + k];
+#pragma unroll
+        for (int c = 0; c < kCols; ++c)
+            if (c0 + c < nv) s = fma(coef[c0 + c], v[c], s);
+    }
     u[k] = (T)s;
 }
 
@@ -763,40 +862,50 @@ void spmv_col(hipStream_t s, int64_t F, int L, const int32_t* rp, const T* val, 
         hipLaunchKernelGGL((k_spmv_col<T, false>), g, blk, 0, s, F, L, rp, val, neigh, slots, x, b, y, partial);
 }
 
-// 4-wide loads need n % 4 == 0 and 32-byte aligned vector starts
-template <typename T>
-static bool vec4_ok(int64_t n, const void* a, const void* b) {
-    return n % 4 == 0 && ((uintptr_t)a % 32) == 0 && ((uintptr_t)b % 32) == 0;
+// 4-wide loads: vectors start on 32 bytes (device allocations do; the basis has a padded ld)
+static void check_vec(const void* a, const void* b, int64_t ld) {
+    if (((uintptr_t)a | (uintptr_t)b) % 32 || ld % 4) throw Error(PBSM3D_EINVAL, "unaligned Krylov vector");
 }
 
 template <typename T>
-void mdot(hipStream_t s, int64_t n, const T* V, int nv, const T* w, double* partial, int nblk) {
-    if (vec4_ok<T>(n, V, w))
-        hipLaunchKernelGGL((k_mdot<T, true>), dim3(nblk), dim3(kBlock), 0, s, n, V, nv, w, partial);
+void mdot(hipStream_t s, int64_t n, const T* V, int64_t ld, int nv, const T* w, double* partial, int nblk,
+          const double* gate) {
+    check_vec(V, w, nv > 1 ? ld : 0);
+    if (n * (int64_t)sizeof(T) <= kCachedVector)
+        hipLaunchKernelGGL((k_mdot<T, 1>), dim3(nblk, nv > kCols ? (nv + kCols - 1) / kCols : 1), dim3(kBlock), 0, s, n,
+                           ld, V, nv, w, partial, gate);
     else
-        hipLaunchKernelGGL((k_mdot<T, false>), dim3(nblk), dim3(kBlock), 0, s, n, V, nv, w, partial);
+        hipLaunchKernelGGL((k_mdot<T, 4>), dim3(nblk), dim3(kBlock), 0, s, n, ld, V, nv, w, partial, gate);
 }
 
 void reduce_cols(hipStream_t s, const double* partial, int nblk, int stride, int ncols, double* out) {
     hipLaunchKernelGGL(k_reduce_cols, dim3(ncols), dim3(kBlock), 0, s, partial, nblk, stride, out);
 }
 
+void gmres_start(hipStream_t s, const GmresSc& a, double beta) {
+    hipLaunchKernelGGL(k_gmres_start, dim3(1), dim3(1), 0, s, a, beta);
+}
+void gmres_h(hipStream_t s, const GmresSc& a, const double* partial, int nblk, int j, int pass) {
+    hipLaunchKernelGGL(k_gmres_h, dim3(j + 2), dim3(kBlock), 0, s, a, partial, nblk, j, pass);
+}
+void gmres_gate(hipStream_t s, const GmresSc& a, const double* ss, int nblk) {
+    hipLaunchKernelGGL(k_gmres_gate, dim3(1), dim3(kBlock), 0, s, a, ss, nblk);
+}
+void gmres_step(hipStream_t s, const GmresSc& a, const double* ss, int nblk, int j, HostSlot* slot, uint64_t seq) {
+    hipLaunchKernelGGL(k_gmres_step, dim3(1), dim3(kBlock), 0, s, a, ss, nblk, j, slot, seq);
+}
+void gmres_y(hipStream_t s, const GmresSc& a, int k) { hipLaunchKernelGGL(k_gmres_y, dim3(1), dim3(64), 0, s, a, k); }
+
 template <typename T>
-void gs_update(hipStream_t s, int64_t n, const T* V, int nv, const double* h, T* w, double* partial, int nblk) {
-    if (vec4_ok<T>(n, V, w))
-        hipLaunchKernelGGL((k_gs_update<T, true>), dim3(nblk), dim3(kBlock), 0, s, n, V, nv, h, w, partial);
-    else
-        hipLaunchKernelGGL((k_gs_update<T, false>), dim3(nblk), dim3(kBlock), 0, s, n, V, nv, h, w, partial);
+void gs_update(hipStream_t s, int64_t n, const T* V, int64_t ld, int nv, const double* coef, const double* scale, T* w,
+               double* partial, int nblk, const double* gate) {
+    check_vec(V, w, ld);
+    hipLaunchKernelGGL((k_gs_update<T>), dim3(nblk), dim3(kBlock), 0, s, n, ld, V, nv, coef, scale, w, partial, gate);
 }
 
 template <typename T>
-void scale_by_inv(hipStream_t s, int64_t n, const T* w, const double* nrm, T* v) {
-    hipLaunchKernelGGL((k_scale_by_inv<T>), dim3(grid_for(n)), dim3(kBlock), 0, s, n, w, nrm, v);
-}
-
-template <typename T>
-void combine(hipStream_t s, int64_t n, const T* V, int nv, const double* y, T* u) {
-    hipLaunchKernelGGL((k_combine<T>), dim3(grid_for(n)), dim3(kBlock), 0, s, n, V, nv, y, u);
+void combine(hipStream_t s, int64_t n, const T* V, int64_t ld, int nv, const double* coef, T* u) {
+    hipLaunchKernelGGL((k_combine<T>), dim3(grid_for(n)), dim3(kBlock), 0, s, n, ld, V, nv, coef, u);
 }
 
 void absmax(hipStream_t s, int64_t n, const double* b, double* partial, int nblk) {
@@ -896,10 +1005,10 @@ void copy_f64(hipStream_t s, int64_t n, const double* a, double* b) {
     template void spmv<T>(hipStream_t, int64_t, const int32_t*, const int32_t*, const T*, const T*, T*);           \
     template void residual<T>(hipStream_t, int64_t, const int32_t*, const int32_t*, const T*, const T*, const T*,   \
                               T*, double*, int);                                                                   \
-    template void mdot<T>(hipStream_t, int64_t, const T*, int, const T*, double*, int);                            \
-    template void gs_update<T>(hipStream_t, int64_t, const T*, int, const double*, T*, double*, int);              \
-    template void scale_by_inv<T>(hipStream_t, int64_t, const T*, const double*, T*);                              \
-    template void combine<T>(hipStream_t, int64_t, const T*, int, const double*, T*);                              \
+    template void mdot<T>(hipStream_t, int64_t, const T*, int64_t, int, const T*, double*, int, const double*);     \
+    template void gs_update<T>(hipStream_t, int64_t, const T*, int64_t, int, const double*, const double*, T*,       \
+                               double*, int, const double*);                                                       \
+    template void combine<T>(hipStream_t, int64_t, const T*, int64_t, int, const double*, T*);                      \
     template void pc_column<T>(hipStream_t, int64_t, int, const T*, const T*, const T*, const T*, T*);             \
     template void pc_jacobi<T>(hipStream_t, int64_t, const double*, const T*, T*);                                \
     template void scale_host<T>(hipStream_t, int64_t, const T*, double, T*);                                       \

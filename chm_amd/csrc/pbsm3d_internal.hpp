@@ -54,7 +54,8 @@ struct DevBuf {
     size_t bytes() const { return n * sizeof(T); }
 };
 
-// Pinned host staging buffer (hipHostMalloc / hipHostFree).
+// Pinned host staging buffer (hipHostMalloc / hipHostFree), coherent: a kernel's stores reach a
+// host that polls them while the stream runs.
 template <typename T>
 struct HostBuf {
     T* p = nullptr;
@@ -69,7 +70,7 @@ struct HostBuf {
         if (count <= n && p) return;
         if (p) (void)hipHostFree(p);
         p = nullptr;
-        PB_HIP(hipHostMalloc((void**)&p, count * sizeof(T), hipHostMallocDefault));
+        PB_HIP(hipHostMalloc((void**)&p, count * sizeof(T), hipHostMallocMapped | hipHostMallocCoherent));
         n = count;
     }
 };
