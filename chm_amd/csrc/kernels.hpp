@@ -418,5 +418,7 @@ void scale_f64_to_f32_host(hipStream_t s, int64_t n, const double* r, double alp
 void axpy_dev_scaled_f32(hipStream_t s, int64_t n, const double* scale, const float* x, double* y);  // y += (*scale) x
 void axpy_f64(hipStream_t s, int64_t n, double alpha, const double* x, double* y);
 void copy_f64(hipStream_t s, int64_t n, const double* a, double* b);
+// out = v + y - ay (out may be y)
+void neumann_step(hipStream_t s, int64_t n, const double* v, const double* y, const double* ay, double* out);
 
 }  // namespace pb

@@ -1,0 +1,68 @@
+"""FP64 GMRES beyond one plain cycle: the cycles on the split operator with the Neumann
+polynomial (from the third cycle of a small system, every cycle of a large one), the plain restarts
+where the split operator is not available, and the iteration limit inside them."""
+import numpy as np
+import pytest
+
+from chm_amd import abi, meshgen
+from tests.conftest import rel_err
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("points,layers,restart", [
+    (13, 2, 1), (13, 5, 3), (300, 5, 3), (300, 16, 4), (300, 17, 4), (2500, 10, 6), (2501, 7, 31),
+    (106000, 10, 30)])  # the last: a basis vector of more than 16 MB
+def test_restarted_gmres_solves_the_same_system(points, layers, restart):
+    """Both solve to 1e-12, so their fields differ by the forward error of that tolerance alone."""
+    from chm_amd import pbsm3d as pb
+
+    print(f"[case] gmres cycles points={points} L={layers} restart={restart}", flush=True)
+    mesh = meshgen.synthetic_mesh(points, seed=5)
+    g = pb.face_geometry(mesh)
+    fo = meshgen.forcing_c2(mesh.n_faces, seed=9)
+    ref = pb.Context(g, pb.default_config(nLayer=layers, tol=1e-12, krylov=abi.KRYLOV_BICGSTAB, max_iters=4000))
+    ro, rst = ref.step(fo, want_fields=True)
+    ctx = pb.Context(g, pb.default_config(nLayer=layers, tol=1e-12, restart=restart, max_iters=4000))
+    for _ in range(2):  # the second step reuses the work vectors
+        ctx.set_state(np.zeros(mesh.n_faces), np.zeros(mesh.n_faces))
+        o, st = ctx.step(fo, want_fields=True)
+        assert rst["susp_resid"] <= 1e-12 and st["susp_resid"] <= 1e-12
+        for k in ("conc", "Qsusp", "Qsubl", "qdep"):
+            assert rel_err(o[k], ro[k]) < 1e-8, (k, rel_err(o[k], ro[k]))
+    ctx.close()
+    ref.close()
+
+
+def test_iteration_limit_inside_the_later_cycles():
+    from chm_amd import pbsm3d as pb
+
+    print("[case] gmres cycles iteration limit", flush=True)
+    mesh = meshgen.synthetic_mesh(2500, seed=0)
+    g = pb.face_geometry(mesh)
+    fo = meshgen.forcing_c2(mesh.n_faces, seed=9)
+    for limit in (8, 9, 11, 13):  # two plain cycles take 8; what is left is 0, 1, 3 and 5
+        ctx = pb.Context(g, pb.default_config(nLayer=10, restart=4, max_iters=limit))
+        with pytest.raises(pb.Pbsm3dError) as e:
+            ctx.step(fo)
+        assert e.value.code == abi.PBSM3D_ENOCONV
+        ctx.close()
+
+
+def test_second_orthogonalisation_pass():
+    """ortho_passes = 2 adds the conditional pass; the solution is the same."""
+    from chm_amd import pbsm3d as pb
+
+    print("[case] gmres two passes", flush=True)
+    mesh = meshgen.synthetic_mesh(1201, seed=6)
+    g = pb.face_geometry(mesh)
+    fo = meshgen.forcing_c2(mesh.n_faces, seed=3)
+    out = []
+    for passes in (1, 2):
+        ctx = pb.Context(g, pb.default_config(nLayer=6, tol=1e-12, ortho_passes=passes, max_iters=4000))
+        o, st = ctx.step(fo, want_fields=True)
+        assert st["susp_resid"] <= 1e-12 and st["dep_resid"] <= 1e-12
+        out.append(o)
+        ctx.close()
+    for k in ("conc", "qdep"):
+        assert rel_err(out[0][k], out[1][k]) < 1e-8
