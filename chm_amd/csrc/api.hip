@@ -259,10 +259,10 @@ std::vector<double> to_jmajor(const double* a, int64_t F) {
 double max_abs(pbsm3d_ctx* c, const double* v, int64_t n) {
     const int nblk = (int)std::min<int64_t>(kReduceBlocks, (n + kBlock - 1) / kBlock);
     absmax(c->stream, n, v, c->red_partial.p, nblk);
-    reduce_max(c->stream, c->red_partial.p, nblk, c->red_out.p);
-    PB_HIP(hipMemcpyAsync(c->red_host.p, c->red_out.p, sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    PB_HIP(hipStreamSynchronize(c->stream));
-    return c->red_host.p[0];
+    report_max(c->stream, c->red_partial.p, nblk, c->red_dslot, ++c->red_seq);
+    PB_HIP(hipGetLastError());
+    wait_slot(c->stream, c->red_slot.p, c->red_seq);
+    return c->red_slot.p[0].v[0];
 }
 
 float ms_between(hipEvent_t a, hipEvent_t b) {
@@ -638,8 +638,9 @@ int pbsm3d_create(pbsm3d_ctx** out, const pbsm3d_mesh* m, const pbsm3d_config* c
         c->ws64.passes = c->ws32.passes = c->wd64.passes = cfg->ortho_passes;
         c->fscal.alloc(3 * F);
         c->red_partial.alloc(kReduceBlocks);
-        c->red_out.alloc(4);
-        c->red_host.alloc(4);
+        c->red_slot.alloc(1);
+        c->red_slot.p[0].seq = 0;
+        PB_HIP(hipHostGetDevicePointer((void**)&c->red_dslot, c->red_slot.p, 0));
         PB_HIP(hipStreamSynchronize(s));
     });
     if (rc != PBSM3D_OK) return rc;

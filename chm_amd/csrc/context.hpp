@@ -70,8 +70,10 @@ struct pbsm3d_ctx {
     pb::GmresWork<float> ws32;
     pb::BicgWork<double> bw64;
     pb::BicgWork<float> bw32;
-    pb::DevBuf<double> red_partial, red_out;
-    pb::HostBuf<double> red_host;
+    pb::DevBuf<double> red_partial;
+    pb::HostBuf<pb::HostSlot> red_slot;
+    pb::HostSlot* red_dslot = nullptr;
+    uint64_t red_seq = 0;
     // learned warm start
     pb::Mlp* warm = nullptr;          // not owned
     pb::DevBuf<float> feat, pred;     // [F x 16], [F x 11]

@@ -170,8 +170,6 @@ inline int64_t spmv_col_blocks(int64_t F) { return (F + kBlock - 1) / kBlock; }
 template <typename T>
 void mdot(hipStream_t s, int64_t n, const T* V, int64_t ld, int nv, const T* w, double* partial, int nblk,
           const double* gate = nullptr);
-// out[c] = sum_b partial[b*stride + c] for c < ncols (fixed order, deterministic)
-void reduce_cols(hipStream_t s, const double* partial, int nblk, int stride, int ncols, double* out);
 // w = (*scale) w - sum_c coef[c] V_c (scale NULL: 1); partial[block] = sum w.w (after the update)
 template <typename T>
 void gs_update(hipStream_t s, int64_t n, const T* V, int64_t ld, int nv, const double* coef, const double* scale, T* w,
@@ -210,6 +208,9 @@ struct HostSlot {
     uint64_t seq;
 };
 void wait_slot(hipStream_t s, const HostSlot* slot, uint64_t seq);
+// slot->v[0] = the sum / the largest of nblk partials (fixed order, deterministic)
+void report_sum(hipStream_t s, const double* partial, int nblk, HostSlot* slot, uint64_t seq);
+void report_max(hipStream_t s, const double* partial, int nblk, HostSlot* slot, uint64_t seq);
 void gmres_start(hipStream_t s, const GmresSc& a, double beta);
 void gmres_h(hipStream_t s, const GmresSc& a, const double* partial, int nblk, int j, int pass);
 void gmres_gate(hipStream_t s, const GmresSc& a, const double* ss, int nblk);
@@ -217,7 +218,6 @@ void gmres_step(hipStream_t s, const GmresSc& a, const double* ss, int nblk, int
 void gmres_y(hipStream_t s, const GmresSc& a, int k);
 // max |b| per block into partial
 void absmax(hipStream_t s, int64_t n, const double* b, double* partial, int nblk);
-void reduce_max(hipStream_t s, const double* partial, int nblk, double* out);
 
 // preconditioners (z = M^-1 r)
 template <typename T>
@@ -402,12 +402,12 @@ void bicg_xr_dev(hipStream_t s, int64_t n, const T* ph, const T* sh, const T* sv
 // stage 0 starts a run (rho, rr; clears sc[SC_STOP]), stage 1 ends an iteration: new rho and
 // rr, and sc[SC_STOP] set when a breakdown was flagged (sc[SC_FLAG] 1: rh.v = 0, 2: omega = 0,
 // 3: non-finite residual), sqrt(rr) <= stop_abs or rr is not finite.  Stage 1 does nothing once
-// sc[SC_STOP] is set.  host_slot (may be NULL): device-visible pinned host memory that
-// receives sc[0 .. SC_COUNT) after the update.  restart_eps > 0: stage 1 restarts the shadow
+// sc[SC_STOP] is set.  slot receives sc[0 .. SC_COUNT) after the update, as report seq.
+// restart_eps > 0: stage 1 restarts the shadow
 // residual when |rh.r| < restart_eps ||rh|| ||r|| (a near breakdown of the Lanczos recurrence):
 // rho = r.r, sc[SC_RESTART] = 1, and the next p kernel sets rh = p = r.
 void bicg_stage(hipStream_t s, const double* partial, int64_t nblk, int stride, int stage, double* sc,
-                double stop_abs = 0.0, double* host_slot = nullptr, double restart_eps = 0.0);
+                double stop_abs, HostSlot* slot, uint64_t seq, double restart_eps);
 
 // conversions / vector updates
 template <typename T>

@@ -63,10 +63,11 @@ void GmresWork<T>::ensure(int64_t n_, int m_) {
     if (pbytes < spmv_blocks) pbytes = spmv_blocks;
     partial.alloc(pbytes);
     ss.alloc(kReduceBlocks);
-    dsc.alloc(GmresSc::kDoubles + 1);
-    hsc.alloc(1);
-    slot.alloc(2);
-    slot.p[0].seq = slot.p[1].seq = seq = 0;
+    dsc.alloc(GmresSc::kDoubles);
+    slot.alloc(4);
+    for (int k = 0; k < 4; ++k) slot.p[k].seq = 0;
+    seq = 0;
+    PB_HIP(hipHostGetDevicePointer((void**)&dslot, slot.p, 0));
 }
 
 // How far the last known residual must lie above the target for the host to queue another Arnoldi
@@ -81,8 +82,6 @@ int gmres_cycle(hipStream_t s, GmresWork<T>& w, const CsrOp<T>& A, const PcFn<T>
     const int nblk = reduce_blocks4(n);
     T* V = w.V.p;
     const GmresSc sc = GmresSc::of(w.dsc.p);
-    HostSlot* dslot = nullptr;
-    PB_HIP(hipHostGetDevicePointer((void**)&dslot, w.slot.p, 0));
     if (max_steps > w.m) max_steps = w.m;
 
     scale_host<T>(s, n, r0, 1.0 / beta, V);
@@ -109,7 +108,7 @@ int gmres_cycle(hipStream_t s, GmresWork<T>& w, const CsrOp<T>& A, const PcFn<T>
             gmres_h(s, sc, w.partial.p, nblk, j, 1);
             gs_update<T>(s, n, V, ld, j + 1, sc.coef, nullptr, vj1, w.ss.p, nblk, sc.gate);
         }
-        gmres_step(s, sc, w.ss.p, nblk, j, dslot + (j & 1), ++w.seq);
+        gmres_step(s, sc, w.ss.p, nblk, j, w.dslot + (j & 1), ++w.seq);
         PB_HIP(hipGetLastError());
     };
     double res = beta;
@@ -135,15 +134,6 @@ int gmres_cycle(hipStream_t s, GmresWork<T>& w, const CsrOp<T>& A, const PcFn<T>
     return known;
 }
 
-double dev_norm2(hipStream_t s, GmresWork<double>& w, int64_t n, const double* v) {
-    const int nblk = reduce_blocks(n);
-    mdot<double>(s, n, nullptr, 0, 0, v, w.partial.p, nblk);
-    reduce_cols(s, w.partial.p, nblk, 1, 1, w.dsc.p + GmresSc::kDoubles);
-    PB_HIP(hipMemcpyAsync(w.hsc.p, w.dsc.p + GmresSc::kDoubles, sizeof(double), hipMemcpyDeviceToHost, s));
-    PB_HIP(hipStreamSynchronize(s));
-    return std::sqrt(w.hsc.p[0]);
-}
-
 namespace {
 // A start whose residual exceeds ||b|| (that of x0 = 0) is dropped: x is reset
 // to zero and the caller recomputes the residual.  Records ||r0|| / ||b||.  The
@@ -157,28 +147,56 @@ bool drop_worse_start(hipStream_t s, SolveInfo& info, double beta, double nb, do
     return true;
 }
 
+// The norms below are queued with the number of their report, and read by norm_report.
 template <typename T>
-double residual_norm(hipStream_t s, GmresWork<T>& w, const CsrOp<double>& A, const double* x, const double* b,
-                     double* r) {
+uint64_t queue_residual(hipStream_t s, GmresWork<T>& w, const CsrOp<double>& A, const double* x, const double* b,
+                        double* r) {
     int nblk = 0;
     {
         ProfScope ps(A.prof, s, PBSM3D_K_RESIDUAL);
         nblk = op_residual(s, A, x, b, r, w.partial.p);
     }
-    reduce_cols(s, w.partial.p, nblk, 1, 1, w.dsc.p + GmresSc::kDoubles);
-    PB_HIP(hipMemcpyAsync(w.hsc.p, w.dsc.p + GmresSc::kDoubles, sizeof(double), hipMemcpyDeviceToHost, s));
-    PB_HIP(hipStreamSynchronize(s));
-    return std::sqrt(w.hsc.p[0]);
+    report_sum(s, w.partial.p, nblk, w.dslot + 2, ++w.seq);
+    return w.seq;
+}
+
+template <typename T>
+uint64_t queue_norm(hipStream_t s, GmresWork<T>& w, int64_t n, const double* v) {
+    const int nblk = reduce_blocks4(n);
+    mdot<double>(s, n, nullptr, 0, 0, v, w.partial.p, nblk);
+    report_sum(s, w.partial.p, nblk, w.dslot + 3, ++w.seq);
+    return w.seq;
+}
+
+template <typename T>
+double norm_report(hipStream_t s, GmresWork<T>& w, int slot, uint64_t seq) {
+    PB_HIP(hipGetLastError());
+    wait_slot(s, w.slot.p + slot, seq);
+    return std::sqrt(w.slot.p[slot].v[0]);
+}
+
+template <typename T>
+double residual_norm(hipStream_t s, GmresWork<T>& w, const CsrOp<double>& A, const double* x, const double* b,
+                     double* r) {
+    return norm_report(s, w, 2, queue_residual(s, w, A, x, b, r));
 }
 
 template <typename T>
 double norm_of(hipStream_t s, GmresWork<T>& w, int64_t n, const double* v) {
-    const int nblk = reduce_blocks(n);
-    mdot<double>(s, n, nullptr, 0, 0, v, w.partial.p, nblk);
-    reduce_cols(s, w.partial.p, nblk, 1, 1, w.dsc.p + GmresSc::kDoubles);
-    PB_HIP(hipMemcpyAsync(w.hsc.p, w.dsc.p + GmresSc::kDoubles, sizeof(double), hipMemcpyDeviceToHost, s));
-    PB_HIP(hipStreamSynchronize(s));
-    return std::sqrt(w.hsc.p[0]);
+    return norm_report(s, w, 3, queue_norm(s, w, n, v));
+}
+
+// ||b|| and the start's residual: one wait for both.  False where b is zero; x is zero then.
+template <typename T>
+bool start_norms(hipStream_t s, GmresWork<T>& w, const CsrOp<double>& A, double* x, const double* b, double* r,
+                 SolveInfo& info, double& nb, double& beta) {
+    const uint64_t qb = queue_norm(s, w, A.n, b), qr = queue_residual(s, w, A, x, b, r);
+    nb = norm_report(s, w, 3, qb);
+    beta = norm_report(s, w, 2, qr);
+    if (nb != 0.0) return true;
+    PB_HIP(hipMemsetAsync(x, 0, sizeof(double) * A.n, s));
+    info.converged = true;
+    return false;
 }
 }  // namespace
 
@@ -218,13 +236,8 @@ SolveInfo gmres_solve(hipStream_t s, GmresWork<double>& w, const CsrOp<double>& 
                       const std::function<SplitCycles()>& later) {
     SolveInfo info;
     w.ensure(A.n, m);
-    const double nb = norm_of(s, w, A.n, b);
-    if (nb == 0.0) {
-        PB_HIP(hipMemsetAsync(x, 0, sizeof(double) * A.n, s));
-        info.converged = true;
-        return info;
-    }
-    double beta = residual_norm(s, w, A, x, b, r);
+    double nb = 0, beta = 0;
+    if (!start_norms(s, w, A, x, b, r, info, nb, beta)) return info;
     if (drop_worse_start(s, info, beta, nb, x, A.n)) beta = residual_norm(s, w, A, x, b, r);
     // The split cycles take `degree` operator applications per basis vector, so a cycle reaches
     // degree times as far for the same basis traffic, and restarts forget the slow modes that much
@@ -270,13 +283,8 @@ SolveInfo mixed_solve(hipStream_t s, GmresWork<float>& w, const CsrOp<double>& A
                       int maxit, double tol, double inner_rtol) {
     SolveInfo info;
     w.ensure(A64.n, m);
-    const double nb = norm_of(s, w, A64.n, b);
-    if (nb == 0.0) {
-        PB_HIP(hipMemsetAsync(x, 0, sizeof(double) * A64.n, s));
-        info.converged = true;
-        return info;
-    }
-    double beta = residual_norm(s, w, A64, x, b, r);
+    double nb = 0, beta = 0;
+    if (!start_norms(s, w, A64, x, b, r, info, nb, beta)) return info;
     if (drop_worse_start(s, info, beta, nb, x, A64.n)) beta = residual_norm(s, w, A64, x, b, r);
     while (true) {
         info.resid = beta / nb;
@@ -313,10 +321,10 @@ void BicgWork<T>::ensure(int64_t n_) {
     dsc.alloc(SC_COUNT);
     ss_partial.alloc(kReduceBlocks);
     xr_partial.alloc(2 * (size_t)kReduceBlocks);
-    hsc.alloc(2 * SC_COUNT);
-    PB_HIP(hipHostGetDevicePointer((void**)&hsc_dev, hsc.p, 0));
-    for (hipEvent_t& e : ev)
-        if (!e) PB_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    slot.alloc(2);
+    slot.p[0].seq = slot.p[1].seq = 0;
+    seq = 0;
+    PB_HIP(hipHostGetDevicePointer((void**)&dslot, slot.p, 0));
 }
 
 namespace {
@@ -355,11 +363,6 @@ int bicg_run(hipStream_t s, BicgWork<T>& w, const CsrOp<T>& A, const PcFn<T>& M,
     T* ph = pc ? w.ph.p : w.p.p;  // the preconditioned search directions
     T* sh = pc ? w.sh.p : w.s.p;
     double* sc = w.dsc.p;
-    double* h = w.hsc.p;
-    auto fetch = [&]() {
-        PB_HIP(hipMemcpyAsync(h, sc, sizeof(double) * SC_COUNT, hipMemcpyDeviceToHost, s));
-        PB_HIP(hipStreamSynchronize(s));
-    };
     // r = b - A x, rh = r, (rh.r, r.r)
     if (x_zero) {
         PB_HIP(hipMemcpyAsync(w.r.p, b, n * sizeof(T), hipMemcpyDeviceToDevice, s));
@@ -372,9 +375,11 @@ int bicg_run(hipStream_t s, BicgWork<T>& w, const CsrOp<T>& A, const PcFn<T>& M,
     }
     PB_HIP(hipMemcpyAsync(w.rh.p, w.r.p, n * sizeof(T), hipMemcpyDeviceToDevice, s));
     mdot<T>(s, n, w.rh.p, 0, 1, w.r.p, w.partial.p, nblk);
-    bicg_stage(s, w.partial.p, nblk, 2, 0, sc);
-    fetch();
-    double rr = std::sqrt(h[SC_RR]);
+    bicg_stage(s, w.partial.p, nblk, 2, 0, sc, 0.0, w.dslot, ++w.seq, 0.0);
+    PB_HIP(hipGetLastError());
+    wait_slot(s, w.slot.p, w.seq);
+    double rr = std::sqrt(w.slot.p[0].v[SC_RR]);
+    const uint64_t seq0 = w.seq;
     *res_out = rr;
     if (stop_rel) stop_abs *= rr;
     if (rr <= stop_abs) return 0;
@@ -413,16 +418,16 @@ int bicg_run(hipStream_t s, BicgWork<T>& w, const CsrOp<T>& A, const PcFn<T>& M,
             bicg_xr_dev<T>(s, n, ph, sh, w.s.p, w.t.p, w.rh.p, sc, x, w.r.p, w.xr_partial.p, nvec, w.partial.p, nb,
                            w.ss_partial.p, nvec);
             // rho, rr, the stop test, and the scalars into host slot it % 2 (no copy launch)
-            bicg_stage(s, w.xr_partial.p, nvec, 2, 1, sc, stop_abs, w.hsc_dev + SC_COUNT * (it & 1), restart_eps);
+            bicg_stage(s, w.xr_partial.p, nvec, 2, 1, sc, stop_abs, w.dslot + (it & 1), ++w.seq, restart_eps);
         }
-        PB_HIP(hipEventRecord(w.ev[it & 1], s));
+        PB_HIP(hipGetLastError());
     };
     if (maxit <= 0) return 0;
     iterate(1);
     for (int it = 1;; ++it) {
         if (it < maxit) iterate(it + 1);
-        PB_HIP(hipEventSynchronize(w.ev[it & 1]));
-        const double* hk = h + SC_COUNT * (it & 1);
+        wait_slot(s, w.slot.p + (it & 1), seq0 + it);
+        const double* hk = w.slot.p[it & 1].v;
         rr = std::sqrt(hk[SC_RR]);
         *res_out = rr;
         if (hk[SC_STOP] != 0.0 || it >= maxit) {
@@ -438,13 +443,8 @@ SolveInfo bicgstab_solve(hipStream_t s, BicgWork<double>& w, GmresWork<double>& 
     SolveInfo info;
     w.ensure(A.n);
     GmresWork<double>& dummy = gw;
-    const double nb = norm_of(s, dummy, A.n, b);
-    if (nb == 0.0) {
-        PB_HIP(hipMemsetAsync(x, 0, sizeof(double) * A.n, s));
-        info.converged = true;
-        return info;
-    }
-    double beta = residual_norm(s, dummy, A, x, b, w.r.p);
+    double nb = 0, beta = 0;
+    if (!start_norms(s, dummy, A, x, b, w.r.p, info, nb, beta)) return info;
     if (drop_worse_start(s, info, beta, nb, x, A.n)) beta = residual_norm(s, dummy, A, x, b, w.r.p);
     while (true) {
         info.resid = beta / nb;
@@ -476,13 +476,8 @@ SolveInfo bicgstab_split(hipStream_t s, BicgWork<T>& w, GmresWork<T>& gw, const 
     SolveInfo info;
     const int64_t n = A64.n;
     w.ensure(n);
-    const double nb = norm_of(s, gw, n, b);
-    if (nb == 0.0) {
-        PB_HIP(hipMemsetAsync(x, 0, sizeof(double) * n, s));
-        info.converged = true;
-        return info;
-    }
-    double beta = residual_norm(s, gw, A64, x, b, r);
+    double nb = 0, beta = 0;
+    if (!start_norms(s, gw, A64, x, b, r, info, nb, beta)) return info;
     if (drop_worse_start(s, info, beta, nb, x, n)) {
         beta = residual_norm(s, gw, A64, x, b, r);
         if (inner_rtol_cold > 0) inner_rtol = inner_rtol_cold;  // the start is x0 = 0 after all
@@ -540,13 +535,8 @@ SolveInfo bicgstab_mixed(hipStream_t s, BicgWork<float>& w, GmresWork<float>& gw
                          float* r32, float* d32, int maxit, double tol, double inner_rtol, double restart_eps32) {
     SolveInfo info;
     w.ensure(A64.n);
-    const double nb = norm_of(s, gw, A64.n, b);
-    if (nb == 0.0) {
-        PB_HIP(hipMemsetAsync(x, 0, sizeof(double) * A64.n, s));
-        info.converged = true;
-        return info;
-    }
-    double beta = residual_norm(s, gw, A64, x, b, r);
+    double nb = 0, beta = 0;
+    if (!start_norms(s, gw, A64, x, b, r, info, nb, beta)) return info;
     if (drop_worse_start(s, info, beta, nb, x, A64.n)) beta = residual_norm(s, gw, A64, x, b, r);
     while (true) {
         info.resid = beta / nb;

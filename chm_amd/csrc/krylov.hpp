@@ -91,9 +91,9 @@ struct GmresWork {
     DevBuf<T> V, z, u;
     DevBuf<double> partial;  // kReduceBlocks * (m + 2)
     DevBuf<double> ss;       // kReduceBlocks partial sums of the new vector's norm
-    DevBuf<double> dsc;      // GmresSc, then the norm that norm_of / residual_norm report
-    HostBuf<double> hsc;     // pinned mirror of that norm
-    HostBuf<HostSlot> slot;  // reports of two Arnoldi steps in flight
+    DevBuf<double> dsc;      // GmresSc
+    HostBuf<HostSlot> slot;  // reports of two Arnoldi steps in flight, and of two norms
+    HostSlot* dslot = nullptr;  // slot in the device address space
     uint64_t seq = 0;        // number of the last report
     void ensure(int64_t n_, int m_);
 };
@@ -125,9 +125,6 @@ SolveInfo mixed_solve(hipStream_t s, GmresWork<float>& w, const CsrOp<double>& A
                       const PcFn<float>& M32, const double* b, double* x, double* r, float* r32, float* d32, int m,
                       int maxit, double tol, double inner_rtol);
 
-// device norm helpers (synchronous: return to host)
-double dev_norm2(hipStream_t s, GmresWork<double>& w, int64_t n, const double* v);
-
 // BiCGStab (van der Vorst 1992), right-preconditioned, as an alternative
 // Krylov method: two SpMV + two preconditioner applications per iteration and
 // a fixed set of vectors, so no Gram-Schmidt cost growing with the iteration.
@@ -138,16 +135,9 @@ struct BicgWork {
     DevBuf<double> partial, dsc;
     DevBuf<double> ss_partial;  // per-block s.s of k_bicg_s_dev (kept apart from the operator's dots)
     DevBuf<double> xr_partial;  // per-block (rh.r, r.r) of k_bicg_xr_dev (read by the closing stage)
-    HostBuf<double> hsc;        // two slots of the scalars (iterations k and k+1 in flight)
-    double* hsc_dev = nullptr;  // hsc in the device address space (the stage kernel writes it)
-    hipEvent_t ev[2] = {};
-    BicgWork() = default;
-    BicgWork(const BicgWork&) = delete;
-    BicgWork& operator=(const BicgWork&) = delete;
-    ~BicgWork() {
-        for (hipEvent_t e : ev)
-            if (e) (void)hipEventDestroy(e);
-    }
+    HostBuf<HostSlot> slot;     // the scalars of iterations k and k+1 in flight
+    HostSlot* dslot = nullptr;  // slot in the device address space
+    uint64_t seq = 0;           // number of the last report
     void ensure(int64_t n_);
 };
 

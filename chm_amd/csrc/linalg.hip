@@ -231,14 +231,21 @@ __global__ void __launch_bounds__(kBlock) k_mdot(int64_t n, int64_t ld, const T*
     partial[(int64_t)blockIdx.x * (nv + 1) + (t < NCH * kCols ? first + t : nv)] = sum;
 }
 
-__global__ void __launch_bounds__(kBlock) k_reduce_cols(const double* __restrict__ partial, int nblk, int stride,
-                                                        double* __restrict__ out) {
+__device__ __forceinline__ void report(HostSlot* slot, uint64_t seq) {
+    __hip_atomic_store(&slot->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// slot->v[0] = sum of nblk partial sums, in a fixed order
+__global__ void __launch_bounds__(kBlock) k_report_sum(const double* __restrict__ partial, int nblk, HostSlot* slot,
+                                                       uint64_t seq) {
     __shared__ double s_red[kBlock / 64];
-    const int c = blockIdx.x;
     double s = 0;
-    for (int b = threadIdx.x; b < nblk; b += blockDim.x) s += partial[(int64_t)b * stride + c];
+    for (int b = threadIdx.x; b < nblk; b += blockDim.x) s += partial[b];
     s = block_sum(s, s_red);
-    if (threadIdx.x == 0) out[c] = s;
+    if (threadIdx.x == 0) {
+        slot->v[0] = s;
+        report(slot, seq);
+    }
 }
 
 // Scalars of one GMRES cycle on the device (GmresSc::of lays them out).
@@ -306,7 +313,7 @@ __global__ void __launch_bounds__(kBlock) k_gmres_step(GmresSc a, const double* 
         a.scal[j + 1] = hn > 0 ? 1.0 / hn : 0.0;
         slot->v[0] = fabs(sn * gj);
         slot->v[1] = hn;
-        __hip_atomic_store(&slot->seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+        report(slot, seq);
     }
     __syncthreads();
     if (t <= j) a.H[(int64_t)j * 32 + t] = s_h[t];
@@ -410,7 +417,8 @@ __global__ void __launch_bounds__(kBlock) k_absmax(int64_t n, const double* __re
     }
 }
 
-__global__ void __launch_bounds__(kBlock) k_reduce_max(const double* __restrict__ partial, int nblk, double* out) {
+__global__ void __launch_bounds__(kBlock) k_report_max(const double* __restrict__ partial, int nblk, HostSlot* slot,
+                                                       uint64_t seq) {
     __shared__ double s_red[kBlock / 64];
     double m = 0;
     for (int b = threadIdx.x; b < nblk; b += blockDim.x) m = fmax(m, partial[b]);
@@ -422,7 +430,8 @@ __global__ void __launch_bounds__(kBlock) k_reduce_max(const double* __restrict_
     if (threadIdx.x == 0) {
         double r = 0;
         for (int k = 0; k < (int)(blockDim.x >> 6); ++k) r = fmax(r, s_red[k]);
-        *out = r;
+        slot->v[0] = r;
+        report(slot, seq);
     }
 }
 
@@ -757,7 +766,7 @@ __global__ void __launch_bounds__(kBlock) k_bicg_xr_dev(int64_t n, const T* __re
 constexpr int kStageThreads = 1024;
 __global__ void __launch_bounds__(kStageThreads) k_bicg_stage(const double* __restrict__ partial, int64_t nblk,
                                                               int stride, int stage, double* __restrict__ sc,
-                                                              double stop_abs, double* __restrict__ host_slot,
+                                                              double stop_abs, HostSlot* slot, uint64_t seq,
                                                               double restart_eps) {
     __shared__ double s_red[kStageThreads / 64];
     if (stage != 0 && sc[SC_STOP] != 0.0) return;  // uniform over the block
@@ -797,8 +806,8 @@ __global__ void __launch_bounds__(kStageThreads) k_bicg_stage(const double* __re
             sc[SC_NRESTART] += 1.0;
         }
     }
-    if (host_slot)  // the scalars straight into the host-visible slot the host waits on
-        for (int k = 0; k < SC_COUNT; ++k) host_slot[k] = sc[k];
+    for (int k = 0; k < SC_COUNT; ++k) slot->v[k] = sc[k];
+    report(slot, seq);
 }
 
 template <typename T>
@@ -878,8 +887,8 @@ void mdot(hipStream_t s, int64_t n, const T* V, int64_t ld, int nv, const T* w, 
         hipLaunchKernelGGL((k_mdot<T, 4>), dim3(nblk), dim3(kBlock), 0, s, n, ld, V, nv, w, partial, gate);
 }
 
-void reduce_cols(hipStream_t s, const double* partial, int nblk, int stride, int ncols, double* out) {
-    hipLaunchKernelGGL(k_reduce_cols, dim3(ncols), dim3(kBlock), 0, s, partial, nblk, stride, out);
+void report_sum(hipStream_t s, const double* partial, int nblk, HostSlot* slot, uint64_t seq) {
+    hipLaunchKernelGGL(k_report_sum, dim3(1), dim3(kBlock), 0, s, partial, nblk, slot, seq);
 }
 
 void gmres_start(hipStream_t s, const GmresSc& a, double beta) {
@@ -911,8 +920,8 @@ void combine(hipStream_t s, int64_t n, const T* V, int64_t ld, int nv, const dou
 void absmax(hipStream_t s, int64_t n, const double* b, double* partial, int nblk) {
     hipLaunchKernelGGL(k_absmax, dim3(nblk), dim3(kBlock), 0, s, n, b, partial);
 }
-void reduce_max(hipStream_t s, const double* partial, int nblk, double* out) {
-    hipLaunchKernelGGL(k_reduce_max, dim3(1), dim3(kBlock), 0, s, partial, nblk, out);
+void report_max(hipStream_t s, const double* partial, int nblk, HostSlot* slot, uint64_t seq) {
+    hipLaunchKernelGGL(k_report_max, dim3(1), dim3(kBlock), 0, s, partial, nblk, slot, seq);
 }
 
 template <typename T>
@@ -970,11 +979,11 @@ void bicg_xr_dev(hipStream_t s, int64_t n, const T* ph, const T* sh, const T* sv
                        dots, dots_nb, ss_part, ss_nb);
 }
 void bicg_stage(hipStream_t s, const double* partial, int64_t nblk, int stride, int stage, double* sc,
-                double stop_abs, double* host_slot, double restart_eps) {
+                double stop_abs, HostSlot* slot, uint64_t seq, double restart_eps) {
     if (stride == 2 && reinterpret_cast<uintptr_t>(partial) % 16 != 0)
         throw Error(PBSM3D_EINVAL, "dot pairs must be 16-byte aligned");
     hipLaunchKernelGGL(k_bicg_stage, dim3(1), dim3(kStageThreads), 0, s, partial, nblk, stride, stage, sc, stop_abs,
-                       host_slot, restart_eps);
+                       slot, seq, restart_eps);
 }
 
 __global__ void __launch_bounds__(kBlock) k_neumann(int64_t n, const double* v, const double* y, const double* ay,
