@@ -409,6 +409,24 @@ void bicg_xr_dev(hipStream_t s, int64_t n, const T* ph, const T* sh, const T* sv
 void bicg_stage(hipStream_t s, const double* partial, int64_t nblk, int stride, int stage, double* sc,
                 double stop_abs, HostSlot* slot, uint64_t seq, double restart_eps);
 
+// Preconditioned conjugate gradients of a symmetric positive definite system on its split operator:
+// D~^-1/2 Ahat D~^1/2 = C^-1 A C^-T with C = (D~ + L) D~^-1/2 and M = C C^T.  In the operator's own
+// variables (x^ = (D~ + U) x, r the residual D~ (D~ + L)^-1 b - Ahat x^) its inner products carry
+// the weight 1 / d~: rho = r . r / d~, p . Ahat p / d~ and p = r + beta p.  Scalars in sc[]; rho
+// alternates between two slots by the iteration's parity, so no workgroup reads one that another
+// is writing.
+enum CgSc { CG_RHO0 = 0, CG_RHO, CG_STOP = CG_RHO + 2, CG_FLAG, CG_COUNT };
+// x = 0, p = r, pw = p / d~ and rho0 (nblk partials in partial)
+void cg_start(hipStream_t s, int64_t n, const double* r, const double* dinv, double* x, double* p, double* pw,
+              double* sc, double* partial, int nblk);
+// Iteration it (from 1): alpha from the operator's pairs (pw . q, q . q), x += alpha p, r -= alpha q and
+// the partials of the new rho; then p = r + beta p, pw, and the report (rho, stop: 1 reached
+// rho <= stop2 rho0, 2 breakdown) to slot.  Both do nothing once sc[CG_STOP] is set.
+void cg_xr(hipStream_t s, int64_t n, int it, const double* p, const double* q, const double* dinv, double* x, double* r,
+           double* sc, const double* dots, int64_t dots_nb, double* partial, int nblk);
+void cg_p(hipStream_t s, int64_t n, int it, const double* r, const double* dinv, double* p, double* pw, double* sc,
+          double stop2, const double* partial, int nblk, HostSlot* slot, uint64_t seq);
+
 // conversions / vector updates
 template <typename T>
 void scale_host(hipStream_t s, int64_t n, const T* a, double alpha, T* b);  // b = alpha * a

@@ -530,6 +530,78 @@ template SolveInfo bicgstab_split<float>(hipStream_t, BicgWork<float>&, GmresWor
                                          const CsrOp<float>&, const double*, double*, double*, float*, float*, float*,
                                          int, double, double, double, const CoarseFn&, double);
 
+void CgWork::ensure(int64_t n_) {
+    if (n == n_ && p.p) return;
+    n = n_;
+    for (DevBuf<double>* v : {&rh, &p, &pw, &q, &xh}) v->alloc(n);
+    work.alloc(n + 1);
+    zero_tail(work, n);
+    dots.alloc(2 * (size_t)pos_spmv_dots_max_blocks(n));
+    partial.alloc(kVecBlocks);
+    sc.alloc(CG_COUNT);
+    slot.alloc(2);
+    slot.p[0].seq = slot.p[1].seq = seq = 0;
+    PB_HIP(hipHostGetDevicePointer((void**)&dslot, slot.p, 0));
+}
+
+SolveInfo cg_split(hipStream_t s, CgWork& w, GmresWork<double>& gw, const CsrOp<double>& A, const CsrOp<double>& Ahat,
+                   const double* b, double* x, double* r, int maxit, double tol) {
+    SolveInfo info;
+    const int64_t n = A.n;
+    w.ensure(n);
+    double nb = 0, beta = 0;
+    if (!start_norms(s, gw, A, x, b, r, info, nb, beta)) return info;
+    if (drop_worse_start(s, info, beta, nb, x, n)) beta = residual_norm(s, gw, A, x, b, r);
+    const double* dinv = Ahat.split->dinv.p;
+    double* sc = w.sc.p;
+    const int nvec = std::min(reduce_blocks(n), kVecBlocks);
+    while (true) {
+        info.resid = beta / nb;
+        if (info.resid <= tol) {
+            info.converged = true;
+            return info;
+        }
+        const int most = maxit - info.iters;
+        if (most <= 0) return info;
+        scale_host<double>(s, n, r, 1.0 / beta, w.work.p);
+        split_op<double>(1, s, *Ahat.co, Ahat.F, Ahat.L, *Ahat.split, w.work.p, w.rh.p, Ahat.mode);
+        cg_start(s, n, w.rh.p, dinv, w.xh.p, w.p.p, w.pw.p, sc, w.partial.p, nvec);
+        // sqrt(rho), the residual's norm under M^-1, stands for ||b - A x||: their reductions lie
+        // within a factor of two of each other
+        const double rel = 0.5 * tol * nb / beta, stop2 = rel * rel;
+        const uint64_t seq0 = w.seq;
+        auto iterate = [&](int it) {
+            const int64_t nd = split_apply_dots<double>(s, *Ahat.co, Ahat.F, Ahat.L, *Ahat.split, w.p.p, w.q.p, w.pw.p,
+                                                        w.dots.p, Ahat.mode, sc + CG_STOP);
+            cg_xr(s, n, it, w.p.p, w.q.p, dinv, w.xh.p, w.rh.p, sc, w.dots.p, nd, w.partial.p, nvec);
+            cg_p(s, n, it, w.rh.p, dinv, w.p.p, w.pw.p, sc, stop2, w.partial.p, nvec, w.dslot + (it & 1), ++w.seq);
+            PB_HIP(hipGetLastError());
+        };
+        double stop = 0;
+        iterate(1);
+        for (int it = 1;; ++it) {
+            if (it < most) iterate(it + 1);
+            wait_slot(s, w.slot.p + (it & 1), seq0 + it);
+            stop = w.slot.p[it & 1].v[1];
+            if (stop != 0.0 || it >= most) {
+                info.iters += it;
+                break;
+            }
+        }
+        if (stop == 2.0) return info;  // x keeps what the runs before gained
+        split_op<double>(2, s, *Ahat.co, Ahat.F, Ahat.L, *Ahat.split, w.xh.p, w.work.p, Ahat.mode);
+        axpy_f64(s, n, beta, w.work.p, x);
+        info.cycles += 1;
+        const double before = beta;
+        beta = residual_norm(s, gw, A, x, b, r);
+        if (!(beta < 0.5 * before)) {
+            info.resid = beta / nb;
+            info.converged = info.resid <= tol;
+            return info;
+        }
+    }
+}
+
 SolveInfo bicgstab_mixed(hipStream_t s, BicgWork<float>& w, GmresWork<float>& gw, const CsrOp<double>& A64,
                          const CsrOp<float>& A32, const PcFn<float>& M32, const double* b, double* x, double* r,
                          float* r32, float* d32, int maxit, double tol, double inner_rtol, double restart_eps32) {

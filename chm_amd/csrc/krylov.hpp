@@ -150,6 +150,22 @@ constexpr double kBicgRestartEps32 = 1e-5;
 
 SolveInfo bicgstab_solve(hipStream_t s, BicgWork<double>& w, GmresWork<double>& gw, const CsrOp<double>& A,
                          const PcFn<double>& M, const double* b, double* x, int maxit, double tol);
+// Conjugate gradients with the D-ILU preconditioner on its split operator, for a symmetric
+// positive definite A: one operator application per iteration (7 launches) where BiCGStab takes two (14) and
+// GMRES orthogonalises against its basis.  r receives the residual.  Not converged on a
+// breakdown (A is not positive definite) or a run that gains nothing.
+struct CgWork {
+    int64_t n = 0;
+    DevBuf<double> rh, p, pw, q, xh, work;  // work: n + 1 entries, entry n zero
+    DevBuf<double> dots, partial, sc;
+    HostBuf<HostSlot> slot;
+    HostSlot* dslot = nullptr;
+    uint64_t seq = 0;
+    void ensure(int64_t n_);
+};
+SolveInfo cg_split(hipStream_t s, CgWork& w, GmresWork<double>& gw, const CsrOp<double>& A, const CsrOp<double>& Ahat,
+                   const double* b, double* x, double* r, int maxit, double tol);
+
 // BiCGStab on the split-preconditioned system (Eisenstat's trick) inside FP64
 // iterative refinement: each cycle takes the FP64 residual r = b - A64 x,
 // transforms r / ||r|| with Ahat's left factor, runs unpreconditioned BiCGStab on

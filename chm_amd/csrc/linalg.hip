@@ -810,6 +810,90 @@ __global__ void __launch_bounds__(kStageThreads) k_bicg_stage(const double* __re
     report(slot, seq);
 }
 
+__global__ void __launch_bounds__(kBlock) k_cg_start(int64_t n, const double* __restrict__ r,
+                                                     const double* __restrict__ dinv, double* __restrict__ x,
+                                                     double* __restrict__ p, double* __restrict__ pw,
+                                                     double* __restrict__ partial) {
+    __shared__ double s_red[kBlock / 64];
+    double acc = 0;
+    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+    for (int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; k < n; k += stride) {
+        const double z = r[k], zw = z * dinv[k];
+        x[k] = 0;
+        p[k] = z;
+        pw[k] = zw;
+        acc = fma(z, zw, acc);
+    }
+    const double sum = block_sum(acc, s_red);
+    if (threadIdx.x == 0) partial[blockIdx.x] = sum;
+}
+__global__ void __launch_bounds__(kBlock) k_cg_rho0(const double* __restrict__ partial, int nblk,
+                                                    double* __restrict__ sc) {
+    __shared__ double s_red[kBlock / 64];
+    const double rho = sum_partials(partial, nblk, 1, 0, s_red);
+    if (threadIdx.x != 0) return;
+    sc[CG_RHO0] = sc[CG_RHO] = rho;
+    sc[CG_STOP] = sc[CG_FLAG] = 0;
+}
+
+__global__ void __launch_bounds__(kBlock) k_cg_xr(int64_t n, int it, const double* __restrict__ p,
+                                                  const double* __restrict__ q, const double* __restrict__ dinv,
+                                                  double* __restrict__ x, double* __restrict__ r,
+                                                  double* __restrict__ sc, const double* __restrict__ dots,
+                                                  int64_t dots_nb, double* __restrict__ partial) {
+    __shared__ double s_red[kBlock / 64], s_alpha;
+    if (sc[CG_STOP] != 0.0) return;  // uniform over the grid
+    const double pq = sum_partials(dots, dots_nb, 2, 0, s_red);
+    if (threadIdx.x == 0) {
+        const bool ok = pq > 0.0 && isfinite(pq);  // else the system is not positive definite
+        s_alpha = ok ? sc[CG_RHO + ((it - 1) & 1)] / pq : 0.0;
+        if (!ok && blockIdx.x == 0) sc[CG_FLAG] = 1;
+    }
+    __syncthreads();
+    const double alpha = s_alpha;
+    double acc = 0;
+    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+    for (int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; k < n; k += stride) {
+        x[k] = fma(alpha, p[k], x[k]);
+        const double rk = fma(-alpha, q[k], r[k]);
+        r[k] = rk;
+        acc = fma(rk, rk * dinv[k], acc);
+    }
+    const double sum = block_sum(acc, s_red);
+    if (threadIdx.x == 0) partial[blockIdx.x] = sum;
+}
+
+__global__ void __launch_bounds__(kBlock) k_cg_p(int64_t n, int it, const double* __restrict__ r,
+                                                 const double* __restrict__ dinv, double* __restrict__ p,
+                                                 double* __restrict__ pw, double* __restrict__ sc, double stop2,
+                                                 const double* __restrict__ partial, int nblk, HostSlot* slot,
+                                                 uint64_t seq) {
+    __shared__ double s_red[kBlock / 64], s_beta;
+    // workgroup 0 sets the stop below: one that starts later may skip its part of a p that no
+    // later launch reads
+    if (sc[CG_STOP] != 0.0) return;
+    const double rho = sum_partials(partial, nblk, 1, 0, s_red);
+    if (threadIdx.x == 0) {
+        s_beta = rho / sc[CG_RHO + ((it - 1) & 1)];
+        if (blockIdx.x == 0) {
+            sc[CG_RHO + (it & 1)] = rho;
+            const double stop = sc[CG_FLAG] != 0.0 || !isfinite(rho) ? 2.0 : rho <= stop2 * sc[CG_RHO0] ? 1.0 : 0.0;
+            sc[CG_STOP] = stop;
+            slot->v[0] = rho;
+            slot->v[1] = stop;
+            report(slot, seq);
+        }
+    }
+    __syncthreads();
+    const double beta = s_beta;
+    const int64_t stride = (int64_t)gridDim.x * blockDim.x;
+    for (int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; k < n; k += stride) {
+        const double pk = fma(beta, p[k], r[k]);
+        p[k] = pk;
+        pw[k] = pk * dinv[k];
+    }
+}
+
 template <typename T>
 __global__ void k_scale_host(int64_t n, const T* a, double alpha, T* b) {
     const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -984,6 +1068,21 @@ void bicg_stage(hipStream_t s, const double* partial, int64_t nblk, int stride, 
         throw Error(PBSM3D_EINVAL, "dot pairs must be 16-byte aligned");
     hipLaunchKernelGGL(k_bicg_stage, dim3(1), dim3(kStageThreads), 0, s, partial, nblk, stride, stage, sc, stop_abs,
                        slot, seq, restart_eps);
+}
+
+void cg_start(hipStream_t s, int64_t n, const double* r, const double* dinv, double* x, double* p, double* pw,
+              double* sc, double* partial, int nblk) {
+    hipLaunchKernelGGL(k_cg_start, dim3(nblk), dim3(kBlock), 0, s, n, r, dinv, x, p, pw, partial);
+    hipLaunchKernelGGL(k_cg_rho0, dim3(1), dim3(kBlock), 0, s, partial, nblk, sc);
+}
+void cg_xr(hipStream_t s, int64_t n, int it, const double* p, const double* q, const double* dinv, double* x, double* r,
+           double* sc, const double* dots, int64_t dots_nb, double* partial, int nblk) {
+    hipLaunchKernelGGL(k_cg_xr, dim3(nblk), dim3(kBlock), 0, s, n, it, p, q, dinv, x, r, sc, dots, dots_nb, partial);
+}
+void cg_p(hipStream_t s, int64_t n, int it, const double* r, const double* dinv, double* p, double* pw, double* sc,
+          double stop2, const double* partial, int nblk, HostSlot* slot, uint64_t seq) {
+    hipLaunchKernelGGL(k_cg_p, dim3(nblk), dim3(kBlock), 0, s, n, it, r, dinv, p, pw, sc, stop2, partial, nblk, slot,
+                       seq);
 }
 
 __global__ void __launch_bounds__(kBlock) k_neumann(int64_t n, const double* v, const double* y, const double* ay,

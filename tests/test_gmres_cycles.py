@@ -66,3 +66,31 @@ def test_second_orthogonalisation_pass():
         ctx.close()
     for k in ("conc", "qdep"):
         assert rel_err(out[0][k], out[1][k]) < 1e-8
+
+
+@pytest.mark.parametrize("points,layers", [(12, 2), (40, 3), (300, 5), (2501, 5), (20011, 5)])
+@pytest.mark.parametrize("smooth", [0.0, 820.0, -2.0e3])
+def test_deposition_cg_and_its_fallback(points, layers, smooth):
+    """The deposition system by conjugate gradients against GMRES with the Jacobi preconditioner, both to
+    1e-12: the default smoothing, none (a diagonal system), and a negative coefficient, whose
+    indefinite system either goes to GMRES or is refused by both."""
+    from chm_amd import pbsm3d as pb
+
+    print(f"[case] deposition cg points={points} smooth={smooth}", flush=True)
+    mesh = meshgen.synthetic_mesh(points, seed=8, extent=1.0e3 if smooth < 0 else 1.0e4)
+    g = pb.face_geometry(mesh)
+    fo = meshgen.forcing_c2(mesh.n_faces, seed=4)
+    res = []
+    for pc in (abi.PC_MCILU0, abi.PC_JACOBI):
+        ctx = pb.Context(g, pb.default_config(nLayer=layers, tol=1e-12, dep_precond=pc, smooth_coeff=smooth,
+                                              max_iters=600))
+        try:
+            o, st = ctx.step(fo, want_fields=True)
+            assert st["dep_resid"] <= 1e-12
+            res.append(o["qdep"])
+        except pb.Pbsm3dError as e:
+            assert smooth < 0 and e.code == abi.PBSM3D_ENOCONV
+        ctx.close()
+    assert len(res) == 2 or smooth < 0
+    if len(res) == 2 and smooth >= 0:
+        assert rel_err(res[0], res[1]) < 1e-8
