@@ -283,41 +283,45 @@ static double split_inner_rtol_default(const pbsm3d_ctx* c, const pbsm3d_config&
     return cfg.warm_start == PBSM3D_WS_LEARNED && c->warm != nullptr ? kSplitInnerLearned : kSplitInnerCold;
 }
 
-// The later GMRES cycles' operator and work vectors, laid out when a solve first gets there (degree
-// 0: no memory for them, the cycles stay plain).
-// The degree trades operator applications (a longer polynomial overshoots the target by more)
-// against basis traffic, which is cheap while the basis is cached.  Suspension solve, mean of five
-// forcings, ms: 999,968 faces x 10 layers, degree 6 75, 8 74, 10 62, 12 64, 16 64; 240,000 x 9 8.1,
-// 8.1, 8.0, 8.5, 8.8; after a plain cycle, 50,000 x 10, degree 3 3.78, 4 3.83, 6 3.93, 8 3.99.
-constexpr int kNeumannLarge = 10, kNeumannCached = 4;
+// The Neumann polynomial's degree trades operator applications (a longer one overshoots the target
+// by more) against basis traffic and launches.  Suspension solve, GMRES(30), mean of three to five
+// forcings, ms: 999,968 faces x 10 layers, degree 6 75, 8 74, 10 62, 12 64, 16 64; 240,000 x 10 4 8.8,
+// 6 8.1, 10 8.3; 200,000 x 9 1 10.5, 2 7.8, 4 6.3, 6 6.1; 125,000 x 7 1 4.54, 2 3.53, 4 2.98, 6 2.98;
+// 50,000 x 10 1 3.12, 2 2.40, 4 2.25, 6 2.29; 5,000 x 5 1 0.82, 2 0.73, 4 0.77 -- in a system that
+// small the launches are the bound, and degree 1 keeps GMRES's own iteration count.
+static int neumann_degree(int64_t N) {
+    if (N < 100000) return 1;
+    return N * (int64_t)sizeof(double) > kCachedVector ? 10 : 4;
+}
 static bool split_fits(int64_t F, int L) {  // what split_op takes
     return L <= 16 && (uint64_t)3 * (uint64_t)F * (uint64_t)L + 1 < (1ull << 32);
 }
-static std::function<SplitCycles()> later_cycles(pbsm3d_ctx* c) {
-    return [c]() -> SplitCycles {
-        const int64_t N = c->F * c->L;
-        try {
-            for (DevBuf<double>& b : c->split64)
-                if (!b.p) {
-                    b.alloc(N + 1);
-                    zero_tail(b, N);
-                }
-        } catch (const Error& e) {
-            if (e.code != PBSM3D_ENOMEM) throw;
-            (void)hipGetLastError();
-            return SplitCycles{};
-        }
-        if (c->split_mode < 0)
-            c->split_mode = tune_split_mode<double>(c->stream, c->co, c->F, c->L, c->dl_s, c->bp.p, c->split64[0].p,
-                                                    nullptr);
-        SplitCycles sp{CsrOp<double>{N, nullptr, nullptr, nullptr, &c->prof, c->F, c->L}, {},
-                       N * (int64_t)sizeof(double) > kCachedVector ? kNeumannLarge : kNeumannCached};
-        sp.Ahat.co = &c->co;
-        sp.Ahat.split = &c->dl_s;
-        sp.Ahat.mode = c->split_mode;
-        for (int k = 0; k < 3; ++k) sp.work[k] = c->split64[k].p;
-        return sp;
-    };
+// GMRES's split operator and work vectors, laid out at the first solve; nothing (plain cycles)
+// where it does not fit or there is no memory for them.
+static SplitCycles split_cycles(pbsm3d_ctx* c) {
+    const int64_t N = c->F * c->L;
+    if (!split_fits(c->F, c->L)) return SplitCycles{};
+    try {
+        for (DevBuf<double>& b : c->split64)
+            if (!b.p) {
+                b.alloc(N + 1);
+                zero_tail(b, N);
+            }
+    } catch (const Error& e) {
+        if (e.code != PBSM3D_ENOMEM) throw;
+        (void)hipGetLastError();
+        return SplitCycles{};
+    }
+    if (c->split_mode < 0)
+        c->split_mode =
+            tune_split_mode<double>(c->stream, c->co, c->F, c->L, c->dl_s, c->bp.p, c->split64[0].p, nullptr);
+    SplitCycles sp{CsrOp<double>{N, nullptr, nullptr, nullptr, &c->prof, c->F, c->L}, {}, neumann_degree(N)};
+    sp.Ahat.co = &c->co;
+    sp.Ahat.split = &c->dl_s;
+    sp.Ahat.mode = c->split_mode;
+    sp.Ahat.prof_class = PBSM3D_K_PRECOND;
+    for (int k = 0; k < 3; ++k) sp.work[k] = c->split64[k].p;
+    return sp;
 }
 
 // Suspension solve with the multicolour D-ILU(0) preconditioner, carried out in
@@ -397,7 +401,7 @@ SolveInfo solve_in_position_order(pbsm3d_ctx* c, const pbsm3d_config& cfg, int64
             si = bicgstab_solve(s, c->bw64, c->ws64, A, M, c->bp.p, c->xp.p, cfg.max_iters, cfg.tol);
         else
             si = gmres_solve(s, c->ws64, A, M, c->bp.p, c->xp.p, c->r_s.p, cfg.restart, cfg.max_iters, cfg.tol,
-                             split_fits(F, L) ? later_cycles(c) : nullptr);
+                             split_cycles(c));
     } else {
         CsrOp<float> A32{N, nullptr, nullptr, nullptr, &c->prof, F, L};
         A32.co = &c->co;

@@ -90,13 +90,14 @@ int gmres_cycle(hipStream_t s, GmresWork<T>& w, const CsrOp<T>& A, const PcFn<T>
     auto queue = [&](int j) {
         T* vj = V + (size_t)j * ld;
         T* vj1 = V + (size_t)(j + 1) * ld;
-        {
+        if (M) {
             ProfScope ps(A.prof, s, PBSM3D_K_PRECOND);
             M(s, vj, w.z.p);
         }
         {
-            ProfScope ps(A.prof, s, sizeof(T) == 8 ? PBSM3D_K_SPMV64 : PBSM3D_K_SPMV32);
-            op_spmv<T>(s, A, w.z.p, vj1);
+            ProfScope ps(A.prof, s,
+                         A.prof_class >= 0 ? A.prof_class : sizeof(T) == 8 ? PBSM3D_K_SPMV64 : PBSM3D_K_SPMV32);
+            op_spmv<T>(s, A, M ? w.z.p : vj, vj1);
         }
         ProfScope ps(A.prof, s, PBSM3D_K_ORTHO);
         mdot<T>(s, n, V, ld, j + 1, vj1, w.partial.p, nblk);
@@ -125,8 +126,8 @@ int gmres_cycle(hipStream_t s, GmresWork<T>& w, const CsrOp<T>& A, const PcFn<T>
         if (res <= stop_abs || sl.v[1] == 0.0) break;
     }
     gmres_y(s, sc, known);
-    combine<T>(s, n, V, ld, known, sc.coef, w.u.p);
-    {
+    combine<T>(s, n, V, ld, known, sc.coef, M ? w.u.p : out);
+    if (M) {
         ProfScope ps(A.prof, s, PBSM3D_K_PRECOND);
         M(s, w.u.p, out);
     }
@@ -213,15 +214,17 @@ int split_cycle(hipStream_t s, GmresWork<double>& w, const SplitCycles& sp, cons
     split_op<double>(1, s, *A.co, A.F, A.L, *A.split, r1, rh, A.mode);
     const double bh = norm_of(s, w, n, rh);
     if (!(bh > 0)) return 0;
-    const PcFn<double> q = [&](hipStream_t st, const double* v, double* z) {
-        // Horner: z = v, then z <- v + z - Ahat z
-        const double* from = v;
-        for (int k = 1; k < sp.degree; ++k) {
-            op_spmv<double>(st, A, from, y);
-            neumann_step(st, n, v, from, y, z);
-            from = z;
-        }
-    };
+    PcFn<double> q;  // degree 1: q = 1
+    if (sp.degree > 1)
+        q = [&](hipStream_t st, const double* v, double* z) {
+            // Horner: z = v, then z <- v + z - Ahat z
+            const double* from = v;
+            for (int k = 1; k < sp.degree; ++k) {
+                op_spmv<double>(st, A, from, y);
+                neumann_step(st, n, v, from, y, z);
+                from = z;
+            }
+        };
     double est = 0;
     const int steps = gmres_cycle<double>(s, w, A, q, rh, bh, stop_rel * bh, max_steps, r1, &est);
     if (!std::isfinite(est)) return 0;
@@ -232,22 +235,17 @@ int split_cycle(hipStream_t s, GmresWork<double>& w, const SplitCycles& sp, cons
 }  // namespace
 
 SolveInfo gmres_solve(hipStream_t s, GmresWork<double>& w, const CsrOp<double>& A, const PcFn<double>& M,
-                      const double* b, double* x, double* r, int m, int maxit, double tol,
-                      const std::function<SplitCycles()>& later) {
+                      const double* b, double* x, double* r, int m, int maxit, double tol, SplitCycles split) {
     SolveInfo info;
     w.ensure(A.n, m);
     double nb = 0, beta = 0;
     if (!start_norms(s, w, A, x, b, r, info, nb, beta)) return info;
     if (drop_worse_start(s, info, beta, nb, x, A.n)) beta = residual_norm(s, w, A, x, b, r);
-    // The split cycles take `degree` operator applications per basis vector, so a cycle reaches
-    // degree times as far for the same basis traffic, and restarts forget the slow modes that much
-    // less often.  They are for systems whose basis does not stay in the caches (kCachedVector),
-    // and for those that two plain cycles do not solve; one that needs part of a second cycle gains
-    // nothing (50,000 faces x 10 layers, 34 to 49 steps: 4.6 ms a step plain, 4.7 with).
-    // Suspension solve, GMRES(30), 999,968 faces x 10 layers, mean of five forcings: 171 ms plain
-    // (three of them), 87 with one plain cycle first, 62 without; 240,000 x 9: 12.4 and 8.0.
-    bool split = static_cast<bool>(later);
-    const bool large = A.n * (int64_t)sizeof(double) > kCachedVector;
+    // The split cycles need no SpMV, and take `degree` operator applications per basis vector: a
+    // cycle reaches degree times as far for the same basis traffic, and restarts forget the slow
+    // modes that much less often.  Suspension solve, GMRES(30), mean of three to five forcings, ms, plain
+    // against split: 5,000 faces x 5 layers 1.05 and 0.82, 50,000 x 10 3.95 and 2.25, 125,000 x 7 5.30
+    // and 2.98, 200,000 x 9 11.6 and 6.3, 999,968 x 10 171 and 62.
     while (true) {
         info.resid = beta / nb;
         if (info.resid <= tol) {
@@ -256,14 +254,13 @@ SolveInfo gmres_solve(hipStream_t s, GmresWork<double>& w, const CsrOp<double>& 
         }
         if (info.iters >= maxit) break;
         int steps = 0;
-        if (split && (large || info.cycles > 1)) {
-            const SplitCycles sp = later();
-            split = sp.degree > 1;
-            const int most = split ? (maxit - info.iters) / sp.degree : 0;
-            if (most > 0) steps = split_cycle(s, w, sp, r, beta, 0.5 * tol * nb / beta, most, x);
+        if (split.degree > 0) {
+            const int most = (maxit - info.iters) / split.degree;
+            // the split residual's norm stands for ||b - A x||; their reductions lie close together
+            if (most > 0) steps = split_cycle(s, w, split, r, beta, 0.8 * tol * nb / beta, most, x);
         }
-        const bool polynomial = steps > 0;
-        if (!polynomial) {
+        const bool plain = steps == 0;
+        if (plain) {
             double est = 0;
             steps = gmres_cycle<double>(s, w, A, M, r, beta, tol * nb, maxit - info.iters, r, &est);
             axpy_f64(s, A.n, 1.0, r, x);
@@ -272,8 +269,8 @@ SolveInfo gmres_solve(hipStream_t s, GmresWork<double>& w, const CsrOp<double>& 
         info.cycles += 1;
         const double before = beta;
         beta = residual_norm(s, w, A, x, b, r);
-        // a spectrum the polynomial does not suit: back to plain cycles
-        if (polynomial && !(beta < 0.5 * before)) split = false;
+        // a spectrum the polynomial does not suit: plain cycles from here
+        if (!plain && !(beta < 0.5 * before)) split.degree = 0;
     }
     return info;
 }

@@ -105,9 +105,8 @@ template <typename T>
 int gmres_cycle(hipStream_t s, GmresWork<T>& w, const CsrOp<T>& A, const PcFn<T>& M, const T* r0, double beta,
                 double stop_abs, int max_steps, T* x_update, double* resid_est);
 
-// What the restart cycles of gmres_solve after the first one run on, where the split operator is
-// available: Ahat (.split set) preconditioned by the Neumann polynomial
-// q(Ahat) = sum_{k < degree} (I - Ahat)^k.
+// What gmres_solve's cycles run on where the split operator is available: Ahat (.split set)
+// preconditioned by the Neumann polynomial q(Ahat) = sum_{k < degree} (I - Ahat)^k.
 struct SplitCycles {
     CsrOp<double> Ahat;
     double* work[3] = {};  // N + 1 entries each, entry N zero
@@ -115,10 +114,10 @@ struct SplitCycles {
 };
 
 // Full FP64 restarted GMRES: x holds the initial guess on entry.  iters counts the applications
-// of the preconditioned operator (one per step, degree per step of a later cycle).
+// of the preconditioned operator (one per step of a plain cycle, degree per step of a split one).
 SolveInfo gmres_solve(hipStream_t s, GmresWork<double>& w, const CsrOp<double>& A, const PcFn<double>& M,
                       const double* b, double* x, double* r, int m, int maxit, double tol,
-                      const std::function<SplitCycles()>& later = nullptr);
+                      SplitCycles split = SplitCycles());
 
 // FP64 iterative refinement around FP32 GMRES cycles.
 SolveInfo mixed_solve(hipStream_t s, GmresWork<float>& w, const CsrOp<double>& A64, const CsrOp<float>& A32,

@@ -1,6 +1,6 @@
-"""FP64 GMRES beyond one plain cycle: the cycles on the split operator with the Neumann
-polynomial (from the third cycle of a small system, every cycle of a large one), the plain restarts
-where the split operator is not available, and the iteration limit inside them."""
+"""FP64 GMRES: the cycles on the split operator with each degree of the Neumann polynomial, the
+plain cycles where the split operator is not available, the iteration limit inside both, and
+the conjugate gradients of the deposition system."""
 import numpy as np
 import pytest
 
@@ -12,7 +12,8 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("points,layers,restart", [
     (13, 2, 1), (13, 5, 3), (300, 5, 3), (300, 16, 4), (300, 17, 4), (2500, 10, 6), (2501, 7, 31),
-    (106000, 10, 30)])  # the last: a basis vector of more than 16 MB
+    (300, 20, 30), (6000, 9, 30), (6000, 9, 4),  # 100,000 rows and more: degree 4
+    (106000, 10, 30)])  # a basis vector of more than 16 MB: degree 10
 def test_restarted_gmres_solves_the_same_system(points, layers, restart):
     """Both solve to 1e-12, so their fields differ by the forward error of that tolerance alone."""
     from chm_amd import pbsm3d as pb
@@ -34,15 +35,16 @@ def test_restarted_gmres_solves_the_same_system(points, layers, restart):
     ref.close()
 
 
-def test_iteration_limit_inside_the_later_cycles():
+@pytest.mark.parametrize("points,layers", [(2500, 10), (6000, 9), (300, 17)])
+def test_iteration_limit_inside_a_cycle(points, layers):
     from chm_amd import pbsm3d as pb
 
-    print("[case] gmres cycles iteration limit", flush=True)
-    mesh = meshgen.synthetic_mesh(2500, seed=0)
+    print(f"[case] gmres iteration limit points={points} L={layers}", flush=True)
+    mesh = meshgen.synthetic_mesh(points, seed=0)
     g = pb.face_geometry(mesh)
     fo = meshgen.forcing_c2(mesh.n_faces, seed=9)
-    for limit in (8, 9, 11, 13):  # two plain cycles take 8; what is left is 0, 1, 3 and 5
-        ctx = pb.Context(g, pb.default_config(nLayer=10, restart=4, max_iters=limit))
+    for limit in (1, 3, 4, 5, 7):  # less than, exactly and more than one step of degree 4
+        ctx = pb.Context(g, pb.default_config(nLayer=layers, restart=2, max_iters=limit))
         with pytest.raises(pb.Pbsm3dError) as e:
             ctx.step(fo)
         assert e.value.code == abi.PBSM3D_ENOCONV
