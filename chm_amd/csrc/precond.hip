@@ -19,6 +19,7 @@
 // gathers r and scatters z once each.  The same kernels serve the 2-D
 // deposition system (one layer).
 #include <algorithm>
+#include <type_traits>
 #include <vector>
 
 #include "kernels.hpp"
@@ -1236,51 +1237,66 @@ int64_t split_apply_t(hipStream_t s, const ColorOrder& co, int64_t F, int L, Dil
     }
     return nb;
 }
-template <typename T, int LM, bool XCD, bool NT>
+template <typename T, int LM, bool EX, bool XCD, bool NT>
 void split_lsolve_t(hipStream_t s, const ColorOrder& co, int64_t F, int L, DiluFactors<T>& d, const T* b, T* bhat) {
     for (int c = 0; c < co.ncolor; ++c) {
         if (co.off[c + 1] == co.off[c]) continue;
         const dim3 g((unsigned)launch_blocks<XCD>(col_blocks(co.off[c], co.off[c + 1])));
-        hipLaunchKernelGGL((k_eis_fwd<T, LM, false, XCD, false, false, false, NT>), g, dim3(kBlock), 0, s, F, L, co.off[c],
+        hipLaunchKernelGGL((k_eis_fwd<T, LM, EX, XCD, false, false, false, NT>), g, dim3(kBlock), 0, s, F, L, co.off[c],
                            co.off[c + 1], co.nbp.p, co.lowmask.p, d.lat.p, d.vert.p, d.dinv.p, d.E.p, b, d.t.p,
                            d.t.p, d.y.p, d.y.p, bhat, (const T*)nullptr, (double*)nullptr, (const double*)nullptr);
     }
 }
-template <typename T, int LM, bool XCD, bool NT>
+template <typename T, int LM, bool EX, bool XCD, bool NT>
 void split_rsolve_t(hipStream_t s, const ColorOrder& co, int64_t F, int L, DiluFactors<T>& d, const T* xhat, T* x) {
     for (int c = co.ncolor - 1; c >= 0; --c) {
         if (co.off[c + 1] == co.off[c]) continue;
         const dim3 g((unsigned)launch_blocks<XCD>(col_blocks(co.off[c], co.off[c + 1])));
-        hipLaunchKernelGGL((k_eis_bwd<T, LM, false, XCD, NT>), g, dim3(kBlock), 0, s, F, L, co.off[c], co.off[c + 1],
+        hipLaunchKernelGGL((k_eis_bwd<T, LM, EX, XCD, NT>), g, dim3(kBlock), 0, s, F, L, co.off[c], co.off[c + 1],
                            co.nbp.p, co.lowmask.p, d.lat.p, d.vert.p, d.dinv.p, xhat, x, x, (const double*)nullptr);
     }
+}
+// Calls fn with the unroll bound of the split sweeps for L layers and whether L is that bound: then the
+// unrolled column has no guards and all its loads are in flight before the first wait.  Every
+// common layer count is exact: a split BiCGStab iteration at 125,000 faces x 7 layers took 108 us
+// with guards (bound 10) and takes 87, at 240,000 x 8 128 and 108, at 500,000 x 9 214 and 205.
+template <typename Fn>
+void with_layers(int L, Fn&& fn) {
+    using std::integral_constant;
+    using Yes = integral_constant<bool, true>;
+    using No = integral_constant<bool, false>;
+    switch (L) {
+        case 1: return fn(integral_constant<int, 1>(), Yes());
+        case 5: return fn(integral_constant<int, 5>(), Yes());
+        case 6: return fn(integral_constant<int, 6>(), Yes());
+        case 7: return fn(integral_constant<int, 7>(), Yes());
+        case 8: return fn(integral_constant<int, 8>(), Yes());
+        case 9: return fn(integral_constant<int, 9>(), Yes());
+        case 10: return fn(integral_constant<int, 10>(), Yes());
+        case 16: return fn(integral_constant<int, 16>(), Yes());
+        default: break;
+    }
+    if (L < 1 || L > 16) throw Error(PBSM3D_EINVAL, "the split D-ILU operator needs nLayer <= 16");
+    if (L < 5)
+        fn(integral_constant<int, 5>(), No());
+    else
+        fn(integral_constant<int, 16>(), No());
 }
 // which: 0 apply, 1 left transform, 2 right transform
 template <typename T, bool XCD, bool NT>
 int64_t split_dispatch(int which, hipStream_t s, const ColorOrder& co, int64_t F, int L, DiluFactors<T>& d,
                        const T* in, T* out, const T* dw, double* partial, const double* stop) {
     int64_t nb = 0;
-#define PB_SPLIT(LMV)                                                           \
-    {                                                                           \
-        if (which == 0)                                                         \
-            nb = L == LMV ? split_apply_t<T, LMV, true, XCD, NT>(s, co, F, L, d, in, out, dw, partial, stop) \
-                          : split_apply_t<T, LMV, false, XCD, NT>(s, co, F, L, d, in, out, dw, partial, stop); \
-        else if (which == 1)                                                    \
-            split_lsolve_t<T, LMV, XCD, NT>(s, co, F, L, d, in, out);           \
-        else                                                                    \
-            split_rsolve_t<T, LMV, XCD, NT>(s, co, F, L, d, in, out);           \
-    }
-    if (L <= 1)
-        PB_SPLIT(1)
-    else if (L <= 5)
-        PB_SPLIT(5)
-    else if (L <= 10)
-        PB_SPLIT(10)
-    else if (L <= 16)
-        PB_SPLIT(16)
-    else
-        throw Error(PBSM3D_EINVAL, "the split D-ILU operator needs nLayer <= 16");
-#undef PB_SPLIT
+    with_layers(L, [&](auto lm, auto ex) {
+        constexpr int LM = decltype(lm)::value;
+        constexpr bool EX = decltype(ex)::value;
+        if (which == 0)
+            nb = split_apply_t<T, LM, EX, XCD, NT>(s, co, F, L, d, in, out, dw, partial, stop);
+        else if (which == 1)
+            split_lsolve_t<T, LM, EX, XCD, NT>(s, co, F, L, d, in, out);
+        else
+            split_rsolve_t<T, LM, EX, XCD, NT>(s, co, F, L, d, in, out);
+    });
     return nb;
 }
 }  // namespace
@@ -1411,24 +1427,10 @@ void split_apply_batch(hipStream_t s, const ColorOrder& co, int64_t F, int L, Di
                        const T* in, T* out, const T* dw, double* partial, const double* stop, int stop_stride) {
     if (co.ncolor > kMaxColors) throw Error(PBSM3D_EINVAL, "too many colours for the batch tables");
     check_split_size(F, L);
-#define PB_BATCH(LMV)                                                                                   \
-    {                                                                                                   \
-        if (L == LMV)                                                                                   \
-            split_apply_batch_t<T, LMV, true>(s, co, F, L, d, st, in, out, dw, partial, stop, stop_stride); \
-        else                                                                                            \
-            split_apply_batch_t<T, LMV, false>(s, co, F, L, d, st, in, out, dw, partial, stop, stop_stride); \
-    }
-    if (L <= 1)
-        PB_BATCH(1)
-    else if (L <= 5)
-        PB_BATCH(5)
-    else if (L <= 10)
-        PB_BATCH(10)
-    else if (L <= 16)
-        PB_BATCH(16)
-    else
-        throw Error(PBSM3D_EINVAL, "the split D-ILU operator needs nLayer <= 16");
-#undef PB_BATCH
+    with_layers(L, [&](auto lm, auto ex) {
+        split_apply_batch_t<T, decltype(lm)::value, decltype(ex)::value>(s, co, F, L, d, st, in, out, dw, partial, stop,
+                                                                         stop_stride);
+    });
     PB_HIP(hipGetLastError());
 }
 
