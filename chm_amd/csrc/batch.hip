@@ -63,6 +63,72 @@ __global__ void __launch_bounds__(kBlock) k_seg_dots2(const int4* __restrict__ c
     }
 }
 
+__device__ __forceinline__ double stage_sum(double v, double* red, double* bc) {
+    const double s = block_sum(v, red);
+    if (threadIdx.x == 0) *bc = s;
+    __syncthreads();
+    const double r = *bc;
+    __syncthreads();
+    return r;
+}
+
+// alpha = rho / rh.v of a member from its ranges rg of the first operator application's pairs;
+// record: the member's scalars are written (one workgroup per member does)
+__device__ __forceinline__ double seg_alpha(double* S, const int64_t* rg, const double* pairs, double* red, double* bc,
+                                            bool record) {
+    double a = 0;
+    for (int c = 0; c < kMaxColors; ++c)
+        for (int64_t k = rg[2 * c] + threadIdx.x; k < rg[2 * c + 1]; k += kStage) a += pairs[2 * k];
+    a = stage_sum(a, red, bc);
+    const bool ok = a != 0.0 && isfinite(a);
+    const double alpha = ok ? S[BS_RHO] / a : 0.0;
+    if (record && threadIdx.x == 0) {
+        S[BS_RHV] = a;
+        S[BS_ALPHA] = alpha;
+        if (!ok) S[BS_FLAG] = 1;  // breakdown: the member stops at the end of the iteration
+    }
+    return alpha;
+}
+// omega from the second application's pairs (s.t, t.t) and the member's partials of s.s: the minimal
+// residual's, enlarged when |cos(t, s)| < 0.7 (as the single solve)
+__device__ __forceinline__ double seg_omega(double* S, const int64_t* rg, const double* pairs, int64_t c0, int64_t c1,
+                                            const double* ssp, double* red, double* bc, bool record) {
+    double st = 0, tt = 0, ss = 0;
+    for (int c = 0; c < kMaxColors; ++c)
+        for (int64_t k = rg[2 * c] + threadIdx.x; k < rg[2 * c + 1]; k += kStage) {
+            st += pairs[2 * k];
+            tt += pairs[2 * k + 1];
+        }
+    st = stage_sum(st, red, bc);
+    tt = stage_sum(tt, red, bc);
+    for (int64_t k = c0 + threadIdx.x; k < c1; k += kStage) ss += ssp[k];
+    ss = stage_sum(ss, red, bc);
+    double omega = 0;
+    int flag = 0;
+    if (tt > 0.0 && isfinite(st) && isfinite(tt)) {
+        omega = st / tt;
+        const double cs = st / sqrt(tt * ss);
+        if (isfinite(cs) && fabs(cs) < 0.7 && fabs(cs) > 0.0) omega *= 0.7 / fabs(cs);
+        if (omega == 0.0) flag = -2;
+    } else {
+        flag = 2;
+    }
+    if (record && threadIdx.x == 0) {
+        S[BS_ST] = st;
+        S[BS_TT] = tt;
+        S[BS_SS] = ss;
+        S[BS_OMEGA] = omega;
+        if (flag == 2 || (flag == -2 && S[BS_FLAG] == 0.0)) S[BS_FLAG] = 2;
+    }
+    return omega;
+}
+// Operator pairs of the largest member up to which the s and x/r kernels form alpha and omega
+// themselves, every workgroup alike (the sums are the stage launches', bit for bit): two launches
+// of 3.6 us less per iteration of 16.  A larger member's pairs would be read once per kChunk
+// elements of it.
+constexpr int64_t kFoldPairs = 512;
+static_assert(kBlock == kStage, "the folded sums run on the element-wise kernels' workgroups");
+
 // p = r + beta (p - omega v), beta = (rho / rho_prev) (alpha / omega) of the member; after a
 // restart of the member's shadow residual, p = r and rh = r
 template <typename T>
@@ -82,16 +148,21 @@ __global__ void __launch_bounds__(kBlock) k_seg_p(const int4* __restrict__ ch, c
         p[q] = (T)fma(beta, fma(-omega, (double)v[q], (double)p[q]), (double)r[q]);
 }
 
-// s = r - alpha v; partial[chunk] = s.s
-template <typename T>
+// s = r - alpha v; partial[chunk] = s.s.  FOLD: alpha from the operator's pairs
+template <typename T, bool FOLD>
 __global__ void __launch_bounds__(kBlock) k_seg_s(const int4* __restrict__ ch, const T* __restrict__ v,
-                                                  const T* __restrict__ r, const double* __restrict__ sc,
-                                                  T* __restrict__ s_out, double* __restrict__ partial) {
-    __shared__ double red[kBlock / 64];
+                                                  const T* __restrict__ r, double* __restrict__ sc,
+                                                  T* __restrict__ s_out, double* __restrict__ partial,
+                                                  const int64_t* __restrict__ chunk_begin,
+                                                  const int64_t* __restrict__ op_rng,
+                                                  const double* __restrict__ pairs) {
+    __shared__ double red[kBlock / 64], bc;
     const int4 e = ch[blockIdx.x];
-    const double* m = sc + (int64_t)e.z * BS_COUNT;
+    double* m = sc + (int64_t)e.z * BS_COUNT;
     if (m[BS_STOP] != 0.0) return;  // uniform over the workgroup; the stage skips stopped members
-    const double alpha = m[BS_ALPHA];
+    const double alpha = FOLD ? seg_alpha(m, op_rng + (int64_t)e.z * 2 * kMaxColors, pairs, red, &bc,
+                                          blockIdx.x == chunk_begin[e.z])
+                              : m[BS_ALPHA];
     double ss = 0;
     for (int64_t q = (int64_t)e.x + threadIdx.x; q < e.y; q += kBlock) {
         const T o = (T)fma(-alpha, (double)v[q], (double)r[q]);
@@ -102,18 +173,25 @@ __global__ void __launch_bounds__(kBlock) k_seg_s(const int4* __restrict__ ch, c
     if (threadIdx.x == 0) partial[blockIdx.x] = ss;
 }
 
-// x += alpha ph + omega sh;  r = s - omega t;  partial[2 chunk] = (rh.r, r.r)
-template <typename T>
+// x += alpha ph + omega sh;  r = s - omega t;  partial[2 chunk] = (rh.r, r.r).  FOLD: omega from
+// the operator's pairs and k_seg_s's partials
+template <typename T, bool FOLD>
 __global__ void __launch_bounds__(kBlock) k_seg_xr(const int4* __restrict__ ch, const T* __restrict__ ph,
                                                    const T* __restrict__ sh, const T* __restrict__ sv,
                                                    const T* __restrict__ tv, const T* __restrict__ rh,
-                                                   const double* __restrict__ sc, T* __restrict__ x, T* __restrict__ r,
-                                                   double* __restrict__ partial) {
-    __shared__ double red[kBlock / 64];
+                                                   double* __restrict__ sc, T* __restrict__ x, T* __restrict__ r,
+                                                   double* __restrict__ partial,
+                                                   const int64_t* __restrict__ chunk_begin,
+                                                   const int64_t* __restrict__ op_rng,
+                                                   const double* __restrict__ pairs, const double* __restrict__ ssp) {
+    __shared__ double red[kBlock / 64], bc;
     const int4 e = ch[blockIdx.x];
-    const double* m = sc + (int64_t)e.z * BS_COUNT;
+    double* m = sc + (int64_t)e.z * BS_COUNT;
     if (m[BS_STOP] != 0.0) return;
-    const double alpha = m[BS_ALPHA], omega = m[BS_OMEGA];
+    const double alpha = m[BS_ALPHA];
+    const double omega = FOLD ? seg_omega(m, op_rng + (int64_t)e.z * 2 * kMaxColors, pairs, chunk_begin[e.z],
+                                          chunk_begin[e.z + 1], ssp, red, &bc, blockIdx.x == chunk_begin[e.z])
+                              : m[BS_OMEGA];
     double d1 = 0, d2 = 0;
     for (int64_t q = (int64_t)e.x + threadIdx.x; q < e.y; q += kBlock) {
         x[q] = (T)fma(omega, (double)sh[q], fma(alpha, (double)ph[q], (double)x[q]));
@@ -206,15 +284,6 @@ __global__ void __launch_bounds__(kBlock) k_seg_axpy(const int4* __restrict__ ch
 // ---------------------------------------------------------------------------
 // stage: one workgroup per member turns that member's partials into its scalars
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ double stage_sum(double v, double* red, double* bc) {
-    const double s = block_sum(v, red);
-    if (threadIdx.x == 0) *bc = s;
-    __syncthreads();
-    const double r = *bc;
-    __syncthreads();
-    return r;
-}
-
 // mode ST_START: (rh.r, r.r) chunk pairs of the starting residual; ST_ALPHA: the first
 // operator application's (rh.v) pairs; ST_OMEGA: the second's (s.t, t.t) pairs and the
 // s.s chunk partials; ST_RHO: the x/r kernel's (rh.r, r.r) chunk pairs.  op_rng holds per
@@ -275,45 +344,10 @@ __global__ void __launch_bounds__(kStage) k_seg_stage(int mode, const int64_t* _
             }
         } else {
             const int64_t* rg = op_rng + (int64_t)m * 2 * kMaxColors;
-            double a = 0, b = 0;
-            for (int c = 0; c < kMaxColors; ++c)
-                for (int64_t k = rg[2 * c] + threadIdx.x; k < rg[2 * c + 1]; k += kStage) {
-                    a += pairs[2 * k];
-                    b += pairs[2 * k + 1];
-                }
-            a = stage_sum(a, red, &bc);
-            if (mode == ST_ALPHA) {
-                if (threadIdx.x == 0) {
-                    const bool ok = a != 0.0 && isfinite(a);
-                    S[BS_RHV] = a;
-                    S[BS_ALPHA] = ok ? S[BS_RHO] / a : 0.0;
-                    if (!ok) S[BS_FLAG] = 1;  // breakdown: the member stops at the end of the iteration
-                }
-            } else {
-                b = stage_sum(b, red, &bc);
-                double ss = 0;
-                for (int64_t k = chunk_begin[m] + threadIdx.x; k < chunk_begin[m + 1]; k += kStage) ss += ssp[k];
-                ss = stage_sum(ss, red, &bc);
-                if (threadIdx.x == 0) {
-                    // minimal-residual omega, enlarged when |cos(t, s)| < 0.7 (as the single solve)
-                    const double st = a, tt = b;
-                    double omega = 0;
-                    int flag = 0;
-                    if (tt > 0.0 && isfinite(st) && isfinite(tt)) {
-                        omega = st / tt;
-                        const double cs = st / sqrt(tt * ss);
-                        if (isfinite(cs) && fabs(cs) < 0.7 && fabs(cs) > 0.0) omega *= 0.7 / fabs(cs);
-                        if (omega == 0.0) flag = -2;
-                    } else {
-                        flag = 2;
-                    }
-                    S[BS_ST] = st;
-                    S[BS_TT] = tt;
-                    S[BS_SS] = ss;
-                    S[BS_OMEGA] = omega;
-                    if (flag == 2 || (flag == -2 && S[BS_FLAG] == 0.0)) S[BS_FLAG] = 2;
-                }
-            }
+            if (mode == ST_ALPHA)
+                (void)seg_alpha(S, rg, pairs, red, &bc, true);
+            else
+                (void)seg_omega(S, rg, pairs, c0, c1, ssp, red, &bc, true);
         }
     }
     if (host_slot) {  // every member's scalars into the host-visible slot the host waits on
@@ -337,6 +371,7 @@ struct Segments {
     DevBuf<double> part;          // nchunk doubles (norm / max partials)
     DevBuf<double> red;           // M doubles
     HostBuf<double> h_red;        // M doubles
+    bool fold = false;            // alpha and omega inside the s and x/r kernels (kFoldPairs)
 };
 
 // color: colour of every union face; face_off: member m owns faces [face_off[m], face_off[m+1])
@@ -436,6 +471,15 @@ void build_segments(Segments& sg, const ColorOrder& co, const std::vector<int32_
     sg.nchunk = (int64_t)ch.size();
     sg.chunks.alloc(ch.size());
     sg.chunk_begin.alloc(M + 1);
+    sg.fold = true;
+    for (int m = 0; m < M; ++m) {
+        int64_t pairs = 0;
+        for (int c = 0; c < kMaxColors; ++c) {
+            const int64_t* r = &rng[((size_t)m * kMaxColors + c) * 2];
+            pairs += r[1] - r[0];
+        }
+        sg.fold = sg.fold && pairs <= kFoldPairs;
+    }
     sg.op_rng.alloc(rng.size());
     sg.part.alloc(std::max<int64_t>(1, sg.nchunk));
     sg.red.alloc(M);
@@ -538,26 +582,39 @@ void enqueue_iteration(hipStream_t s, Segments& sg, const ColorOrder& co, DiluFa
         hipLaunchKernelGGL((k_seg_p<T>), dim3(nch), dim3(kBlock), 0, s, sg.chunks.p, w.r.p, w.v.p, w.sc.p, w.p.p,
                            w.rh.p);
     split_apply_batch<T>(s, co, sg.F, sg.L, d, sg.sweep, w.p.p, w.v.p, w.rh.p, w.op_part.p, stop, BS_COUNT);
-    hipLaunchKernelGGL(k_seg_stage, dim3(M), dim3(kStage), 0, s, (int)ST_ALPHA, sg.chunk_begin.p, sg.op_rng.p,
-                       w.op_part.p, (const double*)nullptr, w.sc.p, (const double*)nullptr, (double*)nullptr, 0.0);
-    hipLaunchKernelGGL((k_seg_s<T>), dim3(nch), dim3(kBlock), 0, s, sg.chunks.p, w.v.p, w.r.p, w.sc.p, w.sv.p,
-                       w.ss_part.p);
+    if (sg.fold) {
+        hipLaunchKernelGGL((k_seg_s<T, true>), dim3(nch), dim3(kBlock), 0, s, sg.chunks.p, w.v.p, w.r.p, w.sc.p, w.sv.p,
+                           w.ss_part.p, sg.chunk_begin.p, sg.op_rng.p, w.op_part.p);
+    } else {
+        hipLaunchKernelGGL(k_seg_stage, dim3(M), dim3(kStage), 0, s, (int)ST_ALPHA, sg.chunk_begin.p, sg.op_rng.p,
+                           w.op_part.p, (const double*)nullptr, w.sc.p, (const double*)nullptr, (double*)nullptr, 0.0);
+        hipLaunchKernelGGL((k_seg_s<T, false>), dim3(nch), dim3(kBlock), 0, s, sg.chunks.p, w.v.p, w.r.p, w.sc.p,
+                           w.sv.p, w.ss_part.p, sg.chunk_begin.p, sg.op_rng.p, w.op_part.p);
+    }
     split_apply_batch<T>(s, co, sg.F, sg.L, d, sg.sweep, w.sv.p, w.t.p, w.sv.p, w.op_part.p, stop, BS_COUNT);
-    hipLaunchKernelGGL(k_seg_stage, dim3(M), dim3(kStage), 0, s, (int)ST_OMEGA, sg.chunk_begin.p, sg.op_rng.p,
-                       w.op_part.p, w.ss_part.p, w.sc.p, (const double*)nullptr, (double*)nullptr, 0.0);
-    hipLaunchKernelGGL((k_seg_xr<T>), dim3(nch), dim3(kBlock), 0, s, sg.chunks.p, w.p.p, w.sv.p, w.sv.p, w.t.p,
-                       w.rh.p, w.sc.p, x, w.r.p, w.xr_part.p);
+    if (sg.fold) {
+        hipLaunchKernelGGL((k_seg_xr<T, true>), dim3(nch), dim3(kBlock), 0, s, sg.chunks.p, w.p.p, w.sv.p, w.sv.p, w.t.p,
+                           w.rh.p, w.sc.p, x, w.r.p, w.xr_part.p, sg.chunk_begin.p, sg.op_rng.p, w.op_part.p,
+                           w.ss_part.p);
+    } else {
+        hipLaunchKernelGGL(k_seg_stage, dim3(M), dim3(kStage), 0, s, (int)ST_OMEGA, sg.chunk_begin.p, sg.op_rng.p,
+                           w.op_part.p, w.ss_part.p, w.sc.p, (const double*)nullptr, (double*)nullptr, 0.0);
+        hipLaunchKernelGGL((k_seg_xr<T, false>), dim3(nch), dim3(kBlock), 0, s, sg.chunks.p, w.p.p, w.sv.p, w.sv.p,
+                           w.t.p, w.rh.p, w.sc.p, x, w.r.p, w.xr_part.p, sg.chunk_begin.p, sg.op_rng.p, w.op_part.p,
+                           w.ss_part.p);
+    }
     hipLaunchKernelGGL(k_seg_stage, dim3(M), dim3(kStage), 0, s, (int)ST_RHO, sg.chunk_begin.p, sg.op_rng.p,
                        w.xr_part.p, (const double*)nullptr, w.sc.p, (const double*)nullptr,
                        w.hsc_dev + (size_t)M * BS_COUNT * slot, sizeof(T) == 4 ? kBicgRestartEps32 : 0.0);
     PB_HIP(hipGetLastError());
 }
 
-// launches per iteration: p (or the copy), three stages, s, x/r and two operator applications
+// launches per iteration: p (or the copy), three stages (one when folded), s, x/r and two operator
+// applications
 inline int64_t iteration_launches(const Segments& sg, const ColorOrder& co) {
     int nc = 0;
     for (int c = 0; c < co.ncolor; ++c) nc += sg.sweep.nblk[c] > 0;
-    return 6 + 2 * (2 * nc - 1);
+    return (sg.fold ? 4 : 6) + 2 * (2 * nc - 1);
 }
 
 // Batched BiCGStab on the split operator Ahat from x = 0: each member runs until its own
