@@ -312,9 +312,10 @@ static SplitCycles split_cycles(pbsm3d_ctx* c) {
         (void)hipGetLastError();
         return SplitCycles{};
     }
+    // among the column modes only: GMRES on the same system gives the same bits in every context
     if (c->split_mode < 0)
-        c->split_mode =
-            tune_split_mode<double>(c->stream, c->co, c->F, c->L, c->dl_s, c->bp.p, c->split64[0].p, nullptr);
+        c->split_mode = tune_split_mode<double>(c->stream, c->co, c->F, c->L, c->dl_s, c->bp.p, c->split64[0].p,
+                                                nullptr, kColumnModes);
     SplitCycles sp{CsrOp<double>{N, nullptr, nullptr, nullptr, &c->prof, c->F, c->L}, {}, neumann_degree(N)};
     sp.Ahat.co = &c->co;
     sp.Ahat.split = &c->dl_s;
@@ -798,7 +799,10 @@ int pbsm3d_step(pbsm3d_ctx* c, const pbsm3d_forcing* fo, int32_t dt_s, pbsm3d_ou
                 // position order (one layer) reach the target in as many iterations as GMRES(30)
                 // and two thirds of BiCGStab's applications.  5,000 faces 0.50 ms with GMRES, now 0.33;
                 // 50,000 0.87 and 0.58; 125,000 0.95 with BiCGStab, now 0.71; 999,968 5.3 and 3.7, now 3.0.
-                dilu_factor<double>(s, c->co, F, 1, c->dep.rp.p, c->dep.val.p, c->slots.p, c->dl_d);
+                // The matrix (areas and edge weights) depends on the mesh alone: one factorisation per context.
+                if (!c->dep_factored)
+                    dilu_factor<double>(s, c->co, F, 1, c->dep.rp.p, c->dep.val.p, c->slots.p, c->dl_d);
+                c->dep_factored = true;
                 to_pos<double, double>(s, c->co, F, 1, c->dep.rhs.p, c->dsplit[0].p);
                 to_pos<double, double>(s, c->co, F, 1, c->dep.x.p, c->dsplit[1].p);
                 CsrOp<double> Dp{F, nullptr, nullptr, nullptr, nullptr, F, 1};
@@ -814,7 +818,7 @@ int pbsm3d_step(pbsm3d_ctx* c, const pbsm3d_forcing* fo, int32_t dt_s, pbsm3d_ou
             }
             if (!si.converged) {  // no D-ILU, or a smoothing coefficient that leaves the system indefinite
                 if (cfg.dep_precond == PBSM3D_PC_MCILU0) {
-                    if (before == 0)
+                    if (!c->dep_factored)
                         dilu_factor<double>(s, c->co, F, 1, c->dep.rp.p, c->dep.val.p, c->slots.p, c->dl_d);
                     M = [c, F](hipStream_t st2, const double* r, double* z) {
                         dilu_apply<double>(st2, c->co, F, 1, c->dl_d, r, z);

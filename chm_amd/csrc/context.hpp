@@ -47,6 +47,7 @@ struct pbsm3d_ctx {
     pb::ColumnFactors colf;
     pb::ColorOrder co;
     pb::DiluFactors<double> dl_s, dl_d;
+    bool dep_factored = false;  // dl_d holds the deposition system's factors (a context, not a batch)
     pb::DiluFactors<float> dl32;
     pb::DevBuf<double> invdiag_s, invdiag_d, r_s, r_d;
     pb::DevBuf<double> bp, xp;  // suspension b and x in the D-ILU position order

@@ -327,11 +327,12 @@ template <typename T>
 void split_apply_batch(hipStream_t s, const ColorOrder& co, int64_t F, int L, DiluFactors<T>& d, const SweepTables& st,
                        const T* in, T* out, const T* dw, double* partial, const double* stop, int stop_stride);
 constexpr int kSplitModes = 8;
-// times split_op(0) in each mode (HIP events on the stream) and returns the fastest;
-// ms_out[kSplitModes] receives the averages (ms), if given.
+constexpr int kColumnModes = 4;  // the modes whose results are the same bit for bit
+// times split_op(0) in the first `modes` modes (HIP events on the stream) and returns the fastest;
+// ms_out[modes] receives the averages (ms), if given.
 template <typename T>
 int tune_split_mode(hipStream_t s, const ColorOrder& co, int64_t F, int L, DiluFactors<T>& d, const T* w, T* o,
-                    float* ms_out);
+                    float* ms_out, int modes = kSplitModes);
 // FP32 copy of FP64 factors (the FP32 preconditioner and operator of the mixed solve)
 void dilu_narrow(hipStream_t s, int64_t N, const DiluFactors<double>& a, DiluFactors<float>& b);
 // y = b - A x with per-block partial sums of y.y, everything in position order, A taken

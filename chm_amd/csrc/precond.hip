@@ -1436,13 +1436,13 @@ void split_apply_batch(hipStream_t s, const ColorOrder& co, int64_t F, int L, Di
 
 template <typename T>
 int tune_split_mode(hipStream_t s, const ColorOrder& co, int64_t F, int L, DiluFactors<T>& d, const T* w, T* o,
-                    float* ms_out) {
+                    float* ms_out, int modes) {
     hipEvent_t e0, e1;
     PB_HIP(hipEventCreate(&e0));
     PB_HIP(hipEventCreate(&e1));
     int best = 0;
     float best_ms = 0;
-    for (int m = 0; m < kSplitModes; ++m) {
+    for (int m = 0; m < modes; ++m) {
         float ms = 0;
         split_op<T>(0, s, co, F, L, d, w, o, m);
         PB_HIP(hipEventRecord(e0, s));
@@ -1603,9 +1603,9 @@ template int64_t split_apply_dots<double>(hipStream_t, const ColorOrder&, int64_
 template int64_t split_apply_dots<float>(hipStream_t, const ColorOrder&, int64_t, int, DiluFactors<float>&,
                                          const float*, float*, const float*, double*, int, const double*);
 template int tune_split_mode<double>(hipStream_t, const ColorOrder&, int64_t, int, DiluFactors<double>&,
-                                     const double*, double*, float*);
+                                     const double*, double*, float*, int);
 template int tune_split_mode<float>(hipStream_t, const ColorOrder&, int64_t, int, DiluFactors<float>&, const float*,
-                                    float*, float*);
+                                    float*, float*, int);
 template bool tune_dilu_xcd<double>(hipStream_t, const ColorOrder&, int64_t, int, DiluFactors<double>&, const double*,
                                     double*, float*);
 template bool tune_dilu_xcd<float>(hipStream_t, const ColorOrder&, int64_t, int, DiluFactors<float>&, const float*,
