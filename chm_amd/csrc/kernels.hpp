@@ -305,6 +305,11 @@ void split_op(int which, hipStream_t s, const ColorOrder& co, int64_t F, int L, 
 template <typename T>
 int64_t split_apply_dots(hipStream_t s, const ColorOrder& co, int64_t F, int L, DiluFactors<T>& d, const T* in, T* out,
                          const T* dw, double* partial, int mode, const double* stop = nullptr);
+// out = v + (y - Ahat y), the Neumann polynomial's recurrence, in the operator's own launches (a
+// column mode): a pass of its own read three vectors more, 55 us beside the operator's 270 at
+// 999,968 faces x 10 layers.  out must differ from v and y.
+void split_neumann(hipStream_t s, const ColorOrder& co, int64_t F, int L, DiluFactors<double>& d, const double* v,
+                   const double* y, double* out, int mode);
 // Workgroup tables of a batch of independent systems held as one union (batch.hip):
 // the union's faces are member-major, so each colour's positions are too, and the
 // sweeps of colour c run as nblk[c] workgroups, tab[c][b] = {k0, k1, member, a} (faces
@@ -437,7 +442,5 @@ void scale_f64_to_f32_host(hipStream_t s, int64_t n, const double* r, double alp
 void axpy_dev_scaled_f32(hipStream_t s, int64_t n, const double* scale, const float* x, double* y);  // y += (*scale) x
 void axpy_f64(hipStream_t s, int64_t n, double alpha, const double* x, double* y);
 void copy_f64(hipStream_t s, int64_t n, const double* a, double* b);
-// out = v + y - ay (out may be y)
-void neumann_step(hipStream_t s, int64_t n, const double* v, const double* y, const double* ay, double* out);
 
 }  // namespace pb

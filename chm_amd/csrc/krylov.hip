@@ -217,12 +217,13 @@ int split_cycle(hipStream_t s, GmresWork<double>& w, const SplitCycles& sp, cons
     PcFn<double> q;  // degree 1: q = 1
     if (sp.degree > 1)
         q = [&](hipStream_t st, const double* v, double* z) {
-            // Horner: z = v, then z <- v + z - Ahat z
+            // Horner: y0 = v, then y <- v + y - Ahat y, alternating between two vectors so that the
+            // last lands in z
             const double* from = v;
             for (int k = 1; k < sp.degree; ++k) {
-                op_spmv<double>(st, A, from, y);
-                neumann_step(st, n, v, from, y, z);
-                from = z;
+                double* to = (sp.degree - 1 - k) % 2 == 0 ? z : y;
+                split_neumann(st, *A.co, A.F, A.L, *A.split, v, from, to, A.mode);
+                from = to;
             }
         };
     double est = 0;

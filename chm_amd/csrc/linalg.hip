@@ -1085,15 +1085,6 @@ void cg_p(hipStream_t s, int64_t n, int it, const double* r, const double* dinv,
                        seq);
 }
 
-__global__ void __launch_bounds__(kBlock) k_neumann(int64_t n, const double* v, const double* y, const double* ay,
-                                                    double* out) {
-    const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k < n) out[k] = v[k] + (y[k] - ay[k]);
-}
-void neumann_step(hipStream_t s, int64_t n, const double* v, const double* y, const double* ay, double* out) {
-    hipLaunchKernelGGL(k_neumann, dim3(grid_for(n)), dim3(kBlock), 0, s, n, v, y, ay, out);
-}
-
 template <typename T>
 void scale_host(hipStream_t s, int64_t n, const T* a, double alpha, T* b) {
     hipLaunchKernelGGL((k_scale_host<T>), dim3(grid_for(n)), dim3(kBlock), 0, s, n, a, alpha, b);

@@ -375,10 +375,12 @@ __global__ void __launch_bounds__(kBlock) k_eis_bwd(int64_t F, int Lrt, int64_t 
 // o = w - acc, v = D~^-1 o (without t: the left transform b^ = D~ (D~ + L)^-1 b).
 // FUSE: colour 0 (no lower neighbours), whose backward sweep runs first in the
 // same thread and whose t stays in registers.
+// NEU: dw is the Neumann recurrence's constant term and o receives dw + (w - o) instead.
 // PRE_DW: the dot vector is loaded with the rest of the column (more loads in flight, ten
 // more VGPRs) rather than in the final loop.  SV = false: v is not stored (the top colour,
 // whose v no higher colour gathers)
-template <typename T, int LM, bool EX, bool WITH_T, bool FUSE, bool DOTS, bool NT, bool PRE_DW = true, bool SV = true>
+template <typename T, int LM, bool EX, bool WITH_T, bool FUSE, bool DOTS, bool NT, bool PRE_DW = true, bool SV = true,
+          bool NEU = false>
 __device__ __forceinline__ void eis_fwd_column(int64_t F, int Lrt, int64_t k, const int32_t* __restrict__ nbp,
                                                const uint8_t* __restrict__ lowmask, const T* __restrict__ lat,
                                                const T* __restrict__ vert, const T* __restrict__ dinv,
@@ -409,7 +411,7 @@ __device__ __forceinline__ void eis_fwd_column(int64_t F, int Lrt, int64_t k, co
         if (z < L) {
             const uint32_t q = qb + (uint32_t)z * qs;
             wv[z] = w[q];
-            if (DOTS && PRE_DW) dwv[z] = dw[q];
+            if ((DOTS && PRE_DW) || NEU) dwv[z] = dw[q];
             dv[z] = ldc<NT>(&dinv[q]);
             vb[z] = z > 0 ? ldc<NT>(&vert[q]) : T(0);
             T acc = 0;
@@ -469,7 +471,7 @@ __device__ __forceinline__ void eis_fwd_column(int64_t F, int Lrt, int64_t k, co
                 vz = dv[z] * oz;
             }
             if (SV) v[q] = vz;
-            o[q] = oz;
+            o[q] = NEU ? dwv[z] + (wv[z] - oz) : oz;
             prev = vz;
             if (DOTS) {
                 d1 = fma((double)(PRE_DW ? dwv[z] : dw[q]), (double)oz, d1);
@@ -479,7 +481,7 @@ __device__ __forceinline__ void eis_fwd_column(int64_t F, int Lrt, int64_t k, co
 }
 
 // DOTS: per-block partial sums (dw . o, o . o) into partial[2 * logical block] (FP64).
-template <typename T, int LM, bool EX, bool XCD, bool WITH_T, bool FUSE, bool DOTS, bool NT, bool SV = true>
+template <typename T, int LM, bool EX, bool XCD, bool WITH_T, bool FUSE, bool DOTS, bool NT, bool SV = true, bool NEU = false>
 __global__ void __launch_bounds__(kBlock) k_eis_fwd(int64_t F, int L, int64_t k0, int64_t k1,
                                                     const int32_t* __restrict__ nbp,
                                                     const uint8_t* __restrict__ lowmask, const T* __restrict__ lat,
@@ -495,8 +497,8 @@ __global__ void __launch_bounds__(kBlock) k_eis_fwd(int64_t F, int L, int64_t k0
     const int64_t k = kb + lb * kBlock + threadIdx.x;
     double d1 = 0, d2 = 0;
     if (k >= k0 && k < k1)
-        eis_fwd_column<T, LM, EX, WITH_T, FUSE, DOTS, NT, true, SV>(F, L, k, nbp, lowmask, lat, vert, dinv, E, w, t,
-                                                                    tnb, vnb, v, o, dw, d1, d2);
+        eis_fwd_column<T, LM, EX, WITH_T, FUSE, DOTS, NT, true, SV, NEU>(F, L, k, nbp, lowmask, lat, vert, dinv, E, w,
+                                                                         t, tnb, vnb, v, o, dw, d1, d2);
     if constexpr (DOTS) {
         // partials indexed by the logical block: the fixed-order sum sees the same faces in
         // the same order with and without the XCD workgroup mapping (blocks past the colour
@@ -1186,13 +1188,19 @@ bool tune_dilu_xcd(hipStream_t s, const ColorOrder& co, int64_t F, int L, DiluFa
 }
 
 namespace {
-// one forward launch of colour c; with dw the block partials of (dw . o, o . o) go to
-// partial[2 * (nb + block)] and nb advances by the launch's block count
+// one forward launch of colour c; with dw and partial the block partials of (dw . o, o . o) go to
+// partial[2 * (nb + block)] and nb advances by the launch's block count; with dw alone o receives
+// the Neumann step dw + (w - o)
 // SV = false for the top colour: its v is not stored, no higher colour gathers it
 template <typename T, int LM, bool EX, bool XCD, bool NT, bool WITH_T, bool FUSE, bool SV>
 void launch_fwd(hipStream_t s, dim3 g, int64_t F, int L, const ColorOrder& co, int c, DiluFactors<T>& d, const T* w,
                 T* o, const T* dw, double* partial, int64_t& nb, const double* stop) {
-    if (dw) {
+    if (dw && !partial) {
+        if constexpr (sizeof(T) == 8)
+            hipLaunchKernelGGL((k_eis_fwd<T, LM, EX, XCD, WITH_T, FUSE, false, NT, SV, true>), g, dim3(kBlock), 0, s, F,
+                               L, co.off[c], co.off[c + 1], co.nbp.p, co.lowmask.p, d.lat.p, d.vert.p, d.dinv.p, d.E.p,
+                               w, d.t.p, d.t.p, d.y.p, d.y.p, o, dw, partial, stop);
+    } else if (dw) {
         hipLaunchKernelGGL((k_eis_fwd<T, LM, EX, XCD, WITH_T, FUSE, true, NT, SV>), g, dim3(kBlock), 0, s, F, L,
                            co.off[c], co.off[c + 1], co.nbp.p, co.lowmask.p, d.lat.p, d.vert.p, d.dinv.p, d.E.p, w,
                            d.t.p, d.t.p, d.y.p, d.y.p, o, dw, partial + 2 * nb, stop);
@@ -1382,6 +1390,12 @@ int64_t split_apply_dots(hipStream_t s, const ColorOrder& co, int64_t F, int L, 
                          const T* dw, double* partial, int mode, const double* stop) {
     check_split_size(F, L);
     return split_mode_dispatch<T>(0, s, co, F, L, d, in, out, dw, partial, mode, stop);
+}
+
+void split_neumann(hipStream_t s, const ColorOrder& co, int64_t F, int L, DiluFactors<double>& d, const double* v,
+                   const double* y, double* out, int mode) {
+    check_split_size(F, L);
+    split_mode_dispatch<double>(0, s, co, F, L, d, y, out, v, nullptr, mode & (kColumnModes - 1), nullptr);
 }
 
 namespace {
