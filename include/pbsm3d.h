@@ -136,15 +136,15 @@ typedef struct pbsm3d_config {
                                        predicted profile on T tiles (face-index ranges)     */
 } pbsm3d_config;
 
-/* Krylov method of the suspension solve (the deposition solve is GMRES(restart)) */
+/* Krylov method of the suspension solve.  The deposition system is symmetric positive definite: with
+ * dep_precond MCILU0 it is solved by conjugate gradients, else (and if it turns out indefinite)
+ * by GMRES(restart). */
 #define PBSM3D_KRYLOV_GMRES 0     /* restarted GMRES(restart), as Belos "GMRES"     */
 #define PBSM3D_KRYLOV_BICGSTAB 1  /* BiCGStab: short recurrences, 2 SpMV/iteration  */
 #define PBSM3D_KRYLOV_BICGSTAB_SPLIT 2  /* BiCGStab on the split D-ILU system (Eisenstat's
                                           trick: each operator application is one backward
                                           and one forward sweep, no SpMV) inside FP64
-                                          refinement; precond MCILU0, nLayer <= 16.  With
-                                          dep_precond MCILU0 the deposition system is solved
-                                          the same way (FP64) */
+                                          refinement; precond MCILU0, nLayer <= 16 */
 
 typedef struct pbsm3d_forcing {
     const double* U_R;            /* [F] m/s at Z_U_R = 50 m                       */
@@ -181,7 +181,8 @@ typedef struct pbsm3d_out {
 typedef struct pbsm3d_stats {
     int32_t suspension_present;
     int32_t deposition_present;
-    int32_t susp_iters;           /* total Krylov iterations (all restarts/cycles)  */
+    int32_t susp_iters;           /* total Krylov iterations (all restarts/cycles);
+                                     GMRES: applications of the preconditioned operator */
     int32_t dep_iters;
     double susp_resid;            /* final ||b - A x|| / ||b|| (explicit)           */
     double dep_resid;
