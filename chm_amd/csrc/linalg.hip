@@ -870,8 +870,11 @@ __global__ void __launch_bounds__(kBlock) k_cg_p(int64_t n, int it, const double
                                                  uint64_t seq) {
     __shared__ double s_red[kBlock / 64], s_beta;
     // workgroup 0 sets the stop below: one that starts later may skip its part of a p that no
-    // later launch reads
-    if (sc[CG_STOP] != 0.0) return;
+    // later launch reads, but its threads have to agree on it
+    __shared__ bool s_stop;
+    if (threadIdx.x == 0) s_stop = sc[CG_STOP] != 0.0;
+    __syncthreads();
+    if (s_stop) return;
     const double rho = sum_partials(partial, nblk, 1, 0, s_red);
     if (threadIdx.x == 0) {
         s_beta = rho / sc[CG_RHO + ((it - 1) & 1)];
