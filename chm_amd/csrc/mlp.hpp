@@ -54,8 +54,10 @@ class Mlp {
     int64_t cap = 0;
     DevBuf<uint16_t> Xb, Ab[3];  // workspace of the layer-by-layer forward
     DevBuf<float> Yp;
-    DevBuf<float> slab;        // gradients of one batch, one slab per workgroup
-    DevBuf<double> loss_part;  // summed squared error per workgroup
+    DevBuf<uint16_t> tiles;    // a batch's activations and gradients by 64-sample tile
+    DevBuf<float> slab;        // its weight gradients, one slab per row range
+    DevBuf<float> bias_part;   // its bias gradients, one row per row block
+    DevBuf<float> loss_part;   // summed squared error per 16 rows
     DevBuf<double> loss_dev;   // the epoch's summed batch losses
     int64_t t_adam = 0;
 };

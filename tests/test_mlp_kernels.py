@@ -102,3 +102,87 @@ def test_training_step_is_adam_on_the_sampled_rows():
     # output rows past the eleven targets are never stepped
     o = p.size - 16 * 128 - 16
     assert np.all(step[o + 11 * 128:o + 16 * 128] == 0) and np.all(step[-5:] == 0)
+
+
+def _uniform_net(seed):
+    """A network whose parameters are exact multiples of uniform counters (no libm in their making)."""
+    from chm_amd import meshgen
+    from chm_amd import pbsm3d as pb
+
+    u = meshgen.uniform(seed, 31, 37264 + 54)
+    p, o = np.zeros(37264, dtype=np.float32), 0
+    for r, c in mlp_oracle.SHAPES:
+        rows = r if r == mlp_oracle.H else mlp_oracle.OUT  # output rows past the targets stay zero
+        p[o:o + rows * c] = (u[o:o + rows * c] - 0.5) * (2.0 * np.sqrt(6.0 / c))
+        o += r * c
+        p[o:o + rows] = (u[o:o + rows] - 0.5) * 0.5
+        o += r
+    v = u[37264:]
+    net = pb.Mlp(seed=seed)
+    net.set_params(p)
+    net.set_normalization(v[:16] - 0.5, 0.5 + v[16:32], v[32:43] - 0.5, 0.5 + v[43:54])
+    return net
+
+
+def _uniform_rows(seed, n):
+    from chm_amd import meshgen
+
+    X = (4.0 * meshgen.uniform(seed, 32, 16 * n) - 2.0).astype(np.float32).reshape(n, 16)
+    return X, (4.0 * meshgen.uniform(seed, 33, 11 * n) - 2.0).astype(np.float32).reshape(n, 11)
+
+
+def _digest(*arrays):
+    import hashlib
+
+    h = hashlib.sha256()
+    for a in arrays:
+        h.update(np.ascontiguousarray(a).tobytes())
+    return h.hexdigest()[:16]
+
+
+def _network_bits(what, n, batch):
+    import torch
+
+    net = _uniform_net(3)
+    X, Y = _uniform_rows(n, n)
+    Xd, Yd = torch.tensor(X, device="cuda:0"), torch.tensor(Y, device="cuda:0")
+    if what == "predict":
+        out = torch.full((n, 11), np.nan, dtype=torch.float32, device="cuda:0")
+        net.predict(Xd, out)
+        return _digest(out.cpu().numpy())
+    if what == "gradients":
+        loss, g = net.gradients(X, Y)
+        return _digest(np.float64(loss), g)
+    loss = net.train(Xd, Yd, epochs=3, batch=batch, lr=2e-3, seed=9)
+    return _digest(np.float64(loss), net.get_params())
+
+
+# Slabs of the weight gradients: one (n < 1024), ends inside a tile (1060), 9 of 576 rows (5000), 64
+# (32768 and more); row blocks of the bias gradients: tiles, or across them (from 32769 on)
+BITS = [
+    ("predict", 1, 0, "751c4467ceb9c22b"),
+    ("predict", 1000, 0, "d68a15674364c0a4"),
+    ("predict", 131137, 0, "cffbd442bdfb2b2a"),
+    ("gradients", 1, 0, "89909ec7c993f64f"),
+    ("gradients", 200, 0, "e43fe30b3edb93a0"),
+    ("gradients", 1060, 0, "aa5d2602d468d0d4"),
+    ("gradients", 5000, 0, "280be4b727e95bf9"),
+    ("gradients", 16484, 0, "9b767333a3ac39b5"),
+    ("gradients", 32768, 0, "f170e5cd60941281"),
+    ("gradients", 32769, 0, "c30b524f2549a11e"),
+    ("gradients", 49159, 0, "f76b28e07e97963c"),
+    ("train", 333, 333, "c094b065aa05a279"),
+    ("train", 20000, 2048, "408658507db1c732"),
+    ("train", 20000, 5000, "9b795a52f2569451"),
+    ("train", 50000, 8192, "bc2d1e79e45b1bff"),
+    ("train", 60000, 40000, "81b93b1810bb50a9"),
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("what,n,batch,want", BITS)
+def test_network_bits(what, n, batch, want):
+    """The kernels keep the bits of the trainer and forward that ran one launch per product, slab sum,
+    column sum and elementwise step: the digests are of its outputs, recorded on an MI355X."""
+    print(f"[case] network bits {what} n={n} batch={batch}", flush=True)
+    assert _network_bits(what, n, batch) == want
