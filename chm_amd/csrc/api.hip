@@ -398,11 +398,23 @@ SolveInfo solve_in_position_order(pbsm3d_ctx* c, const pbsm3d_config& cfg, int64
         PcFn<double> M = [c, F, L](hipStream_t st, const double* r, double* z) {
             dilu_apply<double>(st, c->co, F, L, c->dl_s, r, z, true, (c->dilu_mode[0] & 1) != 0);
         };
-        if (bicg)
+        if (bicg) {
             si = bicgstab_solve(s, c->bw64, c->ws64, A, M, c->bp.p, c->xp.p, cfg.max_iters, cfg.tol);
-        else
-            si = gmres_solve(s, c->ws64, A, M, c->bp.p, c->xp.p, c->r_s.p, cfg.restart, cfg.max_iters, cfg.tol,
-                             split_cycles(c));
+        } else {
+            const SplitCycles split = split_cycles(c);
+            auto gmres = [&](const SplitCycles& sp) {
+                return gmres_solve(s, c->ws64, A, M, c->bp.p, c->xp.p, c->r_s.p, cfg.restart, cfg.max_iters, cfg.tol, sp);
+            };
+            si = gmres(split);
+            if (!si.converged && split.degree > 0) {
+                // A polynomial step takes `degree` of the iterations that max_iters allows (at 107,442
+                // unknowns 28 where plain cycles take 22), and a spectrum the polynomial does not suit
+                // takes more still: from the start once more, with plain cycles alone, so that the limit
+                // bounds GMRES's own iterations.
+                to_pos<double, double>(s, c->co, F, L, c->susp.x.p, c->xp.p);
+                si = gmres(SplitCycles{});
+            }
+        }
     } else {
         CsrOp<float> A32{N, nullptr, nullptr, nullptr, &c->prof, F, L};
         A32.co = &c->co;

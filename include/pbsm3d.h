@@ -181,8 +181,10 @@ typedef struct pbsm3d_out {
 typedef struct pbsm3d_stats {
     int32_t suspension_present;
     int32_t deposition_present;
-    int32_t susp_iters;           /* total Krylov iterations (all restarts/cycles);
-                                     GMRES: applications of the preconditioned operator */
+    int32_t susp_iters;           /* total Krylov iterations (all restarts/cycles), at most
+                                     max_iters.  FP64 GMRES: applications of the preconditioned
+                                     operator; of the plain cycles alone where those on the
+                                     split operator did not converge within max_iters */
     int32_t dep_iters;
     double susp_resid;            /* final ||b - A x|| / ||b|| (explicit)           */
     double dep_resid;

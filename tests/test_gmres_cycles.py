@@ -96,3 +96,47 @@ def test_deposition_cg_and_its_fallback(points, layers, smooth):
     assert len(res) == 2 or smooth < 0
     if len(res) == 2 and smooth >= 0:
         assert rel_err(res[0], res[1]) < 1e-8
+
+
+def _residual(ctx, conc):
+    """||b - A x|| / ||b|| of the exported suspension system, on the host."""
+    import scipy.sparse as sp
+
+    rp, col, val, b = ctx.system(0)
+    A = sp.csr_matrix((val, col, rp), shape=(b.size, b.size))
+    return np.linalg.norm(b - A @ conc) / np.linalg.norm(b)
+
+
+def test_limit_that_plain_cycles_meet(oracle):
+    """max_iters bounds GMRES's own iterations: a limit that GMRES(30) with the same preconditioner
+    meets is met, also where the polynomial's applications would exceed it."""
+    from chm_amd import pbsm3d as pb
+
+    print("[case] gmres limit of plain cycles", flush=True)
+    mesh = meshgen.synthetic_mesh(6000, seed=5)
+    g = pb.face_geometry(mesh)
+    fo = meshgen.forcing_c2(mesh.n_faces, seed=9)
+    orc = oracle.Oracle(g, oracle.oracle_config(nLayer=9, precond=abi.PC_MCILU0))
+    _, ost = orc.step(fo)
+    for limit in (ost["susp_iters"] + 1, ost["susp_iters"] + 3):
+        ctx = pb.Context(g, pb.default_config(nLayer=9, max_iters=limit))
+        o, st = ctx.step(fo, want_fields=True)
+        assert st["susp_iters"] <= limit and st["susp_resid"] <= 1e-8
+        assert _residual(ctx, o["conc"]) <= 1.01e-8
+        ctx.close()
+
+
+def test_spectrum_that_the_polynomial_does_not_suit():
+    """A small negative diffusion constant leaves a system that GMRES(30) solves in 40 iterations and
+    the polynomial's cycles (degree 10 at this size) do not solve in 1000 applications."""
+    from chm_amd import pbsm3d as pb
+
+    print("[case] gmres negative diffusion", flush=True)
+    mesh = meshgen.synthetic_mesh(106000, seed=5)
+    g = pb.face_geometry(mesh)
+    fo = meshgen.forcing_c2(mesh.n_faces, seed=9)
+    ctx = pb.Context(g, pb.default_config(nLayer=10, snow_diffusion_const=-0.024))
+    o, st = ctx.step(fo, want_fields=True)
+    assert st["susp_iters"] < 100 and st["susp_resid"] <= 1e-8
+    assert _residual(ctx, o["conc"]) <= 1.01e-8
+    ctx.close()
