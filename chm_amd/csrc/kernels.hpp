@@ -441,6 +441,8 @@ void axpy_f32_into_f64(hipStream_t s, int64_t n, double alpha, const float* x, d
 void scale_f64_to_f32_host(hipStream_t s, int64_t n, const double* r, double alpha, float* out);  // out = alpha*r
 void axpy_dev_scaled_f32(hipStream_t s, int64_t n, const double* scale, const float* x, double* y);  // y += (*scale) x
 void axpy_f64(hipStream_t s, int64_t n, double alpha, const double* x, double* y);
+// the same, and old = the y before
+void axpy_f64_keep(hipStream_t s, int64_t n, double alpha, const double* x, double* y, double* old);
 void copy_f64(hipStream_t s, int64_t n, const double* a, double* b);
 
 }  // namespace pb

@@ -205,17 +205,18 @@ bool start_norms(hipStream_t s, GmresWork<T>& w, const CsrOp<double>& A, double*
 
 namespace {
 // One cycle on Ahat with the Neumann polynomial: x += (D~ + U)^-1 q(Ahat) y, where y minimises
-// ||rhat - Ahat q(Ahat) y||, rhat = D~ (D~ + L)^-1 r.  Returns the operator applications of its
-// steps, 0 when the polynomial overflowed (x is unchanged then).
-int split_cycle(hipStream_t s, GmresWork<double>& w, const SplitCycles& sp, const double* r, double beta,
-                double stop_rel, int max_steps, double* x) {
+// ||rhat - Ahat q(Ahat) y||, rhat = D~ (D~ + L)^-1 r; sp.work[0] keeps the x before.  *spent receives
+// the operator applications of its steps.  False when the polynomial overflowed (x is unchanged).
+bool split_cycle(hipStream_t s, GmresWork<double>& w, const SplitCycles& sp, const double* r, double beta,
+                 double stop_rel, int max_steps, double* x, int* spent) {
     const CsrOp<double>& A = sp.Ahat;
     const int64_t n = A.n;
     double *r1 = sp.work[0], *rh = sp.work[1], *y = sp.work[2];
     scale_host<double>(s, n, r, 1.0 / beta, r1);
     split_op<double>(1, s, *A.co, A.F, A.L, *A.split, r1, rh, A.mode);
     const double bh = norm_of(s, w, n, rh);
-    if (!(bh > 0)) return 0;
+    *spent = 0;
+    if (!(bh > 0)) return false;
     PcFn<double> q;  // degree 1: q = 1
     if (sp.degree > 1)
         q = [&](hipStream_t st, const double* v, double* z) {
@@ -229,11 +230,11 @@ int split_cycle(hipStream_t s, GmresWork<double>& w, const SplitCycles& sp, cons
             }
         };
     double est = 0;
-    const int steps = gmres_cycle<double>(s, w, A, q, rh, bh, stop_rel * bh, max_steps, r1, &est);
-    if (!std::isfinite(est)) return 0;
+    *spent = sp.degree * gmres_cycle<double>(s, w, A, q, rh, bh, stop_rel * bh, max_steps, r1, &est);
+    if (!std::isfinite(est)) return false;
     split_op<double>(2, s, *A.co, A.F, A.L, *A.split, r1, y, A.mode);
-    axpy_f64(s, n, beta, y, x);
-    return steps * sp.degree;
+    axpy_f64_keep(s, n, beta, y, x, r1);
+    return true;
 }
 }  // namespace
 
@@ -256,24 +257,30 @@ SolveInfo gmres_solve(hipStream_t s, GmresWork<double>& w, const CsrOp<double>& 
             break;
         }
         if (info.iters >= maxit) break;
-        int steps = 0;
+        if (split.degree > maxit - info.iters) split.degree = 0;
         if (split.degree > 0) {
-            const int most = (maxit - info.iters) / split.degree;
+            int spent = 0;
+            const double before = beta;
             // the split residual's norm stands for ||b - A x||; their reductions lie close together
-            if (most > 0) steps = split_cycle(s, w, split, r, beta, 0.8 * tol * nb / beta, most, x);
+            const bool moved = split_cycle(s, w, split, r, beta, 0.8 * tol * nb / beta,
+                                           (maxit - info.iters) / split.degree, x, &spent);
+            info.iters += spent;
+            info.cycles += 1;
+            if (moved) beta = residual_norm(s, w, A, x, b, r);
+            // a spectrum the polynomial does not suit: plain cycles from here, and from the x before
+            // where the residual did not fall
+            if (!moved || !(beta < 0.5 * before)) split.degree = 0;
+            if (moved && !(beta < before)) {
+                copy_f64(s, A.n, split.work[0], x);
+                beta = residual_norm(s, w, A, x, b, r);
+            }
+            continue;
         }
-        const bool plain = steps == 0;
-        if (plain) {
-            double est = 0;
-            steps = gmres_cycle<double>(s, w, A, M, r, beta, tol * nb, maxit - info.iters, r, &est);
-            axpy_f64(s, A.n, 1.0, r, x);
-        }
-        info.iters += steps;
+        double est = 0;
+        info.iters += gmres_cycle<double>(s, w, A, M, r, beta, tol * nb, maxit - info.iters, r, &est);
+        axpy_f64(s, A.n, 1.0, r, x);
         info.cycles += 1;
-        const double before = beta;
         beta = residual_norm(s, w, A, x, b, r);
-        // a spectrum the polynomial does not suit: plain cycles from here
-        if (!plain && !(beta < 0.5 * before)) split.degree = 0;
     }
     return info;
 }

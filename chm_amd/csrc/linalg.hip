@@ -5,7 +5,7 @@
 // Jacobi and per-column tridiagonal preconditioners.
 //
 // Reductions are two-stage and deterministic: every block writes its partial
-// sums, then reduce_cols adds the partials in a fixed order.
+// sums, then one workgroup adds the partials in a fixed order.
 #include <initializer_list>
 
 #include "kernels.hpp"
@@ -923,6 +923,13 @@ __global__ void k_axpy_f64(int64_t n, double alpha, const double* x, double* y) 
     const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (k < n) y[k] = fma(alpha, x[k], y[k]);
 }
+__global__ void k_axpy_f64_keep(int64_t n, double alpha, const double* x, double* y, double* old) {
+    const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (k >= n) return;
+    const double yk = y[k];
+    old[k] = yk;
+    y[k] = fma(alpha, x[k], yk);
+}
 __global__ void k_copy_f64(int64_t n, const double* a, double* b) {
     const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (k < n) b[k] = a[k];
@@ -1107,6 +1114,9 @@ void axpy_dev_scaled_f32(hipStream_t s, int64_t n, const double* scale, const fl
 }
 void axpy_f64(hipStream_t s, int64_t n, double alpha, const double* x, double* y) {
     hipLaunchKernelGGL(k_axpy_f64, dim3(grid_for(n)), dim3(kBlock), 0, s, n, alpha, x, y);
+}
+void axpy_f64_keep(hipStream_t s, int64_t n, double alpha, const double* x, double* y, double* old) {
+    hipLaunchKernelGGL(k_axpy_f64_keep, dim3(grid_for(n)), dim3(kBlock), 0, s, n, alpha, x, y, old);
 }
 void copy_f64(hipStream_t s, int64_t n, const double* a, double* b) {
     hipLaunchKernelGGL(k_copy_f64, dim3(grid_for(n)), dim3(kBlock), 0, s, n, a, b);

@@ -140,3 +140,23 @@ def test_spectrum_that_the_polynomial_does_not_suit():
     assert st["susp_iters"] < 100 and st["susp_resid"] <= 1e-8
     assert _residual(ctx, o["conc"]) <= 1.01e-8
     ctx.close()
+
+
+def test_rejected_cycle_leaves_the_start_as_it_was():
+    """A polynomial cycle after which the residual is larger than before: plain cycles go on from the x
+    before it, so the whole solve takes that cycle's 30 steps of degree 10 and what plain cycles
+    take from the start (which a limit below 300 shows)."""
+    from chm_amd import pbsm3d as pb
+
+    print("[case] gmres rejected cycle", flush=True)
+    mesh = meshgen.synthetic_mesh(106000, seed=5)
+    g = pb.face_geometry(mesh)
+    fo = meshgen.forcing_c2(mesh.n_faces, seed=9)
+    iters = {}
+    for limit in (200, 1000):
+        ctx = pb.Context(g, pb.default_config(nLayer=10, snow_diffusion_const=-0.028, max_iters=limit))
+        o, st = ctx.step(fo, want_fields=True)
+        assert _residual(ctx, o["conc"]) <= 1.01e-8
+        iters[limit] = st["susp_iters"]
+        ctx.close()
+    assert iters[1000] == 300 + iters[200], iters
