@@ -434,6 +434,58 @@ SolveInfo solve_in_position_order(pbsm3d_ctx* c, const pbsm3d_config& cfg, int64
     return si;
 }
 
+// Deposition solve.  The 2-D system is symmetric positive definite (areas and the edge weights of a
+// graph Laplacian) and the D-ILU preconditioner keeps it so: conjugate gradients in the position
+// order (one layer) reach the target in as many iterations as GMRES(30) and two thirds of
+// BiCGStab's applications.  5,000 faces 0.50 ms with GMRES, now 0.33; 50,000 0.87 and 0.58;
+// 125,000 0.95 with BiCGStab, now 0.71; 999,968 5.3 and 3.7, now 3.0.
+// A smoothing coefficient may leave the system indefinite, and a tight max_iters may do for the
+// Krylov method of the configuration and not for CG: that method then solves it from the start.
+SolveInfo solve_deposition(pbsm3d_ctx* c, const pbsm3d_config& cfg) {
+    hipStream_t s = c->stream;
+    const int64_t F = c->F;
+    PcFn<double> M;
+    if (cfg.dep_precond == PBSM3D_PC_MCILU0) {
+        // the matrix depends on the mesh alone: one factorisation per context
+        if (!c->dep_factored)
+            dilu_factor<double>(s, c->co, F, 1, c->dep.rp.p, c->dep.val.p, c->slots.p, c->dl_d);
+        c->dep_factored = true;
+        double *b = c->dsplit[0].p, *x = c->dsplit[1].p;
+        CsrOp<double> Dp{F, nullptr, nullptr, nullptr, nullptr, F, 1};
+        Dp.co = &c->co;
+        Dp.pos = &c->dl_d;
+        CsrOp<double> Dh = Dp;
+        Dh.pos = nullptr;
+        Dh.split = &c->dl_d;
+        to_pos<double, double>(s, c->co, F, 1, c->dep.rhs.p, b);
+        if (!c->dep_indefinite) {
+            to_pos<double, double>(s, c->co, F, 1, c->dep.x.p, x);
+            const SolveInfo si = cg_split(s, c->cgd, c->wd64, Dp, Dh, b, x, c->r_d.p, cfg.max_iters, cfg.tol);
+            if (si.converged) {
+                from_pos<double, double>(s, c->co, F, 1, x, c->dep.x.p);
+                return si;
+            }
+            c->dep_indefinite = si.breakdown;  // no CG in the steps to come
+        }
+        if (cfg.krylov == PBSM3D_KRYLOV_BICGSTAB_SPLIT) {
+            to_pos<double, double>(s, c->co, F, 1, c->dep.x.p, x);
+            const SolveInfo si = bicgstab_split<double>(s, c->bwd64, c->wd64, Dp, Dh, b, x, c->r_d.p, c->dsplit[2].p,
+                                                        c->dsplit[3].p, c->dsplit[4].p, cfg.max_iters, cfg.tol, 0.0);
+            from_pos<double, double>(s, c->co, F, 1, x, c->dep.x.p);
+            return si;
+        }
+        M = [c, F](hipStream_t st, const double* r, double* z) { dilu_apply<double>(st, c->co, F, 1, c->dl_d, r, z); };
+    } else if (cfg.dep_precond == PBSM3D_PC_JACOBI) {
+        M = [c, F](hipStream_t st, const double* r, double* z) { pc_jacobi<double>(st, F, c->invdiag_d.p, r, z); };
+    } else {
+        M = [F](hipStream_t st, const double* r, double* z) {
+            PB_HIP(hipMemcpyAsync(z, r, F * sizeof(double), hipMemcpyDeviceToDevice, st));
+        };
+    }
+    const CsrOp<double> D{F, c->dep.rp.p, c->dep.col.p, c->dep.val.p};
+    return gmres_solve(s, c->wd64, D, M, c->dep.rhs.p, c->dep.x.p, c->r_d.p, cfg.restart, cfg.max_iters, cfg.tol);
+}
+
 }  // namespace
 
 extern "C" {
@@ -801,53 +853,7 @@ int pbsm3d_step(pbsm3d_ctx* c, const pbsm3d_forcing* fo, int32_t dt_s, pbsm3d_ou
 
         // ---- deposition solve + drift (PBSM3D.cpp:1661-1740)
         if (stats.deposition_present) {
-            CsrOp<double> D{F, c->dep.rp.p, c->dep.col.p, c->dep.val.p};
-            PcFn<double> M;
-            SolveInfo si;
-            int before = 0;
-            if (cfg.dep_precond == PBSM3D_PC_MCILU0 && split_fits(F, 1)) {
-                // The 2-D system is symmetric positive definite (areas and the edge weights of a graph
-                // Laplacian) and the same preconditioner keeps it so: conjugate gradients in the
-                // position order (one layer) reach the target in as many iterations as GMRES(30)
-                // and two thirds of BiCGStab's applications.  5,000 faces 0.50 ms with GMRES, now 0.33;
-                // 50,000 0.87 and 0.58; 125,000 0.95 with BiCGStab, now 0.71; 999,968 5.3 and 3.7, now 3.0.
-                // The matrix (areas and edge weights) depends on the mesh alone: one factorisation per context.
-                if (!c->dep_factored)
-                    dilu_factor<double>(s, c->co, F, 1, c->dep.rp.p, c->dep.val.p, c->slots.p, c->dl_d);
-                c->dep_factored = true;
-                to_pos<double, double>(s, c->co, F, 1, c->dep.rhs.p, c->dsplit[0].p);
-                to_pos<double, double>(s, c->co, F, 1, c->dep.x.p, c->dsplit[1].p);
-                CsrOp<double> Dp{F, nullptr, nullptr, nullptr, nullptr, F, 1};
-                Dp.co = &c->co;
-                Dp.pos = &c->dl_d;
-                CsrOp<double> Dh = Dp;
-                Dh.pos = nullptr;
-                Dh.split = &c->dl_d;
-                si = cg_split(s, c->cgd, c->wd64, Dp, Dh, c->dsplit[0].p, c->dsplit[1].p, c->r_d.p, cfg.max_iters,
-                              cfg.tol);
-                before = si.iters;
-                if (si.converged) from_pos<double, double>(s, c->co, F, 1, c->dsplit[1].p, c->dep.x.p);
-            }
-            if (!si.converged) {  // no D-ILU, or a smoothing coefficient that leaves the system indefinite
-                if (cfg.dep_precond == PBSM3D_PC_MCILU0) {
-                    if (!c->dep_factored)
-                        dilu_factor<double>(s, c->co, F, 1, c->dep.rp.p, c->dep.val.p, c->slots.p, c->dl_d);
-                    M = [c, F](hipStream_t st2, const double* r, double* z) {
-                        dilu_apply<double>(st2, c->co, F, 1, c->dl_d, r, z);
-                    };
-                } else if (cfg.dep_precond == PBSM3D_PC_JACOBI) {
-                    M = [c, F](hipStream_t st2, const double* r, double* z) {
-                        pc_jacobi<double>(st2, F, c->invdiag_d.p, r, z);
-                    };
-                } else {
-                    M = [F](hipStream_t st2, const double* r, double* z) {
-                        PB_HIP(hipMemcpyAsync(z, r, F * sizeof(double), hipMemcpyDeviceToDevice, st2));
-                    };
-                }
-                si = gmres_solve(s, c->wd64, D, M, c->dep.rhs.p, c->dep.x.p, c->r_d.p, cfg.restart, cfg.max_iters,
-                                 cfg.tol);
-                si.iters += before;
-            }
+            const SolveInfo si = solve_deposition(c, cfg);
             stats.dep_iters = si.iters;
             stats.dep_resid = si.resid;
             if (!si.converged) throw Error(PBSM3D_ENOCONV, "deposition solver failed to converge");

@@ -47,14 +47,16 @@ struct pbsm3d_ctx {
     pb::ColumnFactors colf;
     pb::ColorOrder co;
     pb::DiluFactors<double> dl_s, dl_d;
-    bool dep_factored = false;  // dl_d holds the deposition system's factors (a context, not a batch)
+    bool dep_factored = false;    // dl_d holds the deposition system's factors (a context, not a batch)
+    bool dep_indefinite = false;  // CG broke down on it
     pb::DiluFactors<float> dl32;
     pb::DevBuf<double> invdiag_s, invdiag_d, r_s, r_d;
     pb::DevBuf<double> bp, xp;  // suspension b and x in the D-ILU position order
     pb::DevBuf<double> split64[3];  // work vectors of the split BiCGStab (FP64 / MIXED)
     pb::DevBuf<float> split32[3];
-    pb::DevBuf<double> dsplit[5];  // deposition b, x (position order); a batch's BiCGStab work vectors
+    pb::DevBuf<double> dsplit[5];  // deposition b, x (position order); split BiCGStab's work vectors
     pb::CgWork cgd;                // deposition CG workspace
+    pb::BicgWork<double> bwd64;    // deposition BiCGStab workspace, laid out when CG does not finish
     // position-order SpMV launch shape per precision (index 0: FP64, 1: FP32), -1 until tuned
     int spmv_variant[2] = {-1, -1};
     float spmv_tune_ms[2][pb::kPosSpmvVariants] = {};

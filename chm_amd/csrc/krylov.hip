@@ -596,7 +596,10 @@ SolveInfo cg_split(hipStream_t s, CgWork& w, GmresWork<double>& gw, const CsrOp<
                 break;
             }
         }
-        if (stop == 2.0) return info;  // x keeps what the runs before gained
+        if (stop == 2.0) {  // x keeps what the runs before gained
+            info.breakdown = std::isfinite(info.resid);  // else the start or b is at fault
+            return info;
+        }
         split_op<double>(2, s, *Ahat.co, Ahat.F, Ahat.L, *Ahat.split, w.xh.p, w.work.p, Ahat.mode);
         axpy_f64(s, n, beta, w.work.p, x);
         info.cycles += 1;

@@ -79,6 +79,7 @@ struct SolveInfo {
     bool cold_fallback = false;  // the initial guess was worse than x0 = 0 and was dropped
     double resid_coarse = 0;     // ||b - A x|| / ||b|| after the first coarse correction (0: none)
     int restarts = 0;            // shadow-residual restarts of the FP32 BiCGStab runs
+    bool breakdown = false;      // CG: the matrix is not positive definite
 };
 
 // Device workspace of one GMRES instance of storage type T.
@@ -151,8 +152,8 @@ SolveInfo bicgstab_solve(hipStream_t s, BicgWork<double>& w, GmresWork<double>& 
                          const PcFn<double>& M, const double* b, double* x, int maxit, double tol);
 // Conjugate gradients with the D-ILU preconditioner on its split operator, for a symmetric
 // positive definite A: one operator application per iteration (7 launches) where BiCGStab takes two (14) and
-// GMRES orthogonalises against its basis.  r receives the residual.  Not converged on a
-// breakdown (A is not positive definite) or a run that gains nothing.
+// GMRES orthogonalises against its basis.  r receives the residual.  Not converged after maxit
+// iterations, on a breakdown (A is not positive definite) or after a run that gains nothing.
 struct CgWork {
     int64_t n = 0;
     DevBuf<double> rh, p, pw, q, xh, work;  // work: n + 1 entries, entry n zero

@@ -137,8 +137,10 @@ typedef struct pbsm3d_config {
 } pbsm3d_config;
 
 /* Krylov method of the suspension solve.  The deposition system is symmetric positive definite: with
- * dep_precond MCILU0 it is solved by conjugate gradients, else (and if it turns out indefinite)
- * by GMRES(restart). */
+ * dep_precond MCILU0 a context solves it by conjugate gradients.  Without MCILU0, and where conjugate
+ * gradients do not finish (the system is indefinite, or max_iters too small for them), by
+ * GMRES(restart), or with KRYLOV_BICGSTAB_SPLIT and MCILU0 by split BiCGStab, as a batch always
+ * does.  dep_iters counts the iterations of the method that finished. */
 #define PBSM3D_KRYLOV_GMRES 0     /* restarted GMRES(restart), as Belos "GMRES"     */
 #define PBSM3D_KRYLOV_BICGSTAB 1  /* BiCGStab: short recurrences, 2 SpMV/iteration  */
 #define PBSM3D_KRYLOV_BICGSTAB_SPLIT 2  /* BiCGStab on the split D-ILU system (Eisenstat's

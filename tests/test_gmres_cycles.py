@@ -160,3 +160,63 @@ def test_rejected_cycle_leaves_the_start_as_it_was():
         iters[limit] = st["susp_iters"]
         ctx.close()
     assert iters[1000] == 300 + iters[200], iters
+
+
+@pytest.mark.parametrize("points,smooth,krylov", [
+    (18, -820.0, abi.KRYLOV_GMRES), (18, -820.0, abi.KRYLOV_BICGSTAB_SPLIT), (18, -1.0e4, abi.KRYLOV_GMRES),
+    (18, -1.0e4, abi.KRYLOV_BICGSTAB), (18, -1.0e4, abi.KRYLOV_BICGSTAB_SPLIT), (60, -300.0, abi.KRYLOV_GMRES),
+    (60, -820.0, abi.KRYLOV_BICGSTAB_SPLIT), (60, -2.0e3, abi.KRYLOV_BICGSTAB_SPLIT)])
+def test_indefinite_deposition_system(points, smooth, krylov):
+    """A negative smoothing coefficient that leaves an indefinite system, on which conjugate gradients
+    break down: the configuration's own method solves it, in the first step and in the next one (which
+    does not try them again), to the solution of the dense system."""
+    from chm_amd import pbsm3d as pb
+
+    print(f"[case] indefinite deposition points={points} smooth={smooth} krylov={krylov}", flush=True)
+    mesh = meshgen.synthetic_mesh(points, seed=8, extent=1.0e3)
+    g = pb.face_geometry(mesh)
+    fo = meshgen.forcing_c2(mesh.n_faces, seed=4)
+    iters = set()
+    ctx = pb.Context(g, pb.default_config(nLayer=5, tol=1e-12, smooth_coeff=smooth, krylov=krylov, max_iters=600))
+    for _ in range(2):
+        ctx.set_state(np.zeros(mesh.n_faces), np.zeros(mesh.n_faces))
+        o, st = ctx.step(fo, want_fields=True)
+        rp, col, val, b = ctx.system(1)
+        A = np.zeros((b.size, b.size))
+        A[np.repeat(np.arange(b.size), np.diff(rp)), col] = val
+        assert np.linalg.eigvalsh(A).min() < 0 < np.linalg.eigvalsh(A).max()
+        want = np.linalg.solve(A, b)
+        # relative residual 1e-12: the error is at most cond(A) times that
+        assert st["dep_resid"] <= 1e-12
+        assert np.linalg.norm(o["qdep"] - want) <= 1e-12 * np.linalg.cond(A) * np.linalg.norm(want)
+        iters.add(st["dep_iters"])
+    ctx.close()
+    assert len(iters) == 1, iters
+
+
+def test_deposition_limit_that_the_configured_method_meets(oracle):
+    """max_iters bounds the deposition solve by the configuration's own method: a limit that GMRES(30), or
+    split BiCGStab (which a batch runs), meets and conjugate gradients do not is met, and no more
+    iterations than it are reported."""
+    from chm_amd import pbsm3d as pb
+
+    print("[case] deposition limit", flush=True)
+    mesh = meshgen.synthetic_mesh(2500, seed=8)
+    g = pb.face_geometry(mesh)
+    fo = meshgen.forcing_c2(mesh.n_faces, seed=4)
+    kw = dict(nLayer=5, settling_scale=30.0, smooth_coeff=1.0e5)  # few suspension, many deposition iterations
+    orc = oracle.Oracle(g, oracle.oracle_config(precond=abi.PC_MCILU0, dep_precond=abi.PC_MCILU0, **kw))
+    _, ost = orc.step(fo)
+    batch = pb.Batch([g], [pb.default_config(krylov=abi.KRYLOV_BICGSTAB_SPLIT, **kw)])
+    _, bst = batch.step([fo])
+    batch.close()
+    for krylov, limit in ((abi.KRYLOV_GMRES, ost["dep_iters"] + 1), (abi.KRYLOV_BICGSTAB_SPLIT, bst[0]["dep_iters"] + 1)):
+        free = pb.Context(g, pb.default_config(krylov=krylov, **kw))
+        fout, fst = free.step(fo, want_fields=True)
+        assert fst["dep_iters"] > limit  # conjugate gradients need more
+        ctx = pb.Context(g, pb.default_config(krylov=krylov, max_iters=limit, **kw))
+        o, st = ctx.step(fo, want_fields=True)
+        assert st["dep_iters"] <= limit and st["dep_resid"] <= 1e-8, st
+        assert rel_err(o["qdep"], fout["qdep"]) < 1e-6
+        ctx.close()
+        free.close()
