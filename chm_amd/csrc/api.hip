@@ -312,10 +312,17 @@ static SplitCycles split_cycles(pbsm3d_ctx* c) {
         (void)hipGetLastError();
         return SplitCycles{};
     }
-    // among the column modes only: GMRES on the same system gives the same bits in every context
-    if (c->split_mode < 0)
-        c->split_mode = tune_split_mode<double>(c->stream, c->co, c->F, c->L, c->dl_s, c->bp.p, c->split64[0].p,
-                                                nullptr, kColumnModes);
+    // Among the column modes only: GMRES on the same system gives the same bits in every context.
+    // Bit 0 is the one that pbsm3d_precond_select fixes and the plain cycles' sweeps share.
+    if (c->dilu_mode[0] < 0) {
+        float ms[kColumnModes];
+        c->split_mode = tune_split_mode<double>(c->stream, c->co, c->F, c->L, c->dl_s, c->bp.p, c->split64[0].p, ms,
+                                                kColumnModes);
+        c->dilu_mode[0] = c->split_mode & 1;
+        for (int m = 0; m < 2; ++m) c->dilu_tune_ms[0][m] = std::min(ms[m], ms[m + 2]);  // bit 1: loads
+    } else if (c->split_mode < 0 || (c->split_mode & 1) != c->dilu_mode[0]) {
+        c->split_mode = c->dilu_mode[0];
+    }
     SplitCycles sp{CsrOp<double>{N, nullptr, nullptr, nullptr, &c->prof, c->F, c->L}, {}, neumann_degree(N)};
     sp.Ahat.co = &c->co;
     sp.Ahat.split = &c->dl_s;
@@ -334,6 +341,7 @@ SolveInfo solve_in_position_order(pbsm3d_ctx* c, const pbsm3d_config& cfg, int64
     hipStream_t s = c->stream;
     const int64_t N = F * L;
     const bool bicg = cfg.krylov == PBSM3D_KRYLOV_BICGSTAB;
+    SplitCycles split;  // of FP64 GMRES
     {
         ProfScope ps(&c->prof, s, PBSM3D_K_FACTOR);
         dilu_factor<double>(s, c->co, F, L, c->susp.rp.p, c->susp.val.p, c->slots.p, c->dl_s);
@@ -355,6 +363,7 @@ SolveInfo solve_in_position_order(pbsm3d_ctx* c, const pbsm3d_config& cfg, int64
                                                      c->dilu_tune_ms[1]);
         }
     } else {
+        if (cfg.precision == PBSM3D_FP64 && !bicg) split = split_cycles(c);
         if (cfg.precision == PBSM3D_FP64 && c->dilu_mode[0] < 0)
             c->dilu_mode[0] = tune_dilu_xcd<double>(s, c->co, F, L, c->dl_s, c->bp.p, c->r_s.p, c->dilu_tune_ms[0]);
         if (cfg.precision == PBSM3D_MIXED && c->dilu_mode[1] < 0)
@@ -401,7 +410,6 @@ SolveInfo solve_in_position_order(pbsm3d_ctx* c, const pbsm3d_config& cfg, int64
         if (bicg) {
             si = bicgstab_solve(s, c->bw64, c->ws64, A, M, c->bp.p, c->xp.p, cfg.max_iters, cfg.tol);
         } else {
-            const SplitCycles split = split_cycles(c);
             auto gmres = [&](const SplitCycles& sp) {
                 return gmres_solve(s, c->ws64, A, M, c->bp.p, c->xp.p, c->r_s.p, cfg.restart, cfg.max_iters, cfg.tol, sp);
             };

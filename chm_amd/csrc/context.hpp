@@ -64,7 +64,7 @@ struct pbsm3d_ctx {
     // D-ILU sweep mode per precision: bit 0 the XCD workgroup mapping, bit 1 (split
     // operator only) the non-temporal factor loads; -1 until tuned
     int dilu_mode[2] = {-1, -1};
-    int split_mode = -1;  // the same for the split sweeps of FP64 GMRES
+    int split_mode = -1;  // of the split sweeps of FP64 GMRES: bit 0 as dilu_mode[0], bit 1 its own
     // shadow-residual restart threshold of the FP32 BiCGStab runs (bicg_stage; 0: never)
     double restart_eps32 = pb::kBicgRestartEps32;
     float dilu_tune_ms[2][pb::kSplitModes] = {};

@@ -291,7 +291,8 @@ int pbsm3d_spmv_select(pbsm3d_ctx* ctx, int which, int variant);
  * (PBSM3D_KRYLOV_BICGSTAB_SPLIT) also bit 1 = the factor arrays read with the
  * non-temporal hint and bit 2 = layer-parallel sweeps (a workgroup per 64 face
  * columns, one wave per layer, the vertical recurrence from LDS) instead of one
- * thread per column; the other solvers tune bit 0 alone.
+ * thread per column; the other solvers report bit 0 alone (FP64 GMRES with nLayer <= 16
+ * that of the split sweeps its cycles run, whose results do not depend on it).
  * ms[PBSM3D_PRECOND_MODES] = average apply time of each mode (ms; 0 if not
  * tried).  pbsm3d_precond_select fixes the mode (0 .. 1, or 0 .. 7 with the
  * split operator) or re-tunes (-1). */

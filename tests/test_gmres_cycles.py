@@ -220,3 +220,34 @@ def test_deposition_limit_that_the_configured_method_meets(oracle):
         assert rel_err(o["qdep"], fout["qdep"]) < 1e-6
         ctx.close()
         free.close()
+
+
+def test_sweep_mode_of_the_split_cycles():
+    """pbsm3d_precond_select(0, ..) fixes the workgroup mapping of the split sweeps that FP64 GMRES runs,
+    pbsm3d_precond_tuning(0) reports the tuner's choice of it and the times of both; the fields are
+    the same bit for bit, and the split BiCGStab's other modes stay refused."""
+    from chm_amd import pbsm3d as pb
+
+    print("[case] gmres sweep mode", flush=True)
+    mesh = meshgen.synthetic_mesh(6000, seed=5)
+    g = pb.face_geometry(mesh)
+    fo = meshgen.forcing_c2(mesh.n_faces, seed=9)
+    ctx = pb.Context(g, pb.default_config(nLayer=9))
+    outs = []
+    for mode in (None, 0, 1, -1):
+        if mode is not None:
+            ctx.precond_select(0, mode)
+        ctx.set_state(np.zeros(mesh.n_faces), np.zeros(mesh.n_faces))
+        o, st = ctx.step(fo, want_fields=True)
+        outs.append((st["susp_iters"], o))
+        tun = ctx.precond_tuning(0)
+        assert tun["mode"] == mode if mode in (0, 1) else tun["mode"] in (0, 1), (mode, tun)
+        assert all(ms > 0 for ms in tun["ms"][:2]) and all(ms == 0 for ms in tun["ms"][2:]), tun
+    for it, o in outs[1:]:
+        assert it == outs[0][0]
+        for k in ("conc", "qdep"):
+            np.testing.assert_array_equal(o[k], outs[0][1][k])
+    for mode in (2, 3):
+        with pytest.raises(pb.Pbsm3dError):
+            ctx.precond_select(0, mode)
+    ctx.close()
