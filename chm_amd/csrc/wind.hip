@@ -124,7 +124,6 @@ template <bool CHECKED>
 __device__ __forceinline__ int tps_sites(int64_t F, int64_t i, const int32_t* neigh, int64_t sf, int64_t sj,
                                          const double* cx, const double* cy, int32_t nb[3], double sx[3],
                                          double sy[3], double* bad) {
-    int n = 0;
 #pragma unroll
     for (int j = 0; j < 3; ++j) {
         nb[j] = neigh[i * sf + j * sj];
@@ -132,80 +131,111 @@ __device__ __forceinline__ int tps_sites(int64_t F, int64_t i, const int32_t* ne
             *bad = 1.0;
             nb[j] = -1;
         }
-        if (nb[j] < 0) continue;
-        sx[n] = cx[nb[j]];
-        sy[n] = cy[nb[j]];
-        ++n;
+        sx[j] = cx[nb[j] < 0 ? i : nb[j]];
+        sy[j] = cy[nb[j] < 0 ? i : nb[j]];
     }
-    return n;
+    // the existing ones to the front, without an index that only the lane knows: such an array
+    // lies in scratch memory
+    const bool h0 = nb[0] >= 0, h1 = nb[1] >= 0, h2 = nb[2] >= 0;
+    if (!h1) {
+        sx[1] = sx[2];
+        sy[1] = sy[2];
+    }
+    if (!h0) {
+        sx[0] = sx[1];
+        sy[0] = sy[1];
+        sx[1] = sx[2];
+        sy[1] = sy[2];
+    }
+    return h0 + h1 + h2;
 }
 
 // The spline's value at (x, y) is linear in the sites' winds, and both the system and the basis
 // depend on the mesh alone.  It reproduces constants, so the weights add up to one and the
 // value is p1 + w2 (p2 - p1) + w3 (p3 - p1) over the sites in order; this form keeps the
-// weights' rounding off the common part of the winds.  w[0] = w2 and w[1] = w3 (0 where there
-// is no such site): the values for a unit wind at that site, from the (n + 1) x (n + 1) system by
-// Gaussian elimination with partial pivoting.
-__device__ __forceinline__ void tps_weights(int n, const double sx[3], const double sy[3], double x, double y,
-                                            double w[2]) {
-    w[0] = w[1] = 0;
-    if (n < 2) return;
-    const int m = n + 1;
-    double A[4][6];
+// weights' rounding off the common part of the winds.  w[0] = w2 and w[1] = w3: the values for a
+// unit wind at that site, from the (N + 1) x (N + 1) system by Gaussian elimination with partial
+// pivoting, unrolled so that the system stays in registers.
+template <int N>
+__device__ __forceinline__ void tps_weights_of(const double sx[3], const double sy[3], double x, double y, double w[2]) {
+    constexpr int M = N + 1, Q = N - 1;  // unknowns, right-hand sides
+    double A[M][M + Q];
 #pragma unroll
-    for (int r = 0; r < 4; ++r)
+    for (int r = 0; r < M; ++r)
 #pragma unroll
-        for (int cc = 0; cc < 6; ++cc) A[r][cc] = 0;
-    for (int r = 0; r < n; ++r)
-        for (int j = r; j < n; ++j) {
+        for (int cc = 0; cc < M + Q; ++cc)
+            A[r][cc] = cc >= M ? (r == cc - M + 1 ? 1.0 : 0.0) : cc == 0 ? (r < N ? 1.0 : 0.0) : r == N ? 1.0 : 0.0;
+#pragma unroll
+    for (int r = 0; r < N; ++r)
+#pragma unroll
+        for (int j = r + 1; j < N; ++j) {
             const double xdiff = sx[r] - sx[j], ydiff = sy[r] - sy[j];
             if (xdiff == 0. && ydiff == 0.) continue;
             const double Rd = tps_basis(sx[r], sy[r], sx[j], sy[j]);
             A[r][j + 1] = Rd;
             A[j][r + 1] = Rd;
         }
-    for (int r = 0; r < m; ++r) {
-        A[r][0] = 1;
-        A[m - 1][r] = 1;
-    }
-    A[m - 1][0] = 0;
-    for (int q = 0; q < 2; ++q)
-        for (int r = 0; r < m; ++r) A[r][m + q] = r == q + 1 && r < n ? 1.0 : 0.0;
-    for (int k = 0; k < m; ++k) {
+#pragma unroll
+    for (int k = 0; k < M; ++k) {
         int p = k;
-        for (int r = k + 1; r < m; ++r)
-            if (fabs(A[r][k]) > fabs(A[p][k])) p = r;
-        if (p != k)
-            for (int cc = 0; cc < m + 2; ++cc) {
-                const double t = A[k][cc];
-                A[k][cc] = A[p][cc];
-                A[p][cc] = t;
+        double big = fabs(A[k][k]);
+#pragma unroll
+        for (int r = k + 1; r < M; ++r)
+            if (fabs(A[r][k]) > big) {
+                big = fabs(A[r][k]);
+                p = r;
             }
-        for (int r = k + 1; r < m; ++r) {
+#pragma unroll
+        for (int r = k + 1; r < M; ++r)
+#pragma unroll
+            for (int cc = k; cc < M + Q; ++cc) {
+                const double t = A[k][cc], u = A[r][cc];
+                A[k][cc] = p == r ? u : t;
+                A[r][cc] = p == r ? t : u;
+            }
+#pragma unroll
+        for (int r = k + 1; r < M; ++r) {
             const double f = A[r][k] / A[k][k];
-            for (int cc = k; cc < m + 2; ++cc) A[r][cc] -= f * A[k][cc];
+#pragma unroll
+            for (int cc = k + 1; cc < M + Q; ++cc) A[r][cc] -= f * A[k][cc];
         }
     }
-    double c[2][4];
-    for (int q = 0; q < 2; ++q)
-        for (int k = m - 1; k >= 0; --k) {
-            double s = A[k][m + q];
-            for (int cc = k + 1; cc < m; ++cc) s -= A[k][cc] * c[q][cc];
+    double c[Q][M];
+#pragma unroll
+    for (int q = 0; q < Q; ++q)
+#pragma unroll
+        for (int k = M - 1; k >= 0; --k) {
+            double s = A[k][M + q];
+#pragma unroll
+            for (int cc = k + 1; cc < M; ++cc) s -= A[k][cc] * c[q][cc];
             c[q][k] = s / A[k][k];
         }
-    for (int r = 1; r < m; ++r) {
+#pragma unroll
+    for (int q = 0; q < Q; ++q) w[q] = c[q][0];
+#pragma unroll
+    for (int r = 1; r < M; ++r) {
         const double b = tps_basis(sx[r - 1], sy[r - 1], x, y);
-        for (int q = 0; q < n - 1; ++q) w[q] = (r == 1 ? c[q][0] : w[q]) + c[q][r] * b;
+#pragma unroll
+        for (int q = 0; q < Q; ++q) w[q] = w[q] + c[q][r] * b;
     }
 }
+// w[0] and w[1] of n sites (0 where there is no such site)
+__device__ __forceinline__ void tps_weights(int n, const double sx[3], const double sy[3], double x, double y,
+                                            double w[2]) {
+    w[0] = w[1] = 0;
+    if (n == 3) tps_weights_of<3>(sx, sy, x, y, w);
+    if (n == 2) tps_weights_of<2>(sx, sy, x, y, w);
+    // The value is the site's wind plus 0 times its basis, which is NaN (the floor) at the site itself.
+    if (n == 1) w[0] = 0 * tps_basis(sx[0], sy[0], x, y);
+}
 
-// The smoothed wind of a face whose neighbours have the winds p[j]; where there is none
-// (nb[j] < 0), p[j] is the face's own.
-__device__ __forceinline__ double smoothed(const int32_t nb[3], const double p[3], double w2, double w3) {
+// The smoothed wind of a face whose neighbours have the winds a, b and c; where there is none
+// (nb[j] < 0), it is the face's own.
+__device__ __forceinline__ double smoothed(const int32_t nb[3], double a, double b, double c, double w2, double w3) {
     const bool h0 = nb[0] >= 0, h1 = nb[1] >= 0, h2 = nb[2] >= 0;
-    const double p1 = h0 ? p[0] : h1 ? p[1] : p[2];
-    const double d2 = h0 ? (h1 ? p[1] - p1 : h2 ? p[2] - p1 : 0.0) : (h1 && h2 ? p[2] - p1 : 0.0);
-    const double d3 = h0 && h1 && h2 ? p[2] - p1 : 0.0;
+    const double p1 = h0 ? a : h1 ? b : c;
+    const double d2 = h0 ? (h1 ? b - p1 : h2 ? c - p1 : 0.0) : (h1 && h2 ? c - p1 : 0.0);
+    const double d3 = h0 && h1 && h2 ? c - p1 : 0.0;
     double z = p1 + (w2 * d2 + w3 * d3);
     // an infinite neighbour makes NaN, and so the floor, as solving the system with it does
     if ((h0 || h1 || h2) && isinf(z)) z = NAN;
@@ -213,7 +243,9 @@ __device__ __forceinline__ double smoothed(const int32_t nb[3], const double p[3
 }
 
 // Smoothing from the caller's own geometry arrays (pbsm3d_wind_run_noalloc, which keeps nothing
-// between calls): the weights are formed on every call.
+// between calls): the weights are formed on every call.  A whole call on 399,968 faces takes 109 us,
+// 100 of them launches, the wait and the flag's copy; 154 us with one right-hand side (the winds)
+// and 182 with the weights' two when the system lay in scratch memory.
 __global__ void __launch_bounds__(kBlock) k_smooth_checked(int64_t F, const int32_t* __restrict__ neigh,
                                                            const double* __restrict__ cx,
                                                            const double* __restrict__ cy,
@@ -227,7 +259,7 @@ __global__ void __launch_bounds__(kBlock) k_smooth_checked(int64_t F, const int3
 #pragma unroll
     for (int j = 0; j < 3; ++j) p[j] = pt[nb[j] < 0 ? i : nb[j]];
     tps_weights(n, sx, sy, cx[i], cy[i], w);
-    out[i] = smoothed(nb, p, w[0], w[1]);
+    out[i] = smoothed(nb, p[0], p[1], p[2], w[0], w[1]);
 }
 
 // The weights of every face: w[i] = w2, w[F + i] = w3.
@@ -246,7 +278,7 @@ __global__ void __launch_bounds__(kBlock) k_weights(int64_t F, const int32_t* __
 
 // Smoothing with the context's weights: three gathers and two products per face, bound by
 // the gathers (12 B of indices, 16 B of weights, 24 B gathered, 8 B out per face).  Solving the
-// spline per call took six E1 series per face: 999,968 faces, both kernels, 262 us, now 33 us.
+// spline per call took six E1 series per face: 999,968 faces, both kernels, 262 us, now 32 us.
 __global__ void __launch_bounds__(kBlock) k_smooth(int64_t F, const int32_t* __restrict__ neigh,
                                                    const double* __restrict__ w, const double* __restrict__ pt,
                                                    double* __restrict__ out) {
@@ -259,7 +291,7 @@ __global__ void __launch_bounds__(kBlock) k_smooth(int64_t F, const int32_t* __r
     const double w2 = w[i], w3 = w[F + i];
 #pragma unroll
     for (int j = 0; j < 3; ++j) p[j] = pt[nb[j] < 0 ? i : nb[j]];
-    out[i] = smoothed(nb, p, w2, w3);
+    out[i] = smoothed(nb, p[0], p[1], p[2], w2, w3);
 }
 
 }  // namespace

@@ -169,6 +169,37 @@ def test_gpu_wind_weights_edges(pb, oracle, points):
 
 
 @pytest.mark.gpu
+def test_gpu_wind_face_at_its_neighbour(pb, oracle):
+    """A face whose centroid is one of its neighbours' (one, two and three of them): the spline's basis
+    is not a number there, and the face gets the 0.1 floor, with and without a context."""
+    import torch
+
+    print("[case] wind coincident centroids", flush=True)
+    mesh = meshgen.synthetic_mesh(300, seed=4, extent=3000.0)
+    F = mesh.n_faces
+    cx, cy = _centroids(mesh)
+    nb = mesh.neigh.copy()
+    for i, keep in ((10, 1), (120, 2), (230, 3)):  # faces far apart, with three neighbours in the mesh
+        assert (nb[i] >= 0).all()
+        cx[i], cy[i] = cx[nb[i, 2]], cy[nb[i, 2]]
+        nb[i, :3 - keep] = -1
+    U_R = meshgen.forcing_c2(F, seed=2)["U_R"]
+    sd = np.full(F, 0.4)
+    want = oracle.scale_wind(nb, cx, cy, None, None, _cfg(), U_R, sd)
+    assert (want[[10, 120, 230]] == 0.1).all()
+    w = pb.Wind(nb, cx, cy, None, None, _cfg())
+    np.testing.assert_allclose(w.run(U_R, sd), want, rtol=1e-12, atol=0)
+    w.close()
+
+    def dev(a, dtype=torch.float64):
+        return torch.tensor(a, dtype=dtype, device="cuda:0")
+
+    out = torch.zeros(F, dtype=torch.float64, device="cuda:0")
+    pb.wind_run_noalloc(dev(nb, torch.int32), dev(cx), dev(cy), dev(U_R), out, snowdepthavg=dev(sd), cfg=_cfg())
+    np.testing.assert_allclose(out.cpu().numpy(), want, rtol=1e-12, atol=0)
+
+
+@pytest.mark.gpu
 def test_gpu_chain_wind_fetch_step(pb, oracle, mesh_c1):
     """U_R -> scale_wind_vert -> U_2m_above_srf and vw_dir -> fetchr -> fetch, both on
     device arrays, feeding the PBSM3D step: the same fields as the oracle chain."""
