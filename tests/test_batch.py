@@ -84,6 +84,31 @@ def test_batch_tiny_members_straddle_tiles(precision):
                 assert rel_err(got[k][f], want[f]) < 1e-8, (step, k, f, rel_err(got[k][f], want[f]))
 
 
+@pytest.mark.parametrize("precision", [abi.FP64, abi.MIXED])
+def test_batch_guarded_layer_counts(precision):
+    """Ragged members with the layer counts that the split sweeps guard (3 below their bound of 5, 11, 13
+    and 15 below 16) and one union of two: equal to the members' own contexts."""
+    from chm_amd import pbsm3d as pb
+
+    print(f"[case] batch guarded layers precision={precision}", flush=True)
+    shape = ((300, 3), (1203, 11), (77, 13), (640, 13), (2001, 15))
+    members = [ensemble.Member(seed=3000 + k, n_points=n, n_layer=L, z0=0.01, settling_scale=1.0, wind_scale=1.0)
+               for k, (n, L) in enumerate(shape)]
+    meshes = [meshgen.synthetic_mesh(m.n_points, seed=m.seed) for m in members]
+    b = ensemble.build_batch(members, meshes, precision=precision, tol=1e-12)
+    assert b.info()["unions"] == 4
+    fos = [ensemble.member_forcing(mesh, m, 0) for m, mesh in zip(members, meshes)]
+    got, st = b.step(fos, want_fields=True)
+    for k, (m, mesh, fo) in enumerate(zip(members, meshes, fos)):
+        ctx = pb.Context(pb.face_geometry(mesh), ensemble.member_config(m, precision, tol=1e-12))
+        want, wst = ctx.step(fo, want_fields=True)
+        assert wst["suspension_present"] == 1 and st[k]["susp_resid"] <= 1e-12 and st[k]["dep_resid"] <= 1e-12
+        for f in ("conc", "Qsusp", "Qsubl", "qdep", "drift_mass"):
+            assert rel_err(got[k][f], want[f]) < 1e-8, (k, f, rel_err(got[k][f], want[f]))
+        ctx.close()
+    b.close()
+
+
 def test_batch_member_without_suspension():
     """A calm member (no suspension, hence no deposition) beside windy ones keeps the
     -9999 defaults and x = 0, as a lone module would; the windy members still solve."""

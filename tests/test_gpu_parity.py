@@ -81,12 +81,13 @@ def test_pattern_and_assembly_c1(pb, oracle, mesh_c1):
 def test_dilu_matches_oracle_dilu(pb, oracle, mesh_c1):
     """The multicolour D-ILU(0) kernels and the oracle's D-ILU(0) (written on the
     generic CSR) are the same preconditioner: GMRES(30) takes the same number of
-    iterations on both, for the 3-D suspension and the 2-D deposition systems."""
+    iterations on both for the 3-D suspension -- on the split operator up to 16 layers, with
+    plain applications at 17 -- and conjugate gradients as many for the 2-D deposition system."""
     _print_case("dilu_vs_oracle")
     F = mesh_c1.n_faces
     fo = meshgen.forcing_c1(F, seed=0)
     g = pb.face_geometry(mesh_c1)
-    for L in (5, 10):
+    for L in (5, 10, 17):
         ctx = pb.Context(g, pb.default_config(nLayer=L, tol=1e-10, precond=abi.PC_MCILU0,
                                               dep_precond=abi.PC_MCILU0))
         orc = oracle.Oracle(g, oracle.oracle_config(nLayer=L, tol=1e-10, precond=abi.PC_MCILU0,
@@ -333,11 +334,13 @@ def test_options_parity(pb, oracle, mesh_small):
 def test_every_spmv_launch_shape(pb, oracle, mesh_c1, precision):
     """Each launch shape of the position-order SpMV and both workgroup mappings of
     the D-ILU sweeps, forced in turn, give the oracle's fields; the tuners'
-    choices are among them and every option was timed."""
+    choices are among them and every option was timed.  FP64 with BiCGStab, which applies
+    both kernels (GMRES runs on the split operator at this layer count), MIXED with GMRES."""
     _print_case("spmv_launch_shapes", precision=precision)
     F = mesh_c1.n_faces
     fo = meshgen.forcing_c1(F, seed=0)
-    g, ctx, orc = _pair(pb, oracle, mesh_c1, L=10, precision=precision, tol=1e-12)
+    krylov = abi.KRYLOV_BICGSTAB if precision == abi.FP64 else abi.KRYLOV_GMRES
+    g, ctx, orc = _pair(pb, oracle, mesh_c1, L=10, precision=precision, tol=1e-12, krylov=krylov)
     og, _ = orc.step(fo)
     which = 0 if precision == abi.FP64 else 1
     gg, st = ctx.step(fo, want_fields=True)
@@ -361,21 +364,22 @@ def test_every_spmv_launch_shape(pb, oracle, mesh_c1, precision):
         ctx.precond_select(which, 2)
 
 
-@pytest.mark.parametrize("L", [7, 10])
+@pytest.mark.parametrize("L", [3, 7, 10, 13])
 @pytest.mark.parametrize("n_points", [18, 38, 39, 392])
 def test_tile_boundaries(pb, oracle, n_points, L):
     """Meshes whose face counts sit on either side of the 64-position tiles of the position
     order -- 26 faces (one partial tile), 63, 65 (a full tile and a tile of one) and 768
-    (twelve full tiles) -- at a layer count the column sweeps unroll exactly (10) and one
-    they guard (7): the mixed and FP64 split BiCGStab and FP64 GMRES with the position-order
-    SpMV and D-ILU reach 1e-12 and match the oracle."""
+    (twelve full tiles) -- at layer counts the split sweeps unroll exactly (7, 10) and ones
+    they guard (3 below 5, 13 below 16): the mixed and FP64 split BiCGStab, FP64 GMRES on
+    the split operator and FP64 BiCGStab with the position-order SpMV and D-ILU reach 1e-12
+    and match the oracle."""
     mesh = meshgen.synthetic_mesh(n_points, seed=0)
     F = mesh.n_faces
     _print_case("tile_boundaries", F=F, L=L)
     fo = meshgen.forcing_c1(F, seed=1)
     og = None
     for precision, krylov in ((abi.MIXED, abi.KRYLOV_BICGSTAB_SPLIT), (abi.FP64, abi.KRYLOV_BICGSTAB_SPLIT),
-                              (abi.FP64, abi.KRYLOV_GMRES)):
+                              (abi.FP64, abi.KRYLOV_GMRES), (abi.FP64, abi.KRYLOV_BICGSTAB)):
         g, ctx, orc = _pair(pb, oracle, mesh, L=L, precision=precision, tol=1e-12, krylov=krylov)
         if og is None:
             og, _ = orc.step(fo)
@@ -515,10 +519,13 @@ def test_c3_mixed_precision_96_steps(pb, oracle, mesh_c1):
 @pytest.mark.parametrize("L,precision,krylov", [
     (2, abi.FP64, abi.KRYLOV_BICGSTAB_SPLIT), (16, abi.MIXED, abi.KRYLOV_BICGSTAB_SPLIT),
     (16, abi.FP64, abi.KRYLOV_BICGSTAB), (20, abi.FP64, abi.KRYLOV_BICGSTAB), (20, abi.MIXED, abi.KRYLOV_GMRES),
-    (64, abi.FP64, abi.KRYLOV_GMRES)])
+    (64, abi.FP64, abi.KRYLOV_GMRES), (11, abi.FP64, abi.KRYLOV_BICGSTAB_SPLIT), (11, abi.MIXED, abi.KRYLOV_BICGSTAB_SPLIT),
+    (11, abi.FP64, abi.KRYLOV_GMRES), (15, abi.FP64, abi.KRYLOV_BICGSTAB_SPLIT), (15, abi.MIXED, abi.KRYLOV_BICGSTAB_SPLIT),
+    (15, abi.FP64, abi.KRYLOV_GMRES)])
 def test_layer_counts(pb, oracle, mesh_small, L, precision, krylov):
-    """The column kernels at the bounds of their unrolled forms (nLayer 2, 16) and the
-    looped forms above 16 (D-ILU sweeps, row-per-thread SpMV), against the oracle."""
+    """The column kernels at the bounds of their unrolled forms (nLayer 2, 16), the split sweeps
+    at the ends of their guarded range (11, 15) and the looped forms above 16 (D-ILU sweeps,
+    row-per-thread SpMV), against the oracle."""
     _print_case("layers", L=L, precision=precision, krylov=krylov)
     F = mesh_small.n_faces
     fo = meshgen.forcing_c2(F, seed=6)
