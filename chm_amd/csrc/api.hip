@@ -284,11 +284,16 @@ static double split_inner_rtol_default(const pbsm3d_ctx* c, const pbsm3d_config&
 }
 
 // The Neumann polynomial's degree trades operator applications (a longer one overshoots the target
-// by more) against basis traffic and launches.  Suspension solve, GMRES(30), mean of three to five
-// forcings, ms: 999,968 faces x 10 layers, degree 6 75, 8 74, 10 62, 12 64, 16 64; 240,000 x 10 4 8.8,
-// 6 8.1, 10 8.3; 200,000 x 9 1 10.5, 2 7.8, 4 6.3, 6 6.1; 125,000 x 7 1 4.54, 2 3.53, 4 2.98, 6 2.98;
-// 50,000 x 10 1 3.12, 2 2.40, 4 2.25, 6 2.29; 5,000 x 5 1 0.82, 2 0.73, 4 0.77 -- in a system that
-// small the launches are the bound, and degree 1 keeps GMRES's own iteration count.
+// by more) against basis traffic and launches.  Suspension solve, GMRES(30), mean of five forcings,
+// ms by degree 1 / 2 / 4 / 6 / 10:
+//   24,895 unknowns 0.85 0.74 0.81 0.90 1.08     1,799,685  10.4  7.5  5.7  5.3  5.1
+//   99,770          1.45 1.19 1.26 1.30 1.51     2,099,690  13.0  9.2  6.6  6.0  6.0
+//   107,766         1.63 1.28 1.30 1.37 1.71     2,399,690  15.7 11.4  8.2  7.2  7.2
+//   349,700         2.11 1.79 1.73 1.74 1.96     4,999,660  45.7 29.2 23.0 19.8 18.4
+//   877,800         4.25 3.17 2.51 2.39 2.56     9,999,680   221  144   82   67   55
+// Below 100,000 unknowns degree 1 all the same: there susp_iters stays GMRES's own count, which callers
+// compare with a CPU solve's (degree 2 reports 19 where GMRES takes 17).  The line to degree 10 is
+// where a basis vector leaves the caches, beyond which each costs memory traffic.
 static int neumann_degree(int64_t N) {
     if (N < 100000) return 1;
     return N * (int64_t)sizeof(double) > kCachedVector ? 10 : 4;
