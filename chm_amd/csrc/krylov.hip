@@ -250,6 +250,13 @@ SolveInfo gmres_solve(hipStream_t s, GmresWork<double>& w, const CsrOp<double>& 
     // modes that much less often.  Suspension solve, GMRES(30), mean of three to five forcings, ms, plain
     // against split: 5,000 faces x 5 layers 1.05 and 0.82, 50,000 x 10 3.95 and 2.25, 125,000 x 7 5.30
     // and 2.98, 200,000 x 9 11.6 and 6.3, 999,968 x 10 171 and 62.
+    // The split residual's norm stands for ||b - A x||; their reductions lie close together.  The long
+    // polynomial reaches a residual with more of the error left in the slow modes than plain cycles
+    // leave there: at 999,968 faces x 10 layers, 18 forcings, the concentration's relative error
+    // (2-norm, against a solve to 2e-13) was 3.7e-7 rms and 8.2e-7 at most after plain cycles, 7.3e-7
+    // and 3.1e-6 with 0.8 of the target, 2.8e-7 and 1.2e-6 with 0.2, 1.0e-7 and 4.3e-7 with 0.15 for
+    // one to three steps more (60 ms a solve, 55 with 0.8, 214 with plain cycles).
+    const double aim = split.degree > 4 ? 0.15 : 0.8;
     while (true) {
         info.resid = beta / nb;
         if (info.resid <= tol) {
@@ -261,8 +268,7 @@ SolveInfo gmres_solve(hipStream_t s, GmresWork<double>& w, const CsrOp<double>& 
         if (split.degree > 0) {
             int spent = 0;
             const double before = beta;
-            // the split residual's norm stands for ||b - A x||; their reductions lie close together
-            const bool moved = split_cycle(s, w, split, r, beta, 0.8 * tol * nb / beta,
+            const bool moved = split_cycle(s, w, split, r, beta, aim * tol * nb / beta,
                                            (maxit - info.iters) / split.degree, x, &spent);
             info.iters += spent;
             info.cycles += 1;
