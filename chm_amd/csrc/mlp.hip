@@ -303,7 +303,7 @@ __device__ __forceinline__ int64_t sample_row(uint64_t key, int64_t t, int64_t n
 // LDS reads and barriers of a tile, the other two by the latency of their loads (13 MB of tiles
 // and 2.4 MB of slabs at a batch of 8,192 stay in the caches).  A batch of 8,192 took 215 us in 29
 // launches (11 GEMMs of 13 us, split-K and column sums, one launch per elementwise step); these
-// three take 20.2 + 8.2 + 4.7 us with the same bits.
+// three take 20.3 + 8.1 + 4.5 us with the same bits.
 constexpr int kTrainCols = 64;
 constexpr int kTrainThreads = 512;
 constexpr int kLs = MlpDims::H + 8;      // LDS row stride (BF16) of [sample][128 features]
@@ -652,7 +652,7 @@ __device__ __forceinline__ void grad_block(const uint16_t* __restrict__ tiles, i
 
 // One wave per workgroup and job: 40 blocks of the weights for each slab, then 6 + 4 groups of 64
 // bias sums for each row block.  A slab's workgroups are eight apart, so that they run on one XCD,
-// whose L2 then reads the slab's tiles once.  A batch of 8,192 takes 8.2 us; 10.2 with four waves per
+// whose L2 then reads the slab's tiles once.  A batch of 8,192 takes 8.1 us; 10.2 with four waves per
 // workgroup, whose 160 workgroups leave CUs idle.
 constexpr int kSlabJobs = 40, kBiasJobs = 10;
 inline int64_t slab_grid(int nslab) { return (int64_t)(nslab + 7) / 8 * 8 * kSlabJobs; }
