@@ -282,7 +282,8 @@ int pbsm3d_profile_sample(pbsm3d_ctx* ctx, int every);
  * not tried). */
 int pbsm3d_spmv_tuning(const pbsm3d_ctx* ctx, int which, int32_t* chosen, float* ms, int32_t n);
 /* Fixes the launch shape (0 .. PBSM3D_SPMV_VARIANTS-1) instead of the tuner's
- * choice, or -1 to tune again at the next solve. */
+ * choice, or -1 to tune again at the next solve.  (FP64 GMRES with nLayer <= 16 runs on
+ * the split operator, without an SpMV: there the shape serves the plain cycles alone.) */
 #define PBSM3D_SPMV_VARIANTS 10
 int pbsm3d_spmv_select(pbsm3d_ctx* ctx, int which, int variant);
 /* The same for the multicolour D-ILU sweeps.  *mode (-1 until tuned) is the
